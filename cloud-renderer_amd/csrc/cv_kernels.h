@@ -18,7 +18,6 @@ constexpr int kBatchSortMax = 8192; // billboards a batched LDS sort takes (64 K
 constexpr int kFillChunk = 4096;    // elements per workgroup of the segmented fill
 constexpr int kChordLdsWords = 4096; // largest LDS bitmap (bricks) per pass-1 tile for chord-fill aggregation
 constexpr int kLightTile = 32;       // pass-1 work item: 32 x 32 light pixels of one billboard
-constexpr unsigned kConeWaves = 6144; // persistent cone-trace wavefronts (256 CUs x 24)
 
 // One mip level in the bricked layout: 4x4x4 bricks, texels Morton-ordered
 // inside a brick (bit order x0 y0 z0 x1 y1 z1), bricks x-fastest.
@@ -93,7 +92,6 @@ struct ConeDesc {
     float alpha_stop;
     float kscale;          // sigma * log2(e) / N
     int cone_mode;
-    int count;             // march: count samples and two-level samples (counter runs only)
     int composite;
     int quantize;
     int compensated;
@@ -227,14 +225,29 @@ void launch_sort_keys(const GridDesc& g, const float4* boards, int S, const floa
                       hipStream_t s);
 void launch_iota(int32_t* order, int S, hipStream_t s);
 int launch_sort(unsigned long long* keys, int S, int32_t* order, int* tie_flag, hipStream_t s);
-// camera tiles in the order the cone waves take them (heaviest first)
+// The items of a cone trace in the order its waves take them (heaviest first):
+// a camera tile, or one of the 1 << shift parts a heavy one is cut into.  A
+// trace has at most 2048^2 tiles of 8 x 8 pixels (22 bits).
+constexpr int kMaxSubShift = 4;
+__host__ __device__ inline int tile_item(int tile, int part, int shift) { return tile | part << 22 | shift << 26; }
+__host__ __device__ inline int item_tile(int it) { return it & 0x3fffff; }
+__host__ __device__ inline int item_part(int it) { return (it >> 22) & 15; }
+__host__ __device__ inline int item_shift(int it) { return it >> 26; }
 struct TileQueue {
-    unsigned int* counter;
+    const int* total;  // on the device
     const int* order;
+    unsigned bound;    // the total is at most this (launch size)
+};
+// rule of the cut: 1 / wave slots, extra items allowed, parts of every tile as
+// a shift (or -1: by weight)
+struct TileSplit {
+    float inv_slots;
+    int budget;
+    int fixed;
 };
 size_t tile_scratch_ints(int ntiles);
 TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int tiles_y, int words,
-                     unsigned long long* masks, int* scratch, hipStream_t s);
+                     unsigned long long* masks, int* scratch, bool every_fragment, hipStream_t s);
 // One scene of a batched cone-trace launch (device resident; the batched
 // kernel reads it with wave-uniform loads).
 struct BatchScene {
@@ -354,7 +367,7 @@ struct ConeLaunch {
     int words;
     void* image;
     unsigned long long* counters;  // 9 counters or null
-    const int* tile_order;
+    TileQueue items;
     MlpDev mlp;
     int learned;
     const float4* nmap;  // noise-march map (32^3 decoded RGBA8_SNORM texels) or null: no noise march

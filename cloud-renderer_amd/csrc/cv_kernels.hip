@@ -2181,24 +2181,73 @@ __global__ void __launch_bounds__(256) k_tile_bucket(const int* __restrict__ til
     __syncthreads();
     if (threadIdx.x < 32 && lh[threadIdx.x] > 0) atomicAdd(&hist[threadIdx.x], lh[threadIdx.x]);
 }
+// Into how many parts (1 << shift) the tiles of each bucket are cut.
+// sp.fixed >= 0: that many for every tile with billboards.  Else by weight (the
+// number of binned billboards, 1.5 times the bucket's lower bound): a bucket
+// is cut until an item's weight is at most the device's share of all of them
+// (sum / slots), the heaviest buckets first while the extra items fit the
+// budget.  One wave, lane k = bucket k < 32; every workgroup computes the
+// same.  Returns the lane's first item; *total: all items.
+__device__ __forceinline__ int tile_split(const int* __restrict__ hist, int lane, const TileSplit& sp, int* shift,
+                                          int* total) {
+    const int n = lane < 32 ? hist[lane] : 0;
+    const float w = lane < 31 ? 1.5f * (float)(1u << (30 - lane)) : 0.0f;
+    float sum = (float)n * w;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+    const float part = fmaxf(sum * sp.inv_slots, 1.0f);
+    int sh = 0;
+    while (sh < kMaxSubShift && w > part * (float)(1 << sh)) ++sh;
+    if (sp.fixed >= 0) sh = lane < 31 ? sp.fixed : 0;
+    // extra items of this and the heavier buckets
+    float ext = (float)n * (float)((1 << sh) - 1), incl = ext;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const float y = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += y;
+    }
+    if (incl > (float)sp.budget) sh = 0;
+    int items = n << sh, first = items;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int y = __shfl_up(first, o, 64);
+        if (lane >= o) first += y;
+    }
+    *total = __builtin_amdgcn_readlane(first, 63);
+    *shift = sh;
+    return first - items;
+}
 // counting-sort scatter: ranks inside a workgroup from LDS atomics, one global
-// atomic per (workgroup, bucket) to reserve the range
+// atomic per (workgroup, bucket) to reserve the range; a tile's parts are
+// consecutive items (tile_item)
 __global__ void __launch_bounds__(256) k_tile_scatter(const int* __restrict__ bucket_of, int ntiles,
                                                       const int* __restrict__ hist, int* __restrict__ cursor,
-                                                      int* __restrict__ tile_order) {
-    __shared__ int lh[32], lbase[32];
+                                                      int* __restrict__ tile_order, TileSplit sp,
+                                                      int* __restrict__ total) {
+    __shared__ int lh[32], lbase[32], bfirst[32], bshift[32];
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (threadIdx.x < 32) lh[threadIdx.x] = 0;
     __syncthreads();
     const int key = t < ntiles ? bucket_of[t] : -1;
     const int lrank = key >= 0 ? atomicAdd(&lh[key], 1) : 0;
+    if (threadIdx.x < 64) {
+        int sh, all;
+        const int f = tile_split(hist, (int)threadIdx.x, sp, &sh, &all);
+        if (threadIdx.x < 32) {
+            bfirst[threadIdx.x] = f;
+            bshift[threadIdx.x] = sh;
+        }
+        if (total && blockIdx.x == 0 && threadIdx.x == 0) *total = all;
+    }
     __syncthreads();
     if (threadIdx.x < 32 && lh[threadIdx.x] > 0) lbase[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], lh[threadIdx.x]);
     __syncthreads();
     if (key < 0) return;
-    int base = 0;
-    for (int k = 0; k < key; ++k) base += hist[k];
-    tile_order[base + lbase[key] + lrank] = t;
+    const int sh = bshift[key];
+    int* o = tile_order + bfirst[key] + ((lbase[key] + lrank) << sh);
+    if (!total) *o = t;  // whole tiles by their index
+    else
+        for (int p = 0; p < 1 << sh; ++p) o[p] = tile_item(t, p, sh);
 }
 
 // ---------------------------------------------------------------------------
@@ -2481,7 +2530,7 @@ struct FtbState {
 // bit-identical to filtering all four channels.  KAHAN: compensated sums.
 // TAB: corner offsets from the workgroup's LDS tables (bit-identical loads).
 template <int FMT, bool KAHAN, bool TAB>
-__device__ __forceinline__ int march_ftb_t(const VolumeDesc& vd, const void* __restrict__ vol, const ConeDesc& cd,
+__device__ __forceinline__ int march_ftb_t(const VolumeDesc& vd, const void* __restrict__ vol, const ConeDesc& cd, bool count,
                                            float p0x, float p0y, float p0z, float dx, float dy, float dz, int i0,
                                            int i1, FtbState& st, uint32_t& nsamp, uint32_t& ntwo, const TabRef& tr) {
     if (i0 >= i1) return 0;
@@ -2536,7 +2585,7 @@ __device__ __forceinline__ int march_ftb_t(const VolumeDesc& vd, const void* __r
         } else {
             sm = sample_levels<FMT, 2>(vol, LA, LB, fr, sx, sy, sz, &two);
         }
-        if (cd.count) {
+        if (count) {
             // counter runs only; the empty asm keeps this a scalar branch
             // (no per-step selects in the timed kernels)
             asm volatile("");
@@ -2565,13 +2614,13 @@ __device__ __forceinline__ int march_ftb_t(const VolumeDesc& vd, const void* __r
     return 0;
 }
 template <int FMT, bool TAB = false>
-__device__ __forceinline__ int march_ftb(const VolumeDesc& vd, const void* __restrict__ vol, const ConeDesc& cd,
+__device__ __forceinline__ int march_ftb(const VolumeDesc& vd, const void* __restrict__ vol, const ConeDesc& cd, bool count,
                                          float p0x, float p0y, float p0z, float dx, float dy, float dz, int i0,
                                          int i1, FtbState& st, uint32_t& nsamp, uint32_t& ntwo,
                                          const TabRef& tr = TabRef{nullptr, nullptr}) {
     return cd.compensated
-               ? march_ftb_t<FMT, true, TAB>(vd, vol, cd, p0x, p0y, p0z, dx, dy, dz, i0, i1, st, nsamp, ntwo, tr)
-               : march_ftb_t<FMT, false, TAB>(vd, vol, cd, p0x, p0y, p0z, dx, dy, dz, i0, i1, st, nsamp, ntwo, tr);
+               ? march_ftb_t<FMT, true, TAB>(vd, vol, cd, count, p0x, p0y, p0z, dx, dy, dz, i0, i1, st, nsamp, ntwo, tr)
+               : march_ftb_t<FMT, false, TAB>(vd, vol, cd, count, p0x, p0y, p0z, dx, dy, dz, i0, i1, st, nsamp, ntwo, tr);
 }
 
 // Far-field features after k samples: last sample position (2x - 1), cone
@@ -2765,8 +2814,87 @@ __device__ __forceinline__ bool noise_fragment(const float4* __restrict__ map, c
     return true;
 }
 
-// Ranks gathered per pass of the cone walk.
-constexpr int kConeChunk = 256;
+// What one wave of the cone walk keeps in LDS: the candidates of a round
+// (billboards binned into the tile, in draw order).
+constexpr int kConeChunk = 64;
+// Fragments of one pixel marched at once under a front-to-back composite:
+// 4 takes plain256's cone (640 x 360) from 261 us (1) over 155 (2) to 104,
+// beyond that more is marched behind pixels that stop (64: no gain, and
+// plain256's 1080p cone 234 -> 241).
+constexpr int kSpeculate = 4;
+struct ConeLds {
+    float4 cw[kConeChunk];  // world centre, radius
+    float4 vv[kConeChunk];  // view-space centre, radius
+    int rank[kConeChunk];   // draw ranks
+};
+
+// LDS writes of the wave's lanes before this are seen by its reads after it
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// The next (at most 64) binned billboards of a tile in draw order (front to
+// back for COMP = 1, back to front for COMP = 0) into L; returns how many, 0
+// once the tile has no more.  A lane holds one of 64 consecutive mask words
+// (bits; w0 = the first word not loaded yet), so a load brings 4096 ranks and
+// a wave scan places the set bits; each candidate is then fetched by a lane
+// of its own, in one round trip for all of them instead of one per billboard.
+template <int COMP>
+__device__ __forceinline__ int cone_candidates(const unsigned long long* __restrict__ tm, int words, int lane,
+                                               const int32_t* __restrict__ order,
+                                               const float4* __restrict__ sph_world,
+                                               const float4* __restrict__ sph_view, int& w0, unsigned long long& bits,
+                                               ConeLds& L) {
+    int nc = 0;
+    while (nc < kConeChunk) {
+        if (__ballot(bits != 0ull) == 0ull) {
+            if (w0 >= words) break;
+            const int k = w0 + lane;
+            bits = k < words ? tm[COMP == 1 ? words - 1 - k : k] : 0ull;
+            w0 += 64;
+            continue;
+        }
+        const int c = __popcll(bits);
+        int incl = c;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+            const int y = __shfl_up(incl, off, 64);
+            if (lane >= off) incl += y;
+        }
+        const int kw = w0 - 64 + lane;  // the lane's word
+        const int r0 = (COMP == 1 ? words - 1 - kw : kw) << 6;
+        for (int pos = nc + incl - c; bits && pos < kConeChunk; ++pos) {
+            const int b = COMP == 1 ? 63 - __clzll((long long)bits) : __ffsll((long long)bits) - 1;
+            bits &= ~(1ull << b);
+            L.rank[pos] = r0 + b;
+        }
+        nc = min(kConeChunk, nc + __builtin_amdgcn_readlane(incl, 63));
+    }
+    wave_lds_sync();
+    if (lane < nc) {
+        const int j = order[L.rank[lane]];
+        const float4 cw = sph_world[j];
+        const float4 vv = sph_view[j];
+        L.cw[lane] = cw;
+        L.vv[lane] = make_float4(vv.x, vv.y, vv.z, cw.w);
+    }
+    wave_lds_sync();
+    return nc;
+}
+
+// !(sphere_contrib(du, dv, s) < 0.01): the discard threshold lies at
+// (dist / s)^2 = 0.9999, so a squared distance clear of it decides without the
+// square roots and the division; only the band around it (and radii whose
+// square leaves the normal range) takes them.
+__device__ __forceinline__ bool sphere_covers(float du, float dv, float s) {
+    const float d2 = du * du + dv * dv, s2 = s * s;
+    const bool tame = s2 > 1e-30f && s2 < 1e30f;
+    if (tame && d2 <= s2 * 0.9998f) return true;
+    if (tame && d2 >= s2 * 0.99995f) return false;
+    return !(sphere_contrib(du, dv, s) < 0.01f);
+}
 
 // CONE: 0 weighted R-sum, 1 front-to-back.  COMP: 0 GL blend, 1 front-to-back.
 // LEARNED (front-to-back only): after cd.learned_k samples the far field of
@@ -2775,33 +2903,45 @@ constexpr int kConeChunk = 256;
 // remaining transmittance, exceeds cd.err_bound (or every cone when
 // err_bound < 0) falls back to the plain march from step k.
 //
-// Shade one camera tile, one pixel per lane, each lane walking only the
-// billboards that cover its own pixel.  The tile's binned billboards are
-// taken in rank order (front to back for COMP = 1, back to front for
-// COMP = 0) in chunks: the wave tests a chunk's billboards against its 64
-// pixels and keeps those that cover any pixel, with the coverage ballot, in
-// LDS (cover[], id[]); then every lane steps through that list to its own
-// next covering billboard and all lanes march their own fragments together.
-// A pixel composites exactly the fragments, in exactly the order, of a walk
-// over every billboard, so the image is the same bit for bit; what changes is
-// that a march no longer idles the lanes the billboard misses.  All lanes of
-// a round start at step 0, so the LOD of step i (and with it the one- or
-// two-level sampling branch) stays uniform across the wave, and in the
-// learned kernels the lanes reach step k together: their cones form the
-// wave's 64-row MLP batch.
+// Shade the pixels of one camera tile, 64 >> sub_shift of them (part `sub` of
+// the tile), one per lane.  The tile's binned billboards are taken 64 at a
+// time in draw order; every pixel tests them and keeps a 64-bit mask of those
+// that cover it.  Rounds then hand the wave's lanes to the pixels that still
+// have fragments: with nl such pixels each takes the next 64 / nl (the first
+// ones one more) of its fragments, every lane marches one, and the pixel
+// blends its results in draw order.  A pixel composites exactly the
+// fragments, in exactly the order, of a walk over every billboard, so the
+// image is the same bit for bit.  A front-to-back pixel that stops drops what
+// was marched beyond; those lanes would have idled.  What bounds the kernel is
+// the chain of dependent steps of its slowest wave, rounds x steps: spare
+// lanes shorten it, and images too small to fill the device split their tiles
+// over several waves (sub_shift).  All lanes of a round start at step 0, so
+// the LOD of step i (and with it the one- or two-level sampling branch) stays
+// uniform across the wave, and in the learned kernels the lanes reach step k
+// together: their cones form the wave's 64-row MLP batch.
 template <int FMT, int CONE, int COMP, int LEARNED, int NM = 0, bool TAB = false>
 __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& vd, const CameraView& cv,
                                           const ConeDesc& cd, const void* __restrict__ vol,
                                           const float4* __restrict__ sph_world, const float4* __restrict__ sph_view,
                                           const int32_t* __restrict__ order,
                                           const unsigned long long* __restrict__ masks, int words,
-                                          void* __restrict__ image, const MlpDev& mlp, uint16_t* xs,
-                                          unsigned long long* cover, int* id, int tile, int lane, uint32_t& nfrag,
+                                          void* __restrict__ image, const MlpDev& mlp, uint16_t* xs, ConeLds& L,
+                                          int tile, int sub, int sub_shift, int lane, bool count, uint32_t& nfrag,
                                           uint32_t& nsamp, uint32_t& ntwo, uint32_t& nrows, uint32_t& nfall,
                                           uint32_t& nevals, const float4* __restrict__ nmap = nullptr,
                                           const TabRef& tr = TabRef{nullptr, nullptr}) {
+    // r = g = b in every colour the front-to-back composite sums (the learned
+    // far field predicts three): one sum stands for all three
+    constexpr bool GREY = COMP == 1 && !LEARNED;
+    const int npix = 64 >> sub_shift;
     const int tx = tile % cv.tiles_x, ty = tile / cv.tiles_x;
-    const int px = tx * cv.tile_w + (lane & (cv.tile_w - 1)), py = ty * cv.tile_h + (lane >> cv.tile_shift);
+    const int pl = sub * npix + (lane & (npix - 1));  // the lane's pixel of the tile
+    int lx = pl & (cv.tile_w - 1), ly = pl >> cv.tile_shift;
+    if (cv.tile_w == 8) {  // Morton order, so that a part is a square or two of the tile
+        lx = (pl & 1) | ((pl >> 1) & 2) | ((pl >> 2) & 4);
+        ly = ((pl >> 1) & 1) | ((pl >> 2) & 2) | ((pl >> 3) & 4);
+    }
+    const int px = tx * cv.tile_w + lx, py = ty * cv.tile_h + ly;
     const bool valid = px < cv.W && py < cv.H;
     const float rx = pixel_ndc(px, cv.W) * cv.kx;
     const float ry = pixel_ndc(py, cv.H) * cv.ky;
@@ -2844,89 +2984,86 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
     } else {
         C0 = C1 = C2 = C3 = 0.0f;
     }
-    bool done = !valid;
+    // the pixel's owner lane (the first of the lanes that hold it) blends
+    bool done = !valid || lane >= npix;
     const unsigned long long* tm = masks + (size_t)tile * words;
-    int wi = 0, wcur = 0;
-    unsigned long long bits = 0;
+    int w0 = 0;
+    unsigned long long bits = 0ull;
 
     while (!__all(done)) {
-        // gather: the next kConeChunk binned billboards that cover any live pixel
-        int n = 0;
-        while (n < kConeChunk) {
-            while (bits == 0 && wi < words) {
-                wcur = COMP == 1 ? (words - 1 - wi) : wi;
-                bits = tm[wcur];
-                ++wi;
-            }
-            if (bits == 0) break;
-            int b;
-            if (COMP == 1) b = 63 - __clzll((long long)bits);
-            else b = __ffsll((long long)bits) - 1;
-            bits &= ~(1ull << b);
-            const int j = order[(wcur << 6) | b];
-            const float4 cw = sph_world[j];
-            const float4 vv = sph_view[j];
-            bool cov = false;
-            if (!done) {
-                const float dz = -vv.z;
-                const float sc = sphere_contrib(rx * dz - vv.x, ry * dz - vv.y, cw.w);
-                cov = !(sc < 0.01f);
-            }
-            const unsigned long long m = __ballot(cov);
-            if (m) {
-                if (lane == 0) {
-                    cover[n] = m;
-                    id[n] = j;
-                }
-                ++n;
-            }
+        const int nc = cone_candidates<COMP>(tm, words, lane, order, sph_world, sph_view, w0, bits, L);
+        if (nc == 0) break;
+        // the candidates that cover the pixel; the lanes of one pixel take
+        // every (1 << sub_shift)-th candidate each
+        unsigned long long mine = 0ull;
+#pragma unroll 4
+        for (int c0 = 0; c0 < nc; c0 += 1 << sub_shift) {
+            const int c = c0 + (lane >> (6 - sub_shift));
+            const float4 v = L.vv[c & (kConeChunk - 1)];
+            const float dz = -v.z;
+            const bool cov = c < nc && sphere_covers(rx * dz - v.x, ry * dz - v.y, v.w);
+            mine |= cov ? 1ull << c : 0ull;
         }
-        if (n == 0) break;
-        __builtin_amdgcn_wave_barrier();
-        // march: each lane its own next covering billboard, until none is left
-        int cur = 0;
+        for (int o = npix; o < 64; o <<= 1) {
+            const uint32_t lo = __shfl_xor((int)(uint32_t)mine, o, 64), hi = __shfl_xor((int)(uint32_t)(mine >> 32), o, 64);
+            mine |= ((unsigned long long)hi << 32) | lo;
+        }
+        if (done) mine = 0ull;
         for (;;) {
-            bool have = false;
-            int j = 0;
-            if (!done) {
-                while (cur < n) {
-                    const unsigned long long m = cover[cur];
-                    const int jj = id[cur];
-                    ++cur;
-                    if ((m >> lane) & 1ull) {
-                        have = true;
-                        j = jj;
-                        break;
-                    }
-                }
+            const unsigned long long lm = __ballot(mine != 0ull);
+            if (lm == 0ull) break;
+            // nl pixels share the 64 lanes: ordinal o takes `share` lanes from
+            // lane `first` on, the first `rem` ordinals one more
+            const int nl = __popcll(lm);
+            int share = 64 / nl, rem = 64 - share * nl;
+            if (COMP == 1 && share >= kSpeculate) { share = kSpeculate; rem = 0; }
+            int first = lane, nt = 1;
+            unsigned long long m = mine;
+            float prx = rx, pry = ry;
+            bool have = mine != 0ull;
+            if (nl < 64) {
+                const int o = (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(lm >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)lm, 0u));
+                first = o * share + min(o, rem);
+                nt = share + (o < rem ? 1 : 0);
+                // owner lanes by ordinal (a permutation: the others follow)
+                const int dst = have ? o : nl + lane - o;
+                const int own = __builtin_amdgcn_ds_permute(dst << 2, lane);
+                // this lane's ordinal k and which of its pixel's fragments, q
+                const int cut = rem * (share + 1);
+                const bool big = lane < cut;
+                const int per = share + (big ? 1 : 0), off = big ? lane : lane - cut;
+                const int kq = (int)(((float)off + 0.5f) * __builtin_amdgcn_rcpf((float)per));  // off / per, off < 64
+                const int q = off - kq * per, k = big ? kq : rem + kq;
+                const int src = __builtin_amdgcn_ds_bpermute(min(k, 63) << 2, own);
+                const uint32_t lo = __shfl((int)(uint32_t)mine, src, 64), hi = __shfl((int)(uint32_t)(mine >> 32), src, 64);
+                m = ((unsigned long long)hi << 32) | lo;
+                prx = __shfl(rx, src, 64);
+                pry = __shfl(ry, src, 64);
+                for (int t = 0; t < q && m; ++t) m &= m - 1ull;
+                have = k < nl && m != 0ull;
             }
-            if (!__any(have)) break;
             ConeFrag f = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
             FtbState st = {0.0f, 0.0f, 0.0f, 0.0f};
-            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = 0.0f;
+            float s0 = 0.0f, s1 = 0.0f, s2 = 0.0f, s3 = -1.0f;  // s3 < 0: no fragment
             float s0u = 0.0f;  // weighted cone: the unclamped indirect
             float fr = 0.0f, fg = 0.0f, fb = 0.0f;  // colour with the predicted far field
             bool pred = false;
             bool alive = false;
+            uint32_t ns = 0, n2 = 0, row = 0;  // the fragment's samples, two-level samples, MLP row (1) and fallback (2)
             float nm_col = 1.0f, nm_alpha = 0.0f;  // noise march (NM): colour factor and fragment alpha
-            if constexpr (NM) {
+            if (have) {
+                const int c = __ffsll((long long)m) - 1;
+                const float4 cw = L.cw[c];
+                const float4 vv = L.vv[c];
+                const float dz = -vv.z;
+                const float du = prx * dz - vv.x;
+                const float dv = pry * dz - vv.y;
                 // the noise branch runs first and may discard the fragment
-                if (have) {
-                    const float4 cw = sph_world[j];
-                    const float4 vv = sph_view[j];
-                    const float dz = -vv.z;
-                    have = noise_fragment(nmap, cd, cv, cw, rx * dz - vv.x, ry * dz - vv.y, nm_col, nm_alpha);
-                }
+                if constexpr (NM) have = noise_fragment(nmap, cd, cv, cw, du, dv, nm_col, nm_alpha);
+                if (have) f = cone_frag(g, cv, cd, cw, du, dv, sphere_contrib(du, dv, cw.w), fN);
             }
             if (have) {
-                const float4 cw = sph_world[j];
-                const float4 vv = sph_view[j];
-                const float dz = -vv.z;
-                const float du = rx * dz - vv.x;
-                const float dv = ry * dz - vv.y;
-                const float sc = sphere_contrib(du, dv, cw.w);
-                ++nfrag;
-                f = cone_frag(g, cv, cd, cw, du, dv, sc, fN);
                 if constexpr (CONE == 0) {
                     float color = 0.0f;
                     for (int i = 0; i < cd.steps; ++i) {
@@ -2934,15 +3071,15 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
                         bool two;
                         float4 sm = sample_lod<FMT, 1>(vol, vd, step_level(cd, i), cd.lfrac[i], fmaf(h, f.dx, f.p0x), fmaf(h, f.dy, f.p0y),
                                                        fmaf(h, f.dz, f.p0z), &two);
-                        ntwo += two ? 1u : 0u;
+                        n2 += two ? 1u : 0u;
                         color = color + (sm.x * (float)(i + 1)) / cd.den;
                     }
-                    nsamp += (uint32_t)cd.steps;
+                    ns = (uint32_t)cd.steps;
                     s0 = s1 = s2 = s3 = clamp01(color);
                     s0u = color;
                 } else {
-                    const int rs = march_ftb<FMT, TAB>(vd, vol, cd, f.p0x, f.p0y, f.p0z, f.dx, f.dy, f.dz, 0,
-                                                             kk_steps, st, nsamp, ntwo, tr);
+                    const int rs = march_ftb<FMT, TAB>(vd, vol, cd, count, f.p0x, f.p0y, f.p0z, f.dx, f.dy, f.dz, 0,
+                                                       kk_steps, st, ns, n2, tr);
                     alive = LEARNED && rs == 0 && kk_steps < cd.steps;
                 }
             }
@@ -2952,7 +3089,7 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
                     float x[kMlpIn];
                     if (alive) {
                         farfield_features<FMT>(vd, vol, cd, f.p0x, f.p0y, f.p0z, f.dx, f.dy, f.dz, fN, x);
-                        nsamp += 4;
+                        ns += 4;
                     } else {
 #pragma unroll
                         for (int q = 0; q < kMlpIn; ++q) x[q] = 0.0f;
@@ -2970,17 +3107,17 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
                     __syncthreads();
                     ++nevals;
                     if (alive) {
-                        ++nrows;
-                        const float rem = 1.0f - st.a;
-                        if (cd.err_bound < 0.0f || !(rem * y[4] <= cd.err_bound)) {
-                            ++nfall;
-                            march_ftb<FMT>(vd, vol, cd, f.p0x, f.p0y, f.p0z, f.dx, f.dy, f.dz, kk_steps,
-                                                 cd.steps, st, nsamp, ntwo);
+                        row = 1;
+                        const float rest = 1.0f - st.a;
+                        if (cd.err_bound < 0.0f || !(rest * y[4] <= cd.err_bound)) {
+                            row = 3;
+                            march_ftb<FMT>(vd, vol, cd, count, f.p0x, f.p0y, f.p0z, f.dx, f.dy, f.dz, kk_steps,
+                                           cd.steps, st, ns, n2);
                         } else {
-                            fr = fmaf(rem, clamp01(y[0]), st.c);
-                            fg = fmaf(rem, clamp01(y[1]), st.c);
-                            fb = fmaf(rem, clamp01(y[2]), st.c);
-                            st.a = st.a + rem * clamp01(y[3]);
+                            fr = fmaf(rest, clamp01(y[0]), st.c);
+                            fg = fmaf(rest, clamp01(y[1]), st.c);
+                            fb = fmaf(rest, clamp01(y[2]), st.c);
+                            st.a = st.a + rest * clamp01(y[3]);
                             pred = true;
                         }
                     }
@@ -2999,13 +3136,44 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
                     s0 = s1 = s2 = clamp01(nm_col * ind);
                     s3 = clamp01(nm_alpha);
                 }
-                blend_frag<COMP>(cd, s0, s1, s2, s3, C0, C1, C2, C3, done);
+            }
+            // each pixel blends its fragments in draw order
+            for (int t = 0; t < share + (rem > 0 ? 1 : 0); ++t) {
+                const int from = first + t;
+                const float v3 = __shfl(s3, from, 64), v0 = __shfl(s0, from, 64);
+                const float v1 = LEARNED ? __shfl(s1, from, 64) : v0, v2 = LEARNED ? __shfl(s2, from, 64) : v0;
+                uint32_t vs = 0, vt = 0, vr = 0;
+                if (count) {
+                    vs = (uint32_t)__shfl((int)ns, from, 64);
+                    vt = (uint32_t)__shfl((int)n2, from, 64);
+                    vr = (uint32_t)__shfl((int)row, from, 64);
+                }
+                if (mine != 0ull && t < nt) {
+                    mine &= mine - 1ull;
+                    if (v3 >= 0.0f) {
+                        if constexpr (GREY) {
+                            const float wgt = (1.0f - C3) * v3;
+                            C0 = fmaf(wgt, v0, C0);
+                            C3 = C3 + wgt;
+                            if (C3 >= cd.alpha_stop) done = true;
+                        } else {
+                            blend_frag<COMP>(cd, v0, v1, v2, v3, C0, C1, C2, C3, done);
+                        }
+                        ++nfrag;
+                        nsamp += vs;
+                        ntwo += vt;
+                        nrows += vr & 1u;
+                        nfall += vr >> 1;
+                        if (COMP == 1 && done) mine = 0ull;
+                    }
+                }
             }
         }
-        // the next gather overwrites the list every lane has finished reading
-        __builtin_amdgcn_wave_barrier();
+        // the next candidates overwrite the list every lane has finished reading
+        wave_lds_sync();
     }
-    if (valid) {
+    if (GREY) C1 = C2 = C0;
+    if (valid && lane < npix) {
         char* row = (char*)image + (size_t)py * cd.pitch;
         if (cd.pixfmt == 0) {
             ((float4*)row)[px] = make_float4(C0, C1, C2, C3);
@@ -3024,19 +3192,19 @@ __global__ void __launch_bounds__(64, LEARNED ? 3 : (NM ? 4 : 6)) k_cone(GridDes
                                              const float4* __restrict__ sph_view, const int32_t* __restrict__ order,
                                              const unsigned long long* __restrict__ masks, int words,
                                              void* __restrict__ image, unsigned long long* __restrict__ counters,
-                                             const int* __restrict__ tile_order, MlpDev mlp,
-                                             const float4* __restrict__ nmap) {
-    // One wavefront per tile; tiles are dispatched heaviest first
-    // (tile_order), so the costly clump-centre tiles do not form the tail.
+                                             TileQueue items, MlpDev mlp, const float4* __restrict__ nmap) {
+    // One wavefront per tile or part of one, the heaviest first, so the
+    // costly clump-centre tiles do not form the tail.
+    if ((int)blockIdx.x >= *items.total) return;
     __shared__ __align__(16) uint16_t xs[LEARNED ? 64 * kMlpInPad : 8];
-    __shared__ unsigned long long cover[kConeChunk];
-    __shared__ int id[kConeChunk];
+    __shared__ ConeLds L;
     const int lane = threadIdx.x;
     uint32_t nfrag = 0, nsamp = 0, ntwo = 0, nrows = 0, nfall = 0, nevals = 0;
-    const int tile = tile_order ? tile_order[blockIdx.x] : (int)blockIdx.x;
+    const int it = __builtin_amdgcn_readfirstlane(items.order[blockIdx.x]);
     cone_tile<FMT, CONE, COMP, LEARNED, NM>(g, vd, cv, cd, vol, sph_world, sph_view, order, masks, words, image,
-                                            mlp, xs, cover, id, tile, lane, nfrag, nsamp, ntwo, nrows, nfall, nevals,
-                                            nmap);
+                                            mlp, xs, L, item_tile(it), item_part(it), item_shift(it), lane,
+                                            counters != nullptr, nfrag, nsamp,
+                                            ntwo, nrows, nfall, nevals, nmap);
     if (counters) {
         unsigned long long a = wave_sum_u64(nfrag), bsum = wave_sum_u64(nsamp), c = wave_sum_u64(ntwo);
         unsigned long long e0 = 0, e1 = 0;
@@ -3079,7 +3247,7 @@ __device__ void build_cone_tabs(const VolumeDesc& vd, const ConeTab& t, uint32_t
 
 // The front-to-back cone trace with table addressing: t.wpg waves per
 // workgroup share the LDS tables of every level (built once per
-// workgroup); wave w of workgroup b shades tile tile_order[b * wpg + w].
+// workgroup); wave w of workgroup b shades item b * wpg + w.
 // Dynamic LDS: the tables (t.words words), then per wave the gather lists
 // (kConeChunk coverage masks and ids).
 template <int FMT, int COMP>
@@ -3090,22 +3258,24 @@ __global__ void __launch_bounds__(512, 6) k_cone_tab(GridDesc g, VolumeDesc vd, 
                                                      const int32_t* __restrict__ order,
                                                      const unsigned long long* __restrict__ masks, int words,
                                                      void* __restrict__ image, unsigned long long* __restrict__ counters,
-                                                     const int* __restrict__ tile_order, int ntiles) {
+                                                     TileQueue items) {
     extern __shared__ __align__(16) uint32_t dyn[];
+    const int nitems = *items.total;
+    if ((int)(blockIdx.x * t.wpg) >= nitems) return;
     build_cone_tabs<FMT>(vd, t, dyn);
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int item = blockIdx.x * t.wpg + wave;
-    if (item >= ntiles) return;
-    unsigned long long* cover = (unsigned long long*)(dyn + t.words) + (size_t)wave * kConeChunk;
-    int* id = (int*)((unsigned long long*)(dyn + t.words) + (size_t)t.wpg * kConeChunk) + (size_t)wave * kConeChunk;
-    const int tile = tile_order ? tile_order[item] : item;
+    if (item >= nitems) return;
+    ConeLds& L = ((ConeLds*)(dyn + t.words))[wave];
+    const int it = __builtin_amdgcn_readfirstlane(items.order[item]);
     uint32_t nfrag = 0, nsamp = 0, ntwo = 0, nrows = 0, nfall = 0, nevals = 0;
     const MlpDev none{nullptr, nullptr, nullptr};
     const TabRef tr{dyn, &t};
     cone_tile<FMT, 1, COMP, 0, 0, true>(g, vd, cv, cd, vol, sph_world, sph_view, order, masks, words, image, none,
-                                        nullptr, cover, id, tile, lane, nfrag, nsamp, ntwo, nrows, nfall, nevals,
-                                        nullptr, tr);
+                                        nullptr, L, item_tile(it), item_part(it), item_shift(it), lane,
+                                        counters != nullptr, nfrag, nsamp, ntwo,
+                                        nrows, nfall, nevals, nullptr, tr);
     if (counters) {
         unsigned long long a = wave_sum_u64(nfrag), b = wave_sum_u64(nsamp), c = wave_sum_u64(ntwo);
         if (lane == 0) {
@@ -3126,8 +3296,7 @@ __global__ void __launch_bounds__(256) k_cone_batch(const BatchScene* __restrict
     const int lane = threadIdx.x & 63;
     const int wpg = blockDim.x >> 6;
     const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    __shared__ unsigned long long cover[4][kConeChunk];  // waves per workgroup <= 4
-    __shared__ int id[4][kConeChunk];
+    __shared__ ConeLds L[4];  // waves per workgroup <= 4
     uint32_t nfrag = 0, nsamp = 0, ntwo = 0, nrows = 0, nfall = 0, nevals = 0;
     const MlpDev none{nullptr, nullptr, nullptr};
     for (int item = blockIdx.x * wpg + wave; item < total; item += gridDim.x * wpg) {
@@ -3141,8 +3310,8 @@ __global__ void __launch_bounds__(256) k_cone_batch(const BatchScene* __restrict
         const int sidx = __builtin_amdgcn_readfirstlane(lo);
         const BatchScene& B = scenes[sidx];
         cone_tile<FMT, CONE, COMP, 0>(B.g, B.vd, B.cv, B.cd, B.levels, B.sph_world, B.sph_view, B.order, B.masks,
-                                            B.words, B.image, none, nullptr, cover[wave], id[wave], gt - B.tile0, lane,
-                                            nfrag, nsamp, ntwo, nrows, nfall, nevals);
+                                      B.words, B.image, none, nullptr, L[wave], gt - B.tile0, 0, 0, lane,
+                                      counters != nullptr, nfrag, nsamp, ntwo, nrows, nfall, nevals);
     }
     if (counters) {
         unsigned long long a = wave_sum_u64(nfrag), b = wave_sum_u64(nsamp), c = wave_sum_u64(ntwo);
@@ -3170,14 +3339,14 @@ __global__ void __launch_bounds__(256) k_segments(GridDesc g, VolumeDesc vd, Con
     const int kk_steps = cd.learned_k;
     FtbState st = {0.0f, 0.0f, 0.0f, 0.0f};
     uint32_t ns = 0, nt = 0;
-    int rs = march_ftb<FMT>(vd, vol, cd, px, py, pz, dx, dy, dz, 0, min(kk_steps, cd.steps), st, ns, nt);
+    int rs = march_ftb<FMT>(vd, vol, cd, false, px, py, pz, dx, dy, dz, 0, min(kk_steps, cd.steps), st, ns, nt);
     const bool rec = rs == 0 && kk_steps < cd.steps;
     float f[kMlpIn];
     float ck = 0.0f, ak = 0.0f;
     if (rec) {
         farfield_features<FMT>(vd, vol, cd, px, py, pz, dx, dy, dz, (float)g.N, f);
         ck = st.c; ak = st.a;
-        march_ftb<FMT>(vd, vol, cd, px, py, pz, dx, dy, dz, kk_steps, cd.steps, st, ns, nt);
+        march_ftb<FMT>(vd, vol, cd, false, px, py, pz, dx, dy, dz, kk_steps, cd.steps, st, ns, nt);
     }
     valid[i] = rec ? 1 : 0;
 #pragma unroll
@@ -3480,7 +3649,28 @@ int launch_sort(unsigned long long* keys, int S, int32_t* order, int* tie_flag, 
     return npad;
 }
 
-size_t tile_scratch_ints(int ntiles) { return 66 + 3 * (size_t)ntiles + 2; }
+// How a trace's tiles are cut into items:
+//   * front-to-back composites: a pixel stops after a few fragments whatever
+//     is binned behind them, so every tile is cut alike, and only where the
+//     whole tiles leave the device idle: a wave of a 64-pixel tile takes
+//     200 us of dependent steps, which 3600 tiles (640 x 360) do not hide
+//     (plain256's cone: 225 us whole, 142 in halves, 104 in quarters, 115 in
+//     eighths), while at 32 400 tiles the device is full and parts only march
+//     more beyond the pixels' ends (234 whole, 232 in halves, 342 in quarters
+//     alone; the frame among others 379 us whole, 387 in halves);
+//   * GL blending marches every fragment, so a tile costs what is binned into
+//     it, and the heaviest (a clump's centre) were the tail: cut by weight.
+static TileSplit tile_split_rule(int ntiles, bool every_fragment) {
+    TileSplit sp;
+    sp.inv_slots = 1.0f / 12288.0f;  // two rounds of the 6144 waves that fit the device
+    sp.fixed = every_fragment ? -1 : ntiles <= 8192 ? 2 : ntiles <= 16384 ? 1 : 0;
+    sp.budget = every_fragment ? std::max(ntiles, 16384) : ntiles * ((1 << sp.fixed) - 1);
+    return sp;
+}
+size_t tile_scratch_ints(int ntiles) {
+    return 66 + 3 * (size_t)ntiles + 2 +
+           (size_t)std::max(tile_split_rule(ntiles, true).budget, tile_split_rule(ntiles, false).budget);
+}
 
 void launch_bin_counts(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int words,
                        unsigned long long* masks, int* tile_count, hipStream_t s) {
@@ -3498,16 +3688,19 @@ void launch_tile_order(const int* tile_count, int ntiles, int* scratch, int* til
     hipLaunchKernelGGL(k_tile_bucket, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, tile_count, ntiles, bucket_of,
                        hist);
     hipLaunchKernelGGL(k_tile_scatter, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, bucket_of, ntiles, hist, cursor,
-                       tile_order);
+                       tile_order, TileSplit{0.0f, 0, 0}, (int*)nullptr);
 }
 
-// Binning plus the heavy-first tile order.  tile scratch (ints): hist[32] |
-// cursor[32] | (2 unused) | tile_count[ntiles] | bucket_of | tile_order.  The
-// masks and the scratch up to tile_count are cleared by one fill launch.
+// Binning plus the heavy-first item order.  tile scratch (ints): hist[32] |
+// cursor[32] | item total, 1 unused | tile_count[ntiles] | bucket_of | items.
+// The masks and the scratch up to tile_count are cleared by one fill launch.
+// every_fragment: the composite blends all of a pixel's fragments (a
+// front-to-back one stops after a few, whatever is binned behind them).
 TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int tiles_y, int words,
-                     unsigned long long* masks, int* scratch, hipStream_t s) {
+                     unsigned long long* masks, int* scratch, bool every_fragment, hipStream_t s) {
     const int ntiles = tiles_x * tiles_y;
-    unsigned int* counter = (unsigned int*)(scratch + 64);
+    int* total = scratch + 64;
+    const TileSplit sp = tile_split_rule(ntiles, every_fragment);
     int* tile_count = scratch + 66;
     int* tile_order = tile_count + 2 * (size_t)ntiles;
     const FillSeg segs[2] = {{(uint64_t*)masks, (uint64_t)ntiles * (uint64_t)words, 0},
@@ -3520,11 +3713,8 @@ TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int til
     hipLaunchKernelGGL(k_tile_bucket, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, tile_count, ntiles, bucket_of,
                        hist);
     hipLaunchKernelGGL(k_tile_scatter, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, bucket_of, ntiles, hist, cursor,
-                       tile_order);
-    TileQueue q;
-    q.counter = counter;
-    q.order = tile_order;
-    return q;
+                       tile_order, sp, total);
+    return TileQueue{total, tile_order, (unsigned)(ntiles + sp.budget)};
 }
 
 template <int FMT, int CONE, int COMP>
@@ -3555,10 +3745,9 @@ void launch_cone_batch(const BatchScene* scenes, const int* tile0, int nscenes, 
     else go(std::integral_constant<int, 2>{});
 }
 
-// dynamic LDS of k_cone_tab: the tables and, per wave, kConeChunk coverage
-// masks (8 bytes) and billboard ids (4 bytes)
+// dynamic LDS of k_cone_tab: the tables and the waves' candidate lists
 static size_t cone_tab_lds_bytes_for(const ConeTab& t, int wpg) {
-    return (size_t)t.words * 4u + (size_t)wpg * kConeChunk * (8u + 4u);
+    return (size_t)t.words * 4u + (size_t)wpg * sizeof(ConeLds);
 }
 size_t cone_tab_lds_bytes(const ConeTab& t) { return cone_tab_lds_bytes_for(t, t.wpg); }
 
@@ -3589,28 +3778,29 @@ bool cone_tab_plan(const VolumeDesc& vd, ConeTab& t) {
 // kernels keep their register budget.
 template <int FMT, int CONE, int COMP, int LEARNED>
 static void launch_cone_t(const ConeLaunch& a, hipStream_t s) {
-    unsigned ntiles = (unsigned)(a.cv.tiles_x * a.cv.tiles_y);
+    // at most; workgroups past the item total end at once
+    const unsigned nitems = a.items.bound;
     if constexpr (!LEARNED && CONE == 1 && FMT != 0) {
         ConeTab t;
         if (!a.nmap && a.table_addressing && cone_tab_plan(a.vd, t)) {
-            const unsigned grid = (ntiles + (unsigned)t.wpg - 1u) / (unsigned)t.wpg;
+            const unsigned grid = (nitems + (unsigned)t.wpg - 1u) / (unsigned)t.wpg;
             hipLaunchKernelGGL((k_cone_tab<FMT, COMP>), dim3(grid), dim3(64 * t.wpg), cone_tab_lds_bytes(t), s, a.g,
                                a.vd, a.cv, a.cd, t, a.levels, a.sph_world, a.sph_view, a.order, a.masks, a.words,
-                               a.image, a.counters, a.tile_order, (int)ntiles);
+                               a.image, a.counters, a.items);
             return;
         }
     }
     if constexpr (!LEARNED) {
         if (a.nmap) {
-            hipLaunchKernelGGL((k_cone<FMT, CONE, COMP, 0, 1>), dim3(ntiles), dim3(64), 0, s, a.g, a.vd, a.cv, a.cd,
+            hipLaunchKernelGGL((k_cone<FMT, CONE, COMP, 0, 1>), dim3(nitems), dim3(64), 0, s, a.g, a.vd, a.cv, a.cd,
                                a.levels, a.sph_world, a.sph_view, a.order, a.masks, a.words, a.image, a.counters,
-                               a.tile_order, a.mlp, a.nmap);
+                               a.items, a.mlp, a.nmap);
             return;
         }
     }
-    hipLaunchKernelGGL((k_cone<FMT, CONE, COMP, LEARNED, 0>), dim3(ntiles), dim3(64), 0, s, a.g, a.vd, a.cv, a.cd,
+    hipLaunchKernelGGL((k_cone<FMT, CONE, COMP, LEARNED, 0>), dim3(nitems), dim3(64), 0, s, a.g, a.vd, a.cv, a.cd,
                        a.levels, a.sph_world, a.sph_view, a.order, a.masks, a.words, a.image, a.counters,
-                       a.tile_order, a.mlp, a.nmap);
+                       a.items, a.mlp, a.nmap);
 }
 
 // R8 volumes hold one channel: only the weighted R-sum cone reads them (the

@@ -1107,7 +1107,6 @@ static void fill_cone_desc(cr_volume v, const cr_light* light, const cr_cone_par
     cd.alpha_stop = p->alpha_stop;
     cd.kscale = (p->sigma * (float)1.4426950408889634) / (float)v->N;
     cd.cone_mode = p->cone_mode;
-    cd.count = 1;
     cd.composite = p->composite;
     cd.quantize = (p->composite == CR_COMPOSITE_GL_BLEND && p->quantize_rgba8) ? 1 : 0;
     cd.compensated = p->compensated ? 1 : 0;
@@ -1369,7 +1368,7 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     if (counters) launch_fill_u64((uint64_t*)counters, 9, 0, s);
     cone_enqueue_sort(v, plan, &ev, cs);
     TileQueue tq = launch_bin(v->d_sph_tiles, v->d_order, plan.S, plan.cv.tiles_x, plan.cv.tiles_y, plan.words,
-                              v->d_masks, v->d_tiles, cs);
+                              v->d_masks, v->d_tiles, plan.cd.composite == CR_COMPOSITE_GL_BLEND, cs);
     ev.mark(3);
     if (overlap) {
         CR_HIP(ctx, hipEventRecord(v->ev_cam, cs));
@@ -1381,7 +1380,6 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     cl.vd = v->vd;
     cl.cv = plan.cv;
     cl.cd = plan.cd;
-    cl.cd.count = counters ? 1 : 0;  // the march counts are read only from counter runs
     cl.levels = v->d_levels;
     cl.sph_world = v->d_sph_world;
     cl.sph_view = v->d_sph_view;
@@ -1390,7 +1388,7 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     cl.words = plan.words;
     cl.image = d_image;
     cl.counters = counters;
-    cl.tile_order = tq.order;
+    cl.items = tq;
     cl.learned = lo ? 1 : 0;
     cl.table_addressing = (ctx->flags & CR_CONTEXT_DIRECT_ADDRESSING) ? 0 : 1;
     if (lo) cl.mlp = mlp_dev(lo->mlp);
