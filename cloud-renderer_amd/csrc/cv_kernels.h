@@ -66,6 +66,10 @@ struct VolumeDesc {
     // the density noise of every level-0 texel (level-0 slot order; binary16
     // bits for RGBA16F volumes, float for RGBA32F), or null: computed in the build
     const void* ntex;
+    // R8 volumes: the trilinear footprints of every level (launch_foot_r8), or
+    // null: the cone samples the texels; fbase: first slot of each level
+    const uint2* foot;
+    uint32_t fbase[kMaxLevels];
 };
 
 struct CameraView {
@@ -89,6 +93,9 @@ struct ConeDesc {
     int steps;
     float tanHalf;
     float den;             // steps * downScaling
+    float inv_den;         // 1 / den when den is a power of two (x / den == x * inv_den exactly), else 0
+    int grows;             // den > 0: the weighted sum never shrinks
+    int tail;              // weighted cone: first of the last steps that all read the 1^3 level L - 1 (steps: none)
     float alpha_stop;
     float kscale;          // sigma * log2(e) / N
     int cone_mode;
@@ -113,6 +120,7 @@ struct ConeDesc {
     float nm_step, nm_opacity, nm_freq_step, nm_pers_step, nm_adjust, nm_min_color, nm_color_scale;
     float nm_off[3];
     float nm_ray[3];
+    int nm_full;           // the amplitudes may overflow: the noise's x and z decide whether the light term is a number
     // sun sprite (GL blend composite): view-space centre, colours, radii
     int sun_on;
     float sun_v[3];
@@ -216,6 +224,12 @@ void launch_noise_tex(const GridDesc& g, const VolumeDesc& vd, void* ntex, hipSt
 void launch_build_levels(const GridDesc& g, const VolumeDesc& vd, const unsigned long long* shellbits,
                          const unsigned long long* fillbits, void* levels, uint8_t* zflags, hipStream_t s);
 void launch_mip(const VolumeDesc& vd, int k, void* levels, hipStream_t s);
+// footprint slots of an R8 volume (fills vd.fbase; 0: too many for 32-bit byte
+// offsets) and their build from the shell words and the R8 levels; zero: one
+// byte per level-0 brick, 1 when its slots hold zero
+size_t foot_slots(VolumeDesc& vd);
+void launch_foot_r8(const GridDesc& g, const VolumeDesc& vd, const unsigned long long* shellbits, const void* levels,
+                    uint2* foot, uint8_t* zero, hipStream_t s);
 void launch_cam_setup(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
                       float4* sph_view, int4* sph_tiles, unsigned long long* keys, hipStream_t s);
 size_t sort_scratch_words(int S);

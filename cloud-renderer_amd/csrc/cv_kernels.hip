@@ -212,6 +212,13 @@ __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v)
     return v;
 }
 
+// LDS writes of the wave's lanes before this are seen by its reads after it
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 __global__ void k_fill_u64(uint64_t* __restrict__ p, uint64_t n, uint64_t value) {
     uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
     uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
@@ -1758,6 +1765,93 @@ __global__ void __launch_bounds__(1024) k_mip_tail(VolumeDesc vd, int k0, void* 
 }
 
 // ---------------------------------------------------------------------------
+// footprints of an R8 volume
+//
+// The weighted cone takes 8 texels per level and sample.  As separate byte
+// loads they made the cone 12 ms on plain256's geometry (8 loads, 8 addresses
+// and 8 decodes each); a footprint slot holds all 8 of a texel (x, y, z), its
+// neighbours x+ = min(x + 1, n - 1) etc., so a sample is one 8-byte load.
+// Byte x + 2 y + 4 z = corner; level 0 (all shell or empty) holds 0 / 1 (its
+// samples need no division), the others the R8 bytes.  Slots are x-fastest:
+// two multiply-adds address one.
+// ---------------------------------------------------------------------------
+// 16 level-0 bricks per wave (4 waves per workgroup), then the upper levels,
+// a texel per thread.  Empty bricks (own and neighbour words 0) whose slots
+// already hold zero are skipped, so the launch writes the shell's slots and
+// reads words (8 + 1 bytes per brick) for the rest.
+constexpr int kFootBricks = 16;
+__global__ void __launch_bounds__(256) k_foot_r8(GridDesc g, VolumeDesc vd,
+                                                 const unsigned long long* __restrict__ shellbits,
+                                                 const uint8_t* __restrict__ levels, uint2* __restrict__ foot,
+                                                 uint8_t* __restrict__ zero, uint32_t nbricks, uint32_t groups0) {
+    if (blockIdx.x < groups0) {
+        __shared__ unsigned long long words[4][kFootBricks][8];
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const uint32_t nb = g.nb0, n = (uint32_t)g.N;
+        const uint32_t b0 = (blockIdx.x * 4u + (uint32_t)wave) * (uint32_t)kFootBricks;
+        bool need = false;
+        if (lane < kFootBricks && b0 + lane < nbricks) {
+            const uint32_t b = b0 + lane, bx = b % nb, by = (b / nb) % nb, bz = b / (nb * nb);
+            unsigned long long any = 0ull;
+#pragma unroll
+            for (uint32_t q = 0; q < 8; ++q) {
+                const uint32_t cx = min(bx + (q & 1u), nb - 1u), cy = min(by + ((q >> 1) & 1u), nb - 1u);
+                const uint32_t cz = min(bz + (q >> 2), nb - 1u);
+                const unsigned long long w = shellbits[(cz * nb + cy) * nb + cx];
+                words[wave][lane][q] = w;
+                any |= w;
+            }
+            need = any != 0ull || zero[b] == 0;
+            if (need) zero[b] = any ? 0 : 1;
+        }
+        wave_lds_sync();
+        uint32_t lx, ly, lz;
+        demorton6((uint32_t)lane, &lx, &ly, &lz);
+        unsigned long long todo = __ballot(need);
+        while (todo) {
+            const uint32_t k = (uint32_t)__ffsll((long long)todo) - 1u;
+            todo &= todo - 1ull;
+            const uint32_t b = b0 + k, bx = b % nb, by = (b / nb) % nb, bz = b / (nb * nb);
+            const uint32_t x = bx * 4u + lx, y = by * 4u + ly, z = bz * 4u + lz;
+            if (x >= n || y >= n || z >= n) continue;
+            uint32_t lo = 0, hi = 0;
+#pragma unroll
+            for (uint32_t c = 0; c < 8; ++c) {
+                const uint32_t X = min(x + (c & 1u), n - 1u), Y = min(y + ((c >> 1) & 1u), n - 1u);
+                const uint32_t Z = min(z + (c >> 2), n - 1u);
+                const uint32_t q = ((X >> 2) - bx) + 2u * ((Y >> 2) - by) + 4u * ((Z >> 2) - bz);
+                const uint32_t bit = (uint32_t)(words[wave][k][q] >> morton6(X & 3u, Y & 3u, Z & 3u)) & 1u;
+                if (c < 4) lo |= bit << (8u * c);
+                else hi |= bit << (8u * (c - 4u));
+            }
+            foot[x + n * (y + n * z)] = make_uint2(lo, hi);
+        }
+        return;
+    }
+    uint64_t t = (uint64_t)(blockIdx.x - groups0) * 256u + threadIdx.x;
+    for (int k = 1; k < vd.L; ++k) {
+        const LevelDesc& Lv = vd.lv[k];
+        const uint32_t n = Lv.n;
+        const uint64_t cnt = (uint64_t)n * n * n;
+        if (t < cnt) {
+            const uint32_t x = (uint32_t)t % n, y = ((uint32_t)t / n) % n, z = (uint32_t)t / (n * n);
+            uint32_t lo = 0, hi = 0;
+#pragma unroll
+            for (uint32_t c = 0; c < 8; ++c) {
+                const uint32_t X = min(x + (c & 1u), n - 1u), Y = min(y + ((c >> 1) & 1u), n - 1u);
+                const uint32_t Z = min(z + (c >> 2), n - 1u);
+                const uint32_t v = levels[brick_addr(Lv, X, Y, Z)];
+                if (c < 4) lo |= v << (8u * c);
+                else hi |= v << (8u * (c - 4u));
+            }
+            foot[vd.fbase[k] + (uint32_t)t] = make_uint2(lo, hi);
+            return;
+        }
+        t -= cnt;
+    }
+}
+
+// ---------------------------------------------------------------------------
 // camera pass setup: world/view centres, draw-order key, tile box
 // ---------------------------------------------------------------------------
 // sort key of billboard j for CloudVolume::sortBoards(point): the distance
@@ -2261,10 +2355,14 @@ __global__ void __launch_bounds__(256) k_tile_scatter(const int* __restrict__ bu
 // A trilinear footprint then takes one slot per y/z corner (4 loads, not 8);
 // readback rebuilds RGBA as (r, r, r, a).
 
+// byte / 255 correctly rounded for byte in [0, 255]: 1 / 255 split into its
+// float and the rest, all 256 quotients equal the division's
+__device__ __forceinline__ float div255(float b) { return fmaf(b, 0x1.010102p-8f, b * -0x1.fdfdfep-33f); }
+
 // r of one texel (R8, or the r of an RGBA slot)
 template <int FMT>
 __device__ __forceinline__ float fetch1(const void* __restrict__ vol, uint64_t i) {
-    if (FMT == 0) return (float)((const uint8_t*)vol)[i] / 255.0f;
+    if (FMT == 0) return div255((float)((const uint8_t*)vol)[i]);
     if (FMT == 1) return ((const float*)vol)[i * 4];
     return h2f(((const unsigned short*)vol)[i * 4]);
 }
@@ -2329,6 +2427,37 @@ __device__ __forceinline__ float trilinear_r(const void* __restrict__ vol, const
     float c01 = lerpF(t001, t101, wx), c11 = lerpF(t011, t111, wx);
     float c0 = lerpF(c00, c10, wy), c1 = lerpF(c01, c11, wy);
     return lerpF(c0, c1, wz);
+}
+
+// GL trilinear filtering (CLAMP_TO_EDGE) of an R8 level from its footprint
+// slots: trilinear_r's result bit for bit.  The texel coordinate is clamped to
+// [0, n - 1]: below the first texel's centre both corners are texel 0 and any
+// weight returns it exactly, as the clamped coordinate's weight 0 does; above
+// the last likewise (its slot's corners coincide).
+template <bool LEVEL0>
+__device__ __forceinline__ float trilinear_foot(const uint2* __restrict__ lvl, uint32_t n, float fn, float sx,
+                                                float sy, float sz) {
+    const float top = fn - 1.0f;
+    const float ux = __builtin_amdgcn_fmed3f(fmaf(sx, fn, -0.5f), 0.0f, top);
+    const float uy = __builtin_amdgcn_fmed3f(fmaf(sy, fn, -0.5f), 0.0f, top);
+    const float uz = __builtin_amdgcn_fmed3f(fmaf(sz, fn, -0.5f), 0.0f, top);
+    const float wx = __builtin_amdgcn_fractf(ux), wy = __builtin_amdgcn_fractf(uy), wz = __builtin_amdgcn_fractf(uz);
+    // n <= 768: n^2 fits the 24-bit multiplier
+    const uint32_t i = __umul24(__umul24((uint32_t)uz, n) + (uint32_t)uy, n) + (uint32_t)ux;
+    const uint2 t = lvl[i];
+    auto dec = [](uint32_t w, int c) {
+        const float b = (float)((w >> (8 * c)) & 0xffu);
+        return LEVEL0 ? b : div255(b);
+    };
+    const float c00 = lerpF(dec(t.x, 0), dec(t.x, 1), wx), c10 = lerpF(dec(t.x, 2), dec(t.x, 3), wx);
+    const float c01 = lerpF(dec(t.y, 0), dec(t.y, 1), wx), c11 = lerpF(dec(t.y, 2), dec(t.y, 3), wx);
+    return lerpF(lerpF(c00, c10, wy), lerpF(c01, c11, wy), wz);
+}
+__device__ __forceinline__ float foot_level(const VolumeDesc& vd, int k, float sx, float sy, float sz) {
+    const uint2* lvl = vd.foot + vd.fbase[k];
+    const uint32_t n = vd.lv[k].n;
+    const float fn = vd.lv[k].fn;
+    return k == 0 ? trilinear_foot<true>(lvl, n, fn, sx, sy, sz) : trilinear_foot<false>(lvl, n, fn, sx, sy, sz);
 }
 
 // Grey sampling split into fetch and filter, so a two-level sample issues
@@ -2659,12 +2788,64 @@ __device__ __forceinline__ void farfield_features(const VolumeDesc& vd, const vo
     }
 }
 
-// Cone start and direction of the fragment that billboard (cw: world centre
-// and radius, vv: view-space centre) leaves at the pixel with view ray
-// (rx, ry), where its sphere contribution sc = sphere_contrib(du, dv, s).
 struct ConeFrag {
     float p0x, p0y, p0z, dx, dy, dz;
 };
+
+// The weighted cone (res/conetrace_frag.glsl:64-79): sum of s.r * (i + 1) / den
+// over every step.  FMT 3: an R8 volume with footprint slots.
+//
+// Two parts of the sum need no sampling.  Once every further step reads the
+// one texel of the 1^3 level (cd.tail; past step 55 of 256 on plain256) its
+// value is the same everywhere, and 0 adds nothing.  And the sum of a positive
+// den never shrinks, so when `sat` * sum has reached 1 (sat > 0: what the
+// caller multiplies the sum by before clamping it to 1) the rest cannot
+// change the clamped product; a wave stops once that holds for all its lanes.
+template <int FMT>
+__device__ __forceinline__ float march_weighted(const VolumeDesc& vd, const void* __restrict__ vol, const ConeDesc& cd,
+                                                bool count, const ConeFrag& f, float sat, uint32_t& ntwo) {
+    float color = 0.0f;
+    auto add = [&](float v, int i) {
+        const float x = v * (float)(i + 1);
+        color = color + (cd.inv_den != 0.0f ? x * cd.inv_den : x / cd.den);
+    };
+    const bool cut = cd.grows && sat > 0.0f && !count;
+    auto full = [&]() { return __ballot(!(cut && color * sat >= 1.0f)) == 0ull; };
+    int i = 0;
+    const int tail = FMT == 3 ? cd.tail : cd.steps;
+    for (; i < tail; ++i) {
+        const float h = cd.h[i], fr = cd.lfrac[i];
+        const int lv = step_level(cd, i);
+        const float sx = fmaf(h, f.dx, f.p0x), sy = fmaf(h, f.dy, f.p0y), sz = fmaf(h, f.dz, f.p0z);
+        const bool two = (__float_as_uint(fr) << 1) != 0u;
+        float v;
+        if constexpr (FMT == 3) {
+            v = foot_level(vd, lv, sx, sy, sz);
+            if (two) v = lerpF(v, foot_level(vd, lv + 1, sx, sy, sz), fr);
+        } else {
+            bool t2;
+            v = sample_lod<FMT, 1>(vol, vd, lv, fr, sx, sy, sz, &t2).x;
+        }
+        ntwo += two ? 1u : 0u;
+        add(v, i);
+        if ((i & 3) == 3 && full()) return color;
+    }
+    if (i < cd.steps) {
+        const int k = vd.L - 1;
+        const uint32_t w = vd.foot[vd.fbase[k]].x & 0xffu;
+        const float v = k == 0 ? (float)w : div255((float)w);
+        if (v != 0.0f)
+            for (; i < cd.steps; ++i) {
+                add(v, i);
+                if ((i & 7) == 7 && full()) break;
+            }
+    }
+    return color;
+}
+
+// Cone start and direction of the fragment that billboard (cw: world centre
+// and radius, vv: view-space centre) leaves at the pixel with view ray
+// (rx, ry), where its sphere contribution sc = sphere_contrib(du, dv, s).
 __device__ __forceinline__ ConeFrag cone_frag(const GridDesc& g, const CameraView& cv, const ConeDesc& cd, float4 cw,
                                               float du, float dv, float sc, float fN) {
     const float s = cw.w;
@@ -2703,8 +2884,8 @@ __device__ __forceinline__ void blend_frag(const ConeDesc& cd, float s0, float s
         C2 = s2 * al + C2 * om;
         C3 = s3 * al + C3 * om;
         if (cd.quantize) {
-            C0 = (float)q8(C0) / 255.0f; C1 = (float)q8(C1) / 255.0f;
-            C2 = (float)q8(C2) / 255.0f; C3 = (float)q8(C3) / 255.0f;
+            C0 = div255((float)q8(C0)); C1 = div255((float)q8(C1));
+            C2 = div255((float)q8(C2)); C3 = div255((float)q8(C3));
         }
     } else {
         const float wgt = (1.0f - C3) * s3;
@@ -2725,27 +2906,30 @@ __device__ __forceinline__ int nm_wrap(float fl) {
     const float r = fl - 32.0f * floorf(fl * 0.03125f);
     return (r == r ? (int)r : 0) & 31;
 }
-// texture(noiseMap, s): GL_LINEAR, GL_REPEAT on the 32^3 map of decoded
-// RGBA8_SNORM texels (x fastest); u = fma(s, 32, -1/2), alpha = u - floor(u),
-// lerps along x, then y, then z
-__device__ __forceinline__ float4 nm_tex(const float4* __restrict__ map, float sx, float sy, float sz) {
+// texture(noiseMap, s) of two channels: GL_LINEAR, GL_REPEAT on the 32^3 map of
+// decoded RGBA8_SNORM texels (x fastest); u = fma(s, 32, -1/2),
+// alpha = u - floor(u), lerps along x, then y, then z.  A texel of the map holds
+// the two channels of x and of x + 1 (wrapped), so a footprint is 4 loads.
+__device__ __forceinline__ float2 nm_tex(const float4* __restrict__ map, float sx, float sy, float sz) {
     const float ux = fmaf(sx, 32.0f, -0.5f), uy = fmaf(sy, 32.0f, -0.5f), uz = fmaf(sz, 32.0f, -0.5f);
     const float fx = floorf(ux), fy = floorf(uy), fz = floorf(uz);
     const float ax = ux - fx, ay = uy - fy, az = uz - fz;
-    const int x0 = nm_wrap(fx), y0 = nm_wrap(fy), z0 = nm_wrap(fz);
-    const int x1 = (x0 + 1) & 31, y1 = (y0 + 1) & 31, z1 = (z0 + 1) & 31;
-    const int r00 = (z0 * 32 + y0) * 32, r10 = (z0 * 32 + y1) * 32, r01 = (z1 * 32 + y0) * 32, r11 = (z1 * 32 + y1) * 32;
-    const float4 t000 = map[r00 + x0], t100 = map[r00 + x1], t010 = map[r10 + x0], t110 = map[r10 + x1];
-    const float4 t001 = map[r01 + x0], t101 = map[r01 + x1], t011 = map[r11 + x0], t111 = map[r11 + x1];
+    int x0, y0, z0;
+    if (fabsf(ux) < 1e9f && fabsf(uy) < 1e9f && fabsf(uz) < 1e9f) {  // the conversion is exact: & 31 is mod 32
+        x0 = (int)fx & 31; y0 = (int)fy & 31; z0 = (int)fz & 31;
+    } else {
+        x0 = nm_wrap(fx); y0 = nm_wrap(fy); z0 = nm_wrap(fz);
+    }
+    const int y1 = (y0 + 1) & 31, z1 = (z0 + 1) & 31;
+    const float4 q0 = map[(z0 << 10) + (y0 << 5) + x0], q1 = map[(z0 << 10) + (y1 << 5) + x0];
+    const float4 q2 = map[(z1 << 10) + (y0 << 5) + x0], q3 = map[(z1 << 10) + (y1 << 5) + x0];
     auto tri = [&](float a000, float a100, float a010, float a110, float a001, float a101, float a011, float a111) {
         const float c00 = lerpF(a000, a100, ax), c10 = lerpF(a010, a110, ax);
         const float c01 = lerpF(a001, a101, ax), c11 = lerpF(a011, a111, ax);
         return lerpF(lerpF(c00, c10, ay), lerpF(c01, c11, ay), az);
     };
-    return make_float4(tri(t000.x, t100.x, t010.x, t110.x, t001.x, t101.x, t011.x, t111.x),
-                       tri(t000.y, t100.y, t010.y, t110.y, t001.y, t101.y, t011.y, t111.y),
-                       tri(t000.z, t100.z, t010.z, t110.z, t001.z, t101.z, t011.z, t111.z),
-                       tri(t000.w, t100.w, t010.w, t110.w, t001.w, t101.w, t011.w, t111.w));
+    return make_float2(tri(q0.x, q0.z, q1.x, q1.z, q2.x, q2.z, q3.x, q3.z),
+                       tri(q0.y, q0.w, q1.y, q1.w, q2.y, q2.w, q3.y, q3.w));
 }
 // glm dot: (x*x' + y*y') + z*z'
 __device__ __forceinline__ float nm_dot(float ax, float ay, float az, float bx, float by, float bz) {
@@ -2793,8 +2977,13 @@ __device__ __forceinline__ bool noise_fragment(const float4* __restrict__ map, c
         float freq = 1.0f, pers = 1.0f;
         for (int o = 0; o < cd.nm_octaves; ++o) {
             const float off = o < 3 ? cd.nm_off[o] : 0.0f;
-            const float4 t = nm_tex(map, (cx + off) * freq, (cy + off) * freq, (cz + off) * freq);
-            n0 = n0 + pers * t.x; n1 = n1 + pers * t.y; n2 = n2 + pers * t.z; n3 = n3 + pers * t.w;
+            const float tx = (cx + off) * freq, ty = (cy + off) * freq, tz = (cz + off) * freq;
+            const float2 t = nm_tex(map, tx, ty, tz);
+            n1 = n1 + pers * t.x; n3 = n3 + pers * t.y;
+            if (cd.nm_full) {
+                const float2 u = nm_tex(map + 32 * 32 * 32, tx, ty, tz);
+                n0 = n0 + pers * u.x; n2 = n2 + pers * u.y;
+            }
             freq = freq * cd.nm_freq_step;
             pers = pers * cd.nm_pers_step;
         }
@@ -2827,13 +3016,6 @@ struct ConeLds {
     float4 vv[kConeChunk];  // view-space centre, radius
     int rank[kConeChunk];   // draw ranks
 };
-
-// LDS writes of the wave's lanes before this are seen by its reads after it
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
 
 // The next (at most 64) binned billboards of a tile in draw order (front to
 // back for COMP = 1, back to front for COMP = 0) into L; returns how many, 0
@@ -2952,8 +3134,8 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
     if (COMP == 0) {
         C0 = cd.clear[0]; C1 = cd.clear[1]; C2 = cd.clear[2]; C3 = cd.clear[3];
         if (cd.quantize) {
-            C0 = (float)q8(C0) / 255.0f; C1 = (float)q8(C1) / 255.0f;
-            C2 = (float)q8(C2) / 255.0f; C3 = (float)q8(C3) / 255.0f;
+            C0 = div255((float)q8(C0)); C1 = div255((float)q8(C1));
+            C2 = div255((float)q8(C2)); C3 = div255((float)q8(C3));
         }
         if (cd.sun_on && valid) {
             // the sun sprite, blended over the clear colour before the clouds
@@ -3065,15 +3247,8 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
             }
             if (have) {
                 if constexpr (CONE == 0) {
-                    float color = 0.0f;
-                    for (int i = 0; i < cd.steps; ++i) {
-                        const float h = cd.h[i];
-                        bool two;
-                        float4 sm = sample_lod<FMT, 1>(vol, vd, step_level(cd, i), cd.lfrac[i], fmaf(h, f.dx, f.p0x), fmaf(h, f.dy, f.p0y),
-                                                       fmaf(h, f.dz, f.p0z), &two);
-                        n2 += two ? 1u : 0u;
-                        color = color + (sm.x * (float)(i + 1)) / cd.den;
-                    }
+                    // nm_col below multiplies the sum before the clamp
+                    const float color = march_weighted<FMT>(vd, vol, cd, count, f, NM ? nm_col : 1.0f, n2);
                     ns = (uint32_t)cd.steps;
                     s0 = s1 = s2 = s3 = clamp01(color);
                     s0u = color;
@@ -3567,6 +3742,24 @@ void launch_build_levels(const GridDesc& g, const VolumeDesc& vd, const unsigned
     if (k < vd.L) hipLaunchKernelGGL(k_mip_tail, dim3(1), dim3(1024), 0, s, vd, k, levels);
 }
 
+size_t foot_slots(VolumeDesc& vd) {
+    if (vd.format != 0 || vd.lv[0].n > 768) return 0;  // trilinear_foot's 24-bit products and 32-bit byte offsets
+    size_t n = 0;
+    for (int k = 0; k < vd.L; ++k) {
+        vd.fbase[k] = (uint32_t)n;
+        n += (size_t)vd.lv[k].n * vd.lv[k].n * vd.lv[k].n;
+    }
+    return n;
+}
+void launch_foot_r8(const GridDesc& g, const VolumeDesc& vd, const unsigned long long* shellbits, const void* levels,
+                    uint2* foot, uint8_t* zero, hipStream_t s) {
+    const uint32_t nbricks = g.nb0 * g.nb0 * g.nb0, groups0 = blocks_for(nbricks, 4 * kFootBricks);
+    uint64_t upper = 0;
+    for (int k = 1; k < vd.L; ++k) upper += (uint64_t)vd.lv[k].n * vd.lv[k].n * vd.lv[k].n;
+    hipLaunchKernelGGL(k_foot_r8, dim3(groups0 + blocks_for(upper, 256)), dim3(256), 0, s, g, vd, shellbits,
+                       (const uint8_t*)levels, foot, zero, nbricks, groups0);
+}
+
 void launch_mip(const VolumeDesc& vd, int k, void* levels, hipStream_t s) {
     uint32_t nb = vd.lv[k].nb;
     uint32_t ntex = nb * nb * nb * 64u;
@@ -3808,9 +4001,9 @@ static void launch_cone_t(const ConeLaunch& a, hipStream_t s) {
 template <int FMT>
 static void launch_cone_f(const ConeLaunch& a, hipStream_t s) {
     const bool weighted = a.cd.cone_mode == 0;
-    if constexpr (FMT == 0) {
-        if (a.cd.composite == 0) launch_cone_t<0, 0, 0, 0>(a, s);
-        else launch_cone_t<0, 0, 1, 0>(a, s);
+    if constexpr (FMT == 0 || FMT == 3) {
+        if (a.cd.composite == 0) launch_cone_t<FMT, 0, 0, 0>(a, s);
+        else launch_cone_t<FMT, 0, 1, 0>(a, s);
     } else {
         if (a.learned) launch_cone_t<FMT, 1, 1, 1>(a, s);
         else if (weighted && a.cd.composite == 0) launch_cone_t<FMT, 0, 0, 0>(a, s);
@@ -3821,7 +4014,8 @@ static void launch_cone_f(const ConeLaunch& a, hipStream_t s) {
 }
 
 void launch_cone(const ConeLaunch& a, hipStream_t s) {
-    if (a.vd.format == 0) launch_cone_f<0>(a, s);
+    if (a.vd.format == 0 && a.vd.foot) launch_cone_f<3>(a, s);
+    else if (a.vd.format == 0) launch_cone_f<0>(a, s);
     else if (a.vd.format == 1) launch_cone_f<1>(a, s);
     else launch_cone_f<2>(a, s);
 }

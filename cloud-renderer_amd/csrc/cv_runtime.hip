@@ -78,7 +78,7 @@ struct cr_volume_s {
     cr_context ctx = nullptr;
     int N = 0, L = 0, format = 0, mode = 0;
     // soft-particle noise march: parameters, the map's bytes and its decoded
-    // texels on the device (null while the march is off)
+    // texel pairs on the device (null while the march is off)
     bool nm_on = false;
     cr_noise_march nm{};
     std::vector<int8_t> nm_bytes;
@@ -101,6 +101,10 @@ struct cr_volume_s {
     void* d_ntex = nullptr;  // density noise texture (vd.ntex), rebuilt by cr_volume_set_noise
     size_t ntex_cap = 0;
     size_t zflags_bytes = 0;
+    // R8 volumes: per set the cone's footprint slots and the level-0 bricks'
+    // zero flags (null without room for them: the cone samples the texels)
+    uint2* d_foot[2] = {nullptr, nullptr};
+    uint8_t* d_fzero[2] = {nullptr, nullptr};
     int cur = 0;
     bool lset_failed = false;
     hipEvent_t ev_release[2] = {nullptr, nullptr};
@@ -538,6 +542,24 @@ int cr_get_stats(cr_context ctx, cr_stats* out) {
     return CR_OK;
 }
 
+// footprint slots of level set `set` of an R8 volume, zeroed on s; without room
+// for them the set keeps none and the cone samples its texels
+static void foot_alloc(cr_volume v, int set, hipStream_t s) {
+    const size_t n = foot_slots(v->vd);
+    if (n == 0) return;
+    const size_t zb = ((size_t)v->nbricks0 + 7) & ~(size_t)7;
+    if (hipMalloc((void**)&v->d_foot[set], n * sizeof(uint2)) != hipSuccess ||
+        hipMalloc((void**)&v->d_fzero[set], zb) != hipSuccess) {
+        (void)hipGetLastError();
+        if (v->d_foot[set]) (void)hipFree(v->d_foot[set]);
+        v->d_foot[set] = nullptr;
+        v->d_fzero[set] = nullptr;
+        return;
+    }
+    launch_fill_u64((uint64_t*)v->d_foot[set], n, 0, s);
+    launch_fill_u64((uint64_t*)v->d_fzero[set], zb / 8, 0x0101010101010101ull, s);
+}
+
 int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const float bounds_hi[3],
                      const float position[3], int levels, int format, int mode, cr_volume* out) {
     if (!ctx || !out || !bounds_lo || !bounds_hi || !position)
@@ -620,6 +642,7 @@ int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const fl
         return fail(ctx, e == hipErrorOutOfMemory ? CR_ENOMEM : CR_EDEVICE, "cr_volume_create: hipMalloc: %s",
                     hipGetErrorString(e));
     }
+    foot_alloc(v, 0, nullptr);
     // zero the volume so reads before the first voxelize are defined
     launch_fill_u64((uint64_t*)v->d_levels, v->levels_bytes / 8, 0, nullptr);
     if (v->d_zflags[0]) launch_fill_u64((uint64_t*)v->d_zflags[0], v->zflags_bytes / 8, 0x0101010101010101ull, nullptr);
@@ -643,7 +666,7 @@ int cr_volume_destroy(cr_volume v) {
                          v->ev_release[1], v->ev_bfree[0], v->ev_bfree[1], v->ev_items, v->ev_lfree[0],
                          v->ev_lfree[1]})
         if (e) (void)hipEventDestroy(e);
-    void* ptrs[] = {v->d_lset[0], v->d_lset[1], v->d_zflags[0], v->d_zflags[1], v->d_shell_s[0], v->d_shell_s[1], v->d_fill_s[0], v->d_fill_s[1],    v->d_boards,    v->d_keys,      v->d_posmap,
+    void* ptrs[] = {v->d_lset[0], v->d_lset[1], v->d_zflags[0], v->d_zflags[1], v->d_foot[0], v->d_foot[1], v->d_fzero[0], v->d_fzero[1], v->d_shell_s[0], v->d_shell_s[1], v->d_fill_s[0], v->d_fill_s[1],    v->d_boards,    v->d_keys,      v->d_posmap,
                     v->d_lbox,   v->d_lcounts, v->d_litems,  v->d_sph_world, v->d_sph_view,  v->d_sph_tiles,
                     v->d_sort,   v->d_order,   v->d_tie,     v->d_masks,     v->d_counters,  v->d_scratch, v->d_tiles,
                     v->cam_spare.sph_world, v->cam_spare.sph_view, v->cam_spare.sph_tiles, v->cam_spare.sort,
@@ -774,11 +797,16 @@ int cr_volume_set_noise_march(cr_volume v, const cr_noise_march* nm) {
     if (!v->d_nmap || !v->nm_on || v->nm.seed != nm->seed || v->nm_bytes.empty()) {
         std::vector<int8_t> m;
         noise_map_build(nm->seed, m);
-        // decoded texels: RGBA8_SNORM -> max(c / 127, -1) (GL 4.4 eq. 2.2)
-        std::vector<float4> t(m.size() / 4);
-        for (size_t i = 0; i < t.size(); ++i)
-            t[i] = make_float4(std::max((float)m[4 * i] / 127.0f, -1.0f), std::max((float)m[4 * i + 1] / 127.0f, -1.0f),
-                               std::max((float)m[4 * i + 2] / 127.0f, -1.0f), std::max((float)m[4 * i + 3] / 127.0f, -1.0f));
+        // decoded texels: RGBA8_SNORM -> max(c / 127, -1) (GL 4.4 eq. 2.2), two
+        // channels of x and x + 1 per texel: (y, w), then the map of (x, z)
+        const size_t n = m.size() / 4;
+        std::vector<float4> t(2 * n);
+        auto dec = [&](size_t i, int c) { return std::max((float)m[4 * i + c] / 127.0f, -1.0f); };
+        for (size_t i = 0; i < n; ++i) {
+            const size_t j = (i & ~(size_t)31) | ((i + 1) & 31);
+            t[i] = make_float4(dec(i, 1), dec(i, 3), dec(j, 1), dec(j, 3));
+            t[n + i] = make_float4(dec(i, 0), dec(i, 2), dec(j, 0), dec(j, 2));
+        }
         // cone traces still queued may read the old map
         CR_HIP(ctx, hipDeviceSynchronize());
         if (!v->d_nmap) CR_HIP(ctx, hipMalloc((void**)&v->d_nmap, t.size() * sizeof(float4)));
@@ -960,6 +988,7 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
     if (ev) ev->mark_on(5, bs);
     launch_build_levels(v->g, v->vd, shell, v->mode == CR_MODE_RGBA ? fill : nullptr, v->d_lset[set],
                         v->d_zflags[set], bs);
+    if (v->d_foot[set]) launch_foot_r8(v->g, v->vd, shell, v->d_lset[set], v->d_foot[set], v->d_fzero[set], bs);
     if (ev) ev->mark_on(4, bs);
 }
 
@@ -1008,6 +1037,7 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
                 v->d_fill_s[1] = fl;
                 launch_fill_u64((uint64_t*)p, v->levels_bytes / 8, 0, s);
                 if (z) launch_fill_u64((uint64_t*)z, v->zflags_bytes / 8, 0x0101010101010101ull, s);
+                foot_alloc(v, 1, s);
                 v->s_sync_needed = true;  // the streams wait for these fills
             }
         }
@@ -1104,6 +1134,18 @@ static void fill_cone_desc(cr_volume v, const cr_light* light, const cr_cone_par
         h = h + r;
     }
     cd.den = (float)p->steps * p->down_scaling;
+    int den_exp;
+    const float den_abs = std::fabs(cd.den);
+    cd.inv_den = den_abs >= 0x1p-125f && den_abs <= 0x1p125f && std::frexp(den_abs, &den_exp) == 0.5f ? 1.0f / cd.den : 0.0f;
+    cd.grows = cd.den > 0.0f ? 1 : 0;
+    cd.tail = p->steps;
+    if (v->vd.lv[v->L - 1].n == 1)
+        while (cd.tail > 0) {
+            const int i = cd.tail - 1;
+            const int lv = (int)((cd.llev4[i >> 2] >> (8 * (i & 3))) & 0xffu);
+            if (lv != v->L - 1 || cd.lfrac[i] != 0.0f) break;
+            cd.tail = i;
+        }
     cd.alpha_stop = p->alpha_stop;
     cd.kscale = (p->sigma * (float)1.4426950408889634) / (float)v->N;
     cd.cone_mode = p->cone_mode;
@@ -1378,6 +1420,7 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     ConeLaunch cl{};
     cl.g = v->g;
     cl.vd = v->vd;
+    cl.vd.foot = v->d_foot[v->cur];
     cl.cv = plan.cv;
     cl.cd = plan.cd;
     cl.levels = v->d_levels;
@@ -1426,6 +1469,12 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
         // viewRay = normalize(vec3(V[0][2], V[1][2], V[2][2])) (res/conetrace_frag.glsl:138)
         const F3 ray = norm3(f3(cl.cv.V[2], cl.cv.V[6], cl.cv.V[10]));
         cd.nm_ray[0] = ray.x; cd.nm_ray[1] = ray.y; cd.nm_ray[2] = ray.z;
+        float pers = 1.0f, sum = 0.0f;
+        for (int o = 0; o < v->nm.octaves; ++o) {
+            sum += std::fabs(pers);
+            pers = pers * v->nm.pers_step;
+        }
+        cd.nm_full = sum < 1e30f ? 0 : 1;
         cl.nmap = v->d_nmap;
     }
     launch_cone(cl, s);
