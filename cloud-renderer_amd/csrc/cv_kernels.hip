@@ -1866,9 +1866,11 @@ __device__ __forceinline__ unsigned long long board_key(float px, float py, floa
 }
 
 __global__ void __launch_bounds__(256) k_sort_keys(GridDesc g, const float4* __restrict__ boards, int S, float px,
-                                                   float py, float pz, unsigned long long* __restrict__ keys) {
+                                                   float py, float pz, unsigned long long* __restrict__ keys,
+                                                   int* __restrict__ ranks) {
     int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j >= S) return;
+    if (ranks) ranks[j] = 0;
     float4 b = boards[j];
     keys[j] = board_key(px, py, pz, g.vpos[0] + b.x, g.vpos[1] + b.y, g.vpos[2] + b.z, j);
 }
@@ -1880,9 +1882,11 @@ __global__ void __launch_bounds__(256) k_iota(int32_t* __restrict__ order, int S
 
 __device__ __forceinline__ void k_cam_setup_body(GridDesc g, CameraView cv, const float4* __restrict__ boards, int S,
                                                    float4* __restrict__ sph_world, float4* __restrict__ sph_view,
-                                                   int4* __restrict__ sph_tiles, unsigned long long* __restrict__ keys, int bid, int nblk) {
+                                                   int4* __restrict__ sph_tiles, unsigned long long* __restrict__ keys,
+                                                   int* __restrict__ ranks, int bid, int nblk) {
     int j = bid * blockDim.x + threadIdx.x;
     if (j >= S) return;
+    if (ranks) ranks[j] = 0;
     float4 b = boards[j];
     float cx = g.vpos[0] + b.x, cy = g.vpos[1] + b.y, cz = g.vpos[2] + b.z, s = b.w;
     float vx = ((cv.V[0] * cx + cv.V[4] * cy) + cv.V[8] * cz) + cv.V[12];
@@ -1912,8 +1916,9 @@ __device__ __forceinline__ void k_cam_setup_body(GridDesc g, CameraView cv, cons
 }
 __global__ void __launch_bounds__(256) k_cam_setup(GridDesc g, CameraView cv, const float4* __restrict__ boards, int S,
                                                    float4* __restrict__ sph_world, float4* __restrict__ sph_view,
-                                                   int4* __restrict__ sph_tiles, unsigned long long* __restrict__ keys) {
-    k_cam_setup_body(g, cv, boards, S, sph_world, sph_view, sph_tiles, keys, (int)blockIdx.x, (int)gridDim.x);
+                                                   int4* __restrict__ sph_tiles, unsigned long long* __restrict__ keys,
+                                                   int* __restrict__ ranks) {
+    k_cam_setup_body(g, cv, boards, S, sph_world, sph_view, sph_tiles, keys, ranks, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -1972,15 +1977,18 @@ __device__ void replay_ties(int S, const I* s_idx, const uint32_t* s_tie, P* pos
 // for a whole segment of such steps is computed in parallel rounds (a chain
 // only waits on smaller steps of the same segment).  A run of equal distances
 // is resolved step by step: the unplaced member with the smallest find() wins.
-// s_idx[t]: bits 0-14 element, bit 15 = same distance as entry t-1;
-// s_D: positions, 0xFFFF = not yet known; placed: one bit per element.
-__device__ void replay_ties_block(int S, const uint16_t* s_idx, uint16_t* s_D, uint32_t* placed,
-                                  int32_t* __restrict__ order) {
+// A step's word w[t] (S <= 16384): bits 0-13 sorted element, bit 14 = same
+// distance as entry t - 1, bit 15 = in a run of equal distances, high half D[t],
+// 0xFFFF = not yet known.  placed: one bit per element.
+constexpr uint32_t kStepElem = 0x3fffu, kStepTie = 0x4000u, kStepRun = 0x8000u, kStepOpen = 0xffff0000u;
+__device__ __forceinline__ int step_D(uint32_t w) { return (int)(w >> 16); }
+__device__ __forceinline__ void step_set_D(uint32_t* w, int t, int d) { ((uint16_t*)(w + t))[1] = (uint16_t)d; }
+__device__ void replay_ties_block(int S, uint32_t* w, uint32_t* placed, int32_t* __restrict__ order) {
     __shared__ int seg_end;
     __shared__ int red_p[16], red_e[16];
     const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63, wid = tid >> 6;
-    auto tie_at = [&](int t) -> bool { return (s_idx[t] >> 15) != 0; };
-    auto elem = [&](int t) -> int { return (int)(s_idx[t] & 0x7fffu); };
+    auto tie_at = [&](int t) -> bool { return (w[t] & kStepTie) != 0u; };
+    auto elem = [&](int t) -> int { return (int)(w[t] & kStepElem); };
     int k0 = 0;
     while (k0 < S) {
         if (k0 + 1 < S && tie_at(k0 + 1)) {
@@ -1993,7 +2001,7 @@ __device__ void replay_ties_block(int S, const uint16_t* s_idx, uint16_t* s_D, u
                     int y = elem(t);
                     if ((placed[y >> 5] >> (y & 31)) & 1u) continue;
                     int x = y;
-                    while (x < k) x = (int)s_D[x];
+                    while (x < k) x = step_D(w[x]);
                     if (x < best_p) { best_p = x; best_e = y; }
                 }
                 for (int off = 32; off > 0; off >>= 1) {
@@ -2005,10 +2013,10 @@ __device__ void replay_ties_block(int S, const uint16_t* s_idx, uint16_t* s_D, u
                 __syncthreads();
                 if (tid == 0) {
                     int p = red_p[0], e = red_e[0];
-                    for (int w = 1; w < nt / 64; ++w)
-                        if (red_p[w] < p) { p = red_p[w]; e = red_e[w]; }
+                    for (int v = 1; v < nt / 64; ++v)
+                        if (red_p[v] < p) { p = red_p[v]; e = red_e[v]; }
                     if (e >= 0) {  // always: ge - k members are unplaced
-                        s_D[k] = (uint16_t)p;
+                        step_set_D(w, k, p);
                         order[k] = e;
                         placed[e >> 5] |= 1u << (e & 31);
                     }
@@ -2033,14 +2041,14 @@ __device__ void replay_ties_block(int S, const uint16_t* s_idx, uint16_t* s_D, u
         while (true) {
             if (!done) {
                 while (true) {
-                    while (x < k0) x = (int)s_D[x];
+                    while (x < k0) x = step_D(w[x]);
                     if (x >= k) {
-                        s_D[k] = (uint16_t)x;
+                        step_set_D(w, k, x);
                         order[k] = elem(k);
                         done = true;
                         break;
                     }
-                    int dx = (int)s_D[x];  // x in [k0, k): known once its own chain finished
+                    int dx = step_D(w[x]);  // x in [k0, k): known once its own chain finished
                     if (dx == 0xFFFF) break;
                     x = dx;
                 }
@@ -2048,6 +2056,101 @@ __device__ void replay_ties_block(int S, const uint16_t* s_idx, uint16_t* s_D, u
             if (__syncthreads_count(done ? 0 : 1) == 0) break;
         }
         k0 = kend;
+    }
+}
+
+// The same replay for few short runs, the usual case (a run or two among 4096
+// billboards, tens among 16384): only the runs need resolving, and a find()
+// visits D at few positions, on average S / (S - k) of them in all for step k.
+// So D is evaluated on demand (in any order of steps, kept in the words), and a
+// thread takes a run of its own: a chain of LDS reads, one per hop.  A chain
+// that reaches a step of a run that is not resolved yet waits for the next
+// round; the first such run waits for none, so every round resolves one.
+// Replaying every step in order was 35 of the 55 us of a 4096-key sort.  False
+// (nothing lost: what D holds is valid) when the runs are too many or too
+// long, or one lies so near the end that its chains take more than kLazyHops
+// hops: the caller replays every step.
+constexpr int kLazyRuns = 256, kLazyLen = 16, kLazyHops = 1500, kLazyDepth = 16;
+__device__ bool replay_ties_lazy(int S, uint32_t* w, int32_t* __restrict__ order) {
+    __shared__ int nrun;
+    __shared__ uint16_t runs[kLazyRuns];
+    __shared__ uint16_t stack[kLazyDepth][kLazyRuns];  // steps whose evaluation waits for a nested one
+    const int tid = threadIdx.x, nt = blockDim.x;
+    auto tie_at = [&](int t) -> bool { return t < S && (w[t] & kStepTie) != 0u; };
+    auto elem = [&](int t) -> int { return (int)(w[t] & kStepElem); };
+    if (tid == 0) nrun = 0;
+    __syncthreads();
+    bool ok = true;
+    for (int t = tid; t < S; t += nt) {
+        if (tie_at(t) || !tie_at(t + 1)) continue;
+        const int slot = atomicAdd(&nrun, 1);
+        if (slot < kLazyRuns) runs[slot] = (uint16_t)t;
+        int n = 1;
+        while (n <= kLazyLen && tie_at(t + n)) atomicOr(&w[t + n++], kStepRun);
+        atomicOr(&w[t], kStepRun);
+        ok = ok && n <= kLazyLen;
+    }
+    if (__syncthreads_or(!ok || nrun > kLazyRuns)) return false;
+    for (int t = tid; t < S; t += nt) order[t] = elem(t);
+    __syncthreads();  // the runs' entries are rewritten below
+    const int r = (tid & 63) * (nt >> 6) + (tid >> 6);  // runs spread over the waves
+    int a = 0, end = 0, k = 0;
+    uint32_t left = 0;  // members not placed yet
+    if (r < nrun) {
+        a = k = (int)runs[r];
+        end = a + 2;
+        while (tie_at(end)) ++end;
+        left = (1u << (end - a)) - 1u;
+    }
+    int hops = 0;
+    for (;;) {
+        bool wait = false;
+        while (k < end && !wait) {
+            int best_p = 0x7fffffff, best = 0;
+            for (uint32_t m = left; m && !wait; m &= m - 1u) {
+                const int i = __ffs((int)m) - 1;
+                // find(elem(a + i), k): walk; where D is unknown evaluate it
+                // first, D[tgt] = find(elem(tgt), tgt), then go on from it
+                int x = elem(a + i), lim = k, depth = 0;
+                for (;;) {
+                    if (++hops > kLazyHops) {
+                        wait = true;
+                        break;
+                    }
+                    if (x >= lim) {
+                        if (depth == 0) break;
+                        step_set_D(w, lim, x);  // the nested step is lim; its waiting walk stood there
+                        --depth;
+                        lim = depth >= kLazyDepth ? k : (int)stack[depth][r];
+                        if (depth >= kLazyDepth) {  // deeper than the stack: start the walk again
+                            x = elem(a + i);
+                            depth = 0;
+                        }
+                        continue;
+                    }
+                    const uint32_t v = w[x];
+                    if (step_D(v) != 0xFFFF) {
+                        x = step_D(v);
+                    } else if (v & kStepRun) {
+                        wait = true;
+                        break;
+                    } else {
+                        if (depth < kLazyDepth) stack[depth][r] = (uint16_t)lim;
+                        ++depth;
+                        lim = x;
+                        x = (int)(v & kStepElem);
+                    }
+                }
+                if (!wait && x < best_p) { best_p = x; best = i; }
+            }
+            if (wait) break;
+            step_set_D(w, k, best_p);
+            order[k] = elem(a + best);
+            left &= ~(1u << best);
+            ++k;
+        }
+        if (__syncthreads_or(hops > kLazyHops)) return false;
+        if (__syncthreads_or(wait) == 0) return true;
     }
 }
 
@@ -2148,47 +2251,104 @@ __device__ __forceinline__ void k_sort_lds_body(const unsigned long long* __rest
         for (int e = 0; e < E; ++e) sk[pos + e] = out[e];
         __syncthreads();
     }
-    // Reuse the key storage: idx u16[npad] (bit 15 = same distance as the
-    // previous key) | pos u16[npad] | at u16[npad].  Chunk c of 1024 keys is
-    // read before its indices are written; those writes cover keys
-    // [256 c, 256 c + 256), all of which were read in chunks <= c, and the
-    // previous key of the next chunk (index 1024 (c+1) - 1) is not touched.
-    uint16_t* s_idx = (uint16_t*)sk;
-    uint16_t* s_pos = s_idx + npad;
-    uint16_t* s_at = s_pos + npad;
+    // Reuse the key storage for the steps' words.  Chunk c of 1024 keys is read
+    // before its words are written; those writes cover keys [512 c, 512 c +
+    // 512), all of which were read in chunks <= c, and the previous key of the
+    // next chunk (index 1024 (c+1) - 1) is not touched.
+    uint32_t* w = (uint32_t*)sk;
     for (int c = 0; c < npad; c += nt) {
         const int i = c + tid;
         uint32_t v = 0;
         if (i < S) {
             unsigned long long k = sk[i];
-            v = (uint32_t)(k & 0xffffffffull);
+            v = (uint32_t)(k & 0xffffffffull) | kStepOpen;
             if (i > 0 && (k >> 32) == (sk[i - 1] >> 32)) {
-                v |= 0x8000u;
+                v |= kStepTie;
                 tie = 1;
             }
         }
         __syncthreads();
-        if (i < S) s_idx[i] = (uint16_t)v;
+        if (i < S) w[i] = v;
         __syncthreads();
     }
     if (!tie) {
-        for (int i = tid; i < S; i += nt) order[i] = (int32_t)s_idx[i];
+        for (int i = tid; i < S; i += nt) order[i] = (int32_t)(w[i] & kStepElem);
         if (tid == 0) *tie_flag = 0;
         return;
     }
     __shared__ uint32_t placed[kLdsSortMax / 32];
-    uint16_t* s_D = s_pos;
-    (void)s_at;
-    for (int i = tid; i < S; i += nt) s_D[i] = 0xFFFFu;
-    for (int w = tid; w < kLdsSortMax / 32; w += nt) placed[w] = 0u;
+    for (int v = tid; v < kLdsSortMax / 32; v += nt) placed[v] = 0u;
     __syncthreads();
-    replay_ties_block(S, s_idx, s_D, placed, order);
+    if (!replay_ties_lazy(S, w, order)) replay_ties_block(S, w, placed, order);
     if (tid == 0) *tie_flag = 1;
 }
-template <int E>
 __global__ void __launch_bounds__(1024) k_sort_lds(const unsigned long long* __restrict__ keys_in, int S,
                                                    int32_t* __restrict__ order, int* __restrict__ tie_flag) {
-    k_sort_lds_body<E>(keys_in, S, order, tie_flag);
+    k_sort_lds_body<1>(keys_in, S, order, tie_flag);
+}
+
+// Draw order of 1025 .. 16384 billboards by counting: a key's rank is the
+// number of smaller keys, S^2 comparisons spread over the whole device (17 M at
+// 4096 keys, 268 M at 16384), where the sort above keeps one CU busy and, at
+// 16384 keys, would need its whole LDS: beside another kernel that fills the
+// device it waited up to a millisecond for one.  Workgroup (x, y) counts the
+// keys of chunk y below its 256 keys.  Only the distance words are compared
+// (the top bit of all is set, so the sign of a difference is the comparison):
+// among equal distances the lower index is first, and away from the diagonal
+// all indices of the chunk are lower or all are higher.
+template <int CHUNK>
+__global__ void __launch_bounds__(256) k_rank(const unsigned long long* __restrict__ keys, int S,
+                                              int* __restrict__ ranks) {
+    static_assert(CHUNK == 128 || CHUNK == 512, "a workgroup's keys lie in whole chunks or its chunk holds them");
+    __shared__ __align__(16) uint32_t hi[CHUNK];
+    const int i = blockIdx.x * 256 + threadIdx.x, j0 = blockIdx.y * CHUNK;
+    const uint32_t own = i < S ? (uint32_t)(keys[i] >> 32) : 0u;
+    for (int j = threadIdx.x; j < CHUNK; j += 256) hi[j] = j0 + j < S ? (uint32_t)(keys[j0 + j] >> 32) : 0xffffffffu;
+    __syncthreads();
+    if (i >= S) return;
+    int below = 0, above = 0;  // keys < own, keys > own
+#pragma unroll 8
+    for (int j = 0; j < CHUNK; j += 4) {
+        const uint4 h = *(const uint4*)&hi[j];
+        below += (int)((h.x - own) >> 31) + (int)((h.y - own) >> 31);
+        below += (int)((h.z - own) >> 31) + (int)((h.w - own) >> 31);
+        above += (int)((own - h.x) >> 31) + (int)((own - h.y) >> 31);
+        above += (int)((own - h.z) >> 31) + (int)((own - h.w) >> 31);
+    }
+    int n = below;
+    if (below + above < CHUNK && i >= j0)  // equal distances (itself on the diagonal): the lower indices
+        for (int j = 0; j < min(CHUNK, i - j0); ++j) n += hi[j] == own ? 1 : 0;
+    if (n) atomicAdd(&ranks[i], n);
+}
+// The order from the ranks, with the replay of equal distances: one workgroup
+// of 1024 (dynamic LDS: the steps' words).
+__global__ void __launch_bounds__(1024) k_rank_order(const unsigned long long* __restrict__ keys,
+                                                     const int* __restrict__ ranks, int S,
+                                                     int32_t* __restrict__ order, int* __restrict__ tie_flag) {
+    extern __shared__ unsigned long long sk[];
+    __shared__ uint32_t placed[kLdsSortMax / 32];
+    uint32_t* w = (uint32_t*)sk;
+    const int tid = threadIdx.x;
+#pragma unroll 4
+    for (int i = tid; i < S; i += 1024) w[ranks[i]] = (uint32_t)i | kStepOpen;
+    if (tid < kLdsSortMax / 32) placed[tid] = 0u;
+    __syncthreads();
+    uint32_t tied = 0;  // bit c: entry 1024 c + tid has the distance of the one before it
+#pragma unroll 4
+    for (int c = 0; c < kLdsSortMax / 1024; ++c) {
+        const int t = c * 1024 + tid;
+        if (t > 0 && t < S && (keys[w[t] & kStepElem] >> 32) == (keys[w[t - 1] & kStepElem] >> 32)) tied |= 1u << c;
+    }
+    const bool any = __syncthreads_or(tied != 0u) != 0;
+    if (tid == 0) *tie_flag = any ? 1 : 0;
+    if (!any) {
+        for (int t = tid; t < S; t += 1024) order[t] = (int32_t)(w[t] & kStepElem);
+        return;
+    }
+    for (int c = 0; tied >> c; ++c)
+        if ((tied >> c) & 1u) w[c * 1024 + tid] |= kStepTie;
+    __syncthreads();
+    if (!replay_ties_lazy(S, w, order)) replay_ties_block(S, w, placed, order);
 }
 
 // global-memory bitonic stage for more billboards than one LDS holds
@@ -3766,11 +3926,19 @@ void launch_mip(const VolumeDesc& vd, int k, void* levels, hipStream_t s) {
     hipLaunchKernelGGL(k_mip, dim3(blocks_for(ntex, 256)), dim3(256), 0, s, vd, k, levels, ntex);
 }
 
+// ranks of a sort by counting, behind the keys (zeroed with them), or null
+static int* sort_ranks(unsigned long long* keys, int S) {
+    if (S <= 1024 || S > kLdsSortMax) return nullptr;
+    int npad = 2048;
+    while (npad < S) npad <<= 1;
+    return (int*)(keys + npad);
+}
+
 void launch_cam_setup(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
                       float4* sph_view, int4* sph_tiles, unsigned long long* keys, hipStream_t s) {
     if (S <= 0) return;
     hipLaunchKernelGGL(k_cam_setup, dim3(blocks_for(S, 256)), dim3(256), 0, s, g, cv, boards, S, sph_world, sph_view,
-                       sph_tiles, keys);
+                       sph_tiles, keys, sort_ranks(keys, S));
 }
 
 // Scratch `keys` (sort_scratch_words(S) u64 words): [0, npad) the keys written
@@ -3782,28 +3950,11 @@ size_t sort_scratch_words(int S) {
     return 5 * npad;
 }
 
-template <int E>
-static int launch_sort_lds(const unsigned long long* keys, int S, int32_t* order, int* tie_flag, hipStream_t s) {
-    static_assert(1024 * E <= kLdsSortMax, "one workgroup's LDS");
-    const int bytes = 1024 * E * (int)sizeof(unsigned long long);
-    if (bytes > 64 * 1024) {
-        static bool attr_set = false;  // raise the dynamic LDS limit once per instantiation
-        if (!attr_set) {
-            if (hipFuncSetAttribute((const void*)k_sort_lds<E>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) !=
-                hipSuccess)
-                return -1;
-            attr_set = true;
-        }
-    }
-    hipLaunchKernelGGL(k_sort_lds<E>, dim3(1), dim3(1024), (size_t)bytes, s, keys, S, order, tie_flag);
-    return 1024 * E;
-}
-
 void launch_sort_keys(const GridDesc& g, const float4* boards, int S, const float point[3], unsigned long long* keys,
                       hipStream_t s) {
     if (S <= 0) return;
     hipLaunchKernelGGL(k_sort_keys, dim3(blocks_for(S, 256)), dim3(256), 0, s, g, boards, S, point[0], point[1],
-                       point[2], keys);
+                       point[2], keys, sort_ranks(keys, S));
 }
 
 void launch_iota(int32_t* order, int S, hipStream_t s) {
@@ -3815,17 +3966,26 @@ int launch_sort(unsigned long long* keys, int S, int32_t* order, int* tie_flag, 
     if (S <= 0) return 0;
     int npad = 2;
     while (npad < S) npad <<= 1;
-    if (npad <= kLdsSortMax) {
-        int r;
-        switch (npad < 1024 ? 1024 : npad) {
-            case 1024: r = launch_sort_lds<1>(keys, S, order, tie_flag, s); break;
-            case 2048: r = launch_sort_lds<2>(keys, S, order, tie_flag, s); break;
-            case 4096: r = launch_sort_lds<4>(keys, S, order, tie_flag, s); break;
-            case 8192: r = launch_sort_lds<8>(keys, S, order, tie_flag, s); break;
-            default: r = launch_sort_lds<16>(keys, S, order, tie_flag, s); break;
-        }
-        if (r > 0) return r;  // else (LDS limit not raised): the global-memory sort below
+    if (S <= 1024) {  // one workgroup, 8 KB of LDS: 8 us, the two launches of the counting take 10
+        hipLaunchKernelGGL(k_sort_lds, dim3(1), dim3(1024), 1024 * sizeof(unsigned long long), s, keys, S, order,
+                           tie_flag);
+        return 1024;
     }
+    // above 13 k keys the order's LDS passes the default limit of 64 KB
+    if (S <= kLdsSortMax && (4 * S <= 52 * 1024 ||
+                             hipFuncSetAttribute((const void*)k_rank_order, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                 4 * kLdsSortMax) == hipSuccess)) {
+        int* ranks = sort_ranks(keys, S);
+        // short loops while the device is not full: 4096 keys are 512 workgroups of 128 comparisons
+        if (S <= 8192)
+            hipLaunchKernelGGL(k_rank<128>, dim3(blocks_for(S, 256), blocks_for(S, 128)), dim3(256), 0, s, keys, S,
+                               ranks);
+        else
+            hipLaunchKernelGGL(k_rank<512>, dim3(blocks_for(S, 256), blocks_for(S, 512)), dim3(256), 0, s, keys, S,
+                               ranks);
+        hipLaunchKernelGGL(k_rank_order, dim3(1), dim3(1024), 4 * (size_t)S, s, keys, ranks, S, order, tie_flag);
+        return npad;
+    }  // else (LDS limit not raised): the global-memory sort below
     unsigned long long* pk = keys + npad;
     uint32_t* g_idx = (uint32_t*)(keys + 2 * (size_t)npad);
     uint32_t* g_tie = g_idx + npad;
@@ -4135,7 +4295,8 @@ __global__ void __launch_bounds__(1024) kb_mip_tail(const BatchVox* __restrict__
 __global__ void __launch_bounds__(256) kb_cam_setup(const BatchVox* __restrict__ sc, BatchStage st) {
     const StageSlot q = stage_slot(st);
     const BatchVox& B = sc[q.sc];
-    k_cam_setup_body(B.g, B.cv, B.boards, B.S, B.sph_world, B.sph_view, B.sph_tiles, B.sortkeys, q.bid, q.nblk);
+    k_cam_setup_body(B.g, B.cv, B.boards, B.S, B.sph_world, B.sph_view, B.sph_tiles, B.sortkeys, nullptr, q.bid,
+                     q.nblk);
 }
 __global__ void __launch_bounds__(256) kb_iota(const BatchVox* __restrict__ sc, BatchStage st) {
     const StageSlot q = stage_slot(st);
