@@ -83,13 +83,16 @@ typedef __bf16 cv_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float cv_f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int cv_u32x4 __attribute__((ext_vector_type(4)));
 
-__device__ __forceinline__ uint32_t f2bf_bits(float x) {
-    uint32_t u = __float_as_uint(x);
-    if ((u & 0x7f800000u) == 0x7f800000u) return (u >> 16) | ((u & 0xffffu) ? 0x40u : 0u);  // inf / nan
-    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+// two floats to bf16, round to nearest even, on v_cvt_pk_bf16_f32 (one
+// instruction where shifts and adds took fourteen for the pair)
+__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    const f2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
 }
+__device__ __forceinline__ uint32_t f2bf_bits(float x) { return pack_bf2(x, 0.0f) & 0xffffu; }
 __device__ __forceinline__ float bf2f(uint32_t b) { return __uint_as_float(b << 16); }
-__device__ __forceinline__ uint32_t pack_bf2(float lo, float hi) { return f2bf_bits(lo) | (f2bf_bits(hi) << 16); }
 
 __device__ __forceinline__ cv_bf16x8 as_bf16x8(cv_u32x4 v) { return __builtin_bit_cast(cv_bf16x8, v); }
 
@@ -142,27 +145,6 @@ __device__ __forceinline__ cv_u32x4 x_operand(const uint16_t* xs, int n, int s, 
     cv_u32x4 v;
     v.x = lo.x; v.y = lo.y; v.z = hi.x; v.w = hi.y;
     return v;
-}
-
-// One hidden layer l (1..3) or the first layer (from B operands), 64 outputs.
-// in[s][nt]: B operands, KS steps; out: 2 x 2 accumulators (pre-activation).
-template <int KS>
-__device__ __forceinline__ void mlp_layer64(const MlpDev& w, int l, const cv_u32x4 (&in)[4][2], cv_f32x16 (&acc)[2][2],
-                                            int lane) {
-    const int h = lane >> 5;
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-        cv_f32x16 c0 = bias_init(w.bias, mlp_bpad0(l) + 32 * mt, h);
-        cv_f32x16 c1 = c0;
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            cv_u32x4 a = load_blk(w.fwd, mlp_fblk0(l) + mt * KS + s, lane);
-            c0 = mfma_bf16(a, in[s][0], c0);
-            c1 = mfma_bf16(a, in[s][1], c1);
-        }
-        acc[mt][0] = c0;
-        acc[mt][1] = c1;
-    }
 }
 
 // Forward pass of one 32-row half (N-tile nt) of the wave's batch: layers

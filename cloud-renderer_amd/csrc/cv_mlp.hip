@@ -14,269 +14,329 @@
 namespace cv {
 
 // ---------------------------------------------------------------------------
-// batched inference: rows X[n][17] -> Y[n][5], one wave per 64 rows
+// batched inference: rows X[n][17] -> Y[n][5], one wave per 32 rows
+//
+// Bound by the GELUs (128 per lane and tile, two of their eight instructions at
+// a fraction of the rate) and, for fewer rows than fill the device, by the
+// chain of layers: 32 rows per wave are one chain and twice the waves of 64.
+// The 544 features of a tile are contiguous, so the loads are whole lines.
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(64) k_mlp_forward(MlpDev w, const float* __restrict__ X, int n,
-                                                    float* __restrict__ Y) {
-    __shared__ __align__(16) uint16_t xs[64 * kMlpInPad];
-    const int lane = threadIdx.x;
-    const int row = blockIdx.x * 64 + lane;
-    const bool valid = row < n;
+constexpr int kFwdWaves = 4;
+__global__ void __launch_bounds__(64 * kFwdWaves) k_mlp_forward(MlpDev w, const float* __restrict__ X, int n,
+                                                                float* __restrict__ Y) {
+    __shared__ __align__(16) uint16_t xs[kFwdWaves][32 * kMlpInPad];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int row0 = (blockIdx.x * kFwdWaves + wave) * 32;
+    uint16_t* tile = xs[wave];
+    const size_t base = (size_t)row0 * kMlpIn, end = (size_t)n * kMlpIn;
 #pragma unroll
-    for (int k = 0; k < kMlpInPad; ++k) {
-        float v = (valid && k < kMlpIn) ? X[(size_t)row * kMlpIn + k] : 0.0f;
-        xs[lane * kMlpInPad + k] = (uint16_t)f2bf_bits(v);
+    for (int q = 0; q < 8; ++q) ((uint32_t*)tile)[q * 64 + lane] = 0u;  // the pads, and rows past n
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < (32 * kMlpIn + 63) / 64; ++q) {
+        const int i = q * 64 + lane;
+        if (i < 32 * kMlpIn && base + i < end) tile[(i / kMlpIn) * kMlpInPad + i % kMlpIn] = (uint16_t)f2bf_bits(X[base + i]);
     }
     __syncthreads();
-    float out[kMlpOut];
-    mlp_forward_wave(w, xs, lane, out);
-    if (valid) {
+    if (row0 >= n) return;
+    const cv_f32x16 y = mlp_forward_tile(w, tile, 0, lane);
+    // outputs 0..3 in registers 0..3 of half 0, output 4 in register 0 of half 1
+    const int row = row0 + (lane & 31);
+    if (row >= n) return;
+    float* o = Y + (size_t)row * kMlpOut;
+    if (lane < 32) {
 #pragma unroll
-        for (int q = 0; q < kMlpOut; ++q) Y[(size_t)row * kMlpOut + q] = out[q];
+        for (int q = 0; q < 4; ++q) o[q] = y[q];
+    } else {
+        o[4] = y[0];
     }
 }
 
 // ---------------------------------------------------------------------------
-// training: one wave per 64 rows; writes every parameter's partial gradient
+// training: a workgroup per 64 rows; writes every parameter's partial gradient
 // of this workgroup (no atomics) and its partial loss
+//
+// Four waves: wave (mt, nt) holds output units 32 mt .. + 31 of rows
+// 32 nt .. + 31 of every layer.  A wave's accumulators are half of the next
+// layer's B operand for its rows; the halves are exchanged through LDS (two
+// 16-byte words per lane and layer).  Z stays in the waves' registers for the
+// backward pass.  The work is a chain of layers, so what counts is how little
+// of it one wave does and that 16384 rows are one workgroup per CU: with one
+// wave per 64 rows a step took 105 us of this kernel, of which the matrix
+// instructions were 3.
 // ---------------------------------------------------------------------------
 struct TrainLds {
     uint16_t xs[64 * kMlpInPad];        // layer-0 input, row-major
     uint16_t hs[5][64 * 64];            // H_l as [unit][row] (l = 0 uses 32 units)
     uint16_t gs[64 * 64];               // dL/dZ_l as [unit][row]
-    float zs[4][4][16][64];             // Z_l (l = 0..3) in accumulator order [mt*2+nt][j][lane]
+    cv_u32x4 xch[2][2][4][64];          // B operands [buffer][nt][step][lane]
+    float fx[2][2][8][64];              // [mt][from nt]: the half of a wave's gradients whose row sums the other takes
+    float loss[64];
 };
 
 __device__ __forceinline__ cv_u32x4 lds_row8(const uint16_t* base) { return *(const cv_u32x4*)base; }
 
-// sum over the 32 lanes of each half (rows of the batch) of each register
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
+}
+// sum over the 32 lanes of each half (rows of the batch): the butterfly over
+// lane distances 1, 2, 4, 8, 16, on lane permutes inside a row of 16 (mirrors
+// serve for 4 and 8, where the groups they swap already hold equal sums)
 __device__ __forceinline__ float half_sum(float v) {
-#pragma unroll
-    for (int off = 1; off < 32; off <<= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    v = dpp_add<0xB1>(v);   // quad_perm 1 0 3 2
+    v = dpp_add<0x4E>(v);   // quad_perm 2 3 0 1
+    v = dpp_add<0x141>(v);  // row_half_mirror
+    v = dpp_add<0x140>(v);  // row_mirror
+    return v + __int_as_float(__builtin_amdgcn_ds_swizzle(__float_as_int(v), 0x401F));  // lane ^ 16
 }
 
-// G (accumulators of layer l's outputs, MT m-tiles) -> bias partials, LDS copy
-template <int MT>
-__device__ __forceinline__ void store_grad(const cv_f32x16 (&g)[2][2], int l, TrainLds& S, float* __restrict__ part,
-                                           int lane) {
+// the wave's gradients (accumulator registers) into LDS: bf16 for the weight
+// gradients, the next layer's B operand, and the half of the bias terms that
+// the wave of the other rows sums
+__device__ __forceinline__ void store_grad(const cv_f32x16& g, TrainLds& S, int buf, int mt, int nt, int lane) {
     const int h = lane >> 5, c = lane & 31;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
+    for (int j = 0; j < 16; ++j) S.gs[(32 * mt + mlp_crow(h, j)) * 64 + 32 * nt + c] = (uint16_t)f2bf_bits(g[j]);
 #pragma unroll
-        for (int j = 0; j < 16; ++j) {
-            const int unit = 32 * mt + mlp_crow(h, j);
-            S.gs[unit * 64 + c] = (uint16_t)f2bf_bits(g[mt][0][j]);
-            S.gs[unit * 64 + 32 + c] = (uint16_t)f2bf_bits(g[mt][1][j]);
-            float sm = half_sum(g[mt][0][j] + g[mt][1][j]);
-            if (c == 0 && unit < mlp_out(l)) part[mlp_boff(l) + unit] = sm;
-        }
+    for (int s = 0; s < 2; ++s) S.xch[buf][nt][2 * mt + s][lane] = chain_b(g, s);
+#pragma unroll
+    for (int q = 0; q < 8; ++q) S.fx[mt][nt][q][lane] = nt == 0 ? g[8 + q] : g[q];
+}
+// bias gradients: registers 0..7 by the wave of rows 0..31, 8..15 by the other
+__device__ __forceinline__ void bias_grad(const cv_f32x16& g, int l, const TrainLds& S, float* __restrict__ part,
+                                          int mt, int nt, int lane) {
+    const int h = lane >> 5, c = lane & 31;
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+        const float own = nt == 0 ? g[q] : g[8 + q];
+        const float sm = half_sum(own + S.fx[mt][nt ^ 1][q][lane]);
+        const int unit = 32 * mt + (nt == 0 ? mlp_crow(h, q) : mlp_crow(h, 8 + q));
+        if (c == 0 && unit < mlp_out(l)) part[mlp_boff(l) + unit] = sm;
     }
 }
 
-// dW_l = G H_l^T over the 64 rows (K = rows), written to the partials
-template <int MT, int NT>
-__device__ __forceinline__ void weight_grad(int l, const TrainLds& S, float* __restrict__ part, int lane) {
+// dW_l = G H_l^T over the 64 rows (K = rows), outputs 32 mt .., inputs
+// 32 nt .., written to the partials
+__device__ __forceinline__ void weight_grad(int l, const TrainLds& S, float* __restrict__ part, int mt, int nt,
+                                            int lane) {
     const int h = lane >> 5, c = lane & 31;
     const int nin = mlp_in(l), nout = mlp_out(l);
+    cv_f32x16 acc;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
+    for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
 #pragma unroll
-        for (int nt = 0; nt < NT; ++nt) {
-            cv_f32x16 acc;
+    for (int s = 0; s < 4; ++s) {
+        cv_u32x4 a = lds_row8(S.gs + (32 * mt + c) * 64 + 16 * s + 8 * h);
+        cv_u32x4 b = lds_row8(S.hs[l] + (32 * nt + c) * 64 + 16 * s + 8 * h);
+        acc = mfma_bf16(a, b, acc);
+    }
+    const int in = 32 * nt + c;
 #pragma unroll
-            for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                cv_u32x4 a = lds_row8(S.gs + (32 * mt + c) * 64 + 16 * s + 8 * h);
-                cv_u32x4 b = lds_row8(S.hs[l] + (32 * nt + c) * 64 + 16 * s + 8 * h);
-                acc = mfma_bf16(a, b, acc);
-            }
-            const int in = 32 * nt + c;
-#pragma unroll
-            for (int j = 0; j < 16; ++j) {
-                const int out = 32 * mt + mlp_crow(h, j);
-                if (out < nout && in < nin) part[mlp_woff(l) + out * nin + in] = acc[j];
-            }
-        }
+    for (int j = 0; j < 16; ++j) {
+        const int out = 32 * mt + mlp_crow(h, j);
+        if (out < nout && in < nin) part[mlp_woff(l) + out * nin + in] = acc[j];
     }
 }
 
 // dH_l = W_l^T G_l (layers 1..4), then G_{l-1} = dH_l * GELU'(Z_{l-1})
 template <int KS>
-__device__ __forceinline__ void back_layer(const MlpDev& w, int l, cv_f32x16 (&g)[2][2], const TrainLds& S,
-                                           int lane) {
-    cv_u32x4 B[4][2];
+__device__ __forceinline__ void back_layer(const MlpDev& w, int l, const TrainLds& S, int buf, const cv_f32x16& z,
+                                           cv_f32x16& g, int mt, int nt, int lane) {
+    cv_f32x16 d;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) d[j] = 0.0f;
 #pragma unroll
     for (int s = 0; s < KS; ++s)
+        d = mfma_bf16(load_blk(w.bwd, mlp_bblk0(l) + mt * KS + s, lane), S.xch[buf][nt][s][lane], d);
 #pragma unroll
-        for (int nt = 0; nt < 2; ++nt) B[s][nt] = chain_b(g[s >> 1][nt], s & 1);
-    cv_f32x16 d[2][2];
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-        cv_f32x16 c0, c1;
-#pragma unroll
-        for (int j = 0; j < 16; ++j) { c0[j] = 0.0f; c1[j] = 0.0f; }
-#pragma unroll
-        for (int s = 0; s < KS; ++s) {
-            cv_u32x4 a = load_blk(w.bwd, mlp_bblk0(l) + mt * KS + s, lane);
-            c0 = mfma_bf16(a, B[s][0], c0);
-            c1 = mfma_bf16(a, B[s][1], c1);
-        }
-        d[mt][0] = c0;
-        d[mt][1] = c1;
-    }
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-        for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-            for (int j = 0; j < 16; ++j) g[mt][nt][j] = d[mt][nt][j] * gelu_grad(S.zs[l - 1][mt * 2 + nt][j][lane]);
+    for (int j = 0; j < 16; ++j) g[j] = d[j] * gelu_grad(z[j]);
 }
 
-__global__ void __launch_bounds__(64) k_mlp_train(MlpDev w, const float* __restrict__ X, const float* __restrict__ T,
-                                                  int n, float inv_n, float* __restrict__ partial,
-                                                  float* __restrict__ loss_part) {
+__global__ void __launch_bounds__(256) k_mlp_train(MlpDev w, const float* __restrict__ X, const float* __restrict__ T,
+                                                   int n, float inv_n, float* __restrict__ partial,
+                                                   float* __restrict__ loss_part) {
     __shared__ __align__(16) TrainLds S;
-    const int lane = threadIdx.x;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int mt = wave >> 1, nt = wave & 1;
     const int h = lane >> 5, c = lane & 31;
     const int row0 = blockIdx.x * 64;
     float* part = partial + (size_t)blockIdx.x * kMlpParamsPad;
     {
-        const int row = row0 + lane;
-        const bool valid = row < n;
+        // features 8 wave .. + 7 of row `lane`
+        const int row = row0 + lane, k0 = 8 * wave;
+        float v[8];
 #pragma unroll
-        for (int k = 0; k < kMlpInPad; ++k) {
-            float v = (valid && k < kMlpIn) ? X[(size_t)row * kMlpIn + k] : 0.0f;
-            uint16_t b = (uint16_t)f2bf_bits(v);
-            S.xs[lane * kMlpInPad + k] = b;
-            S.hs[0][k * 64 + lane] = b;
+        for (int q = 0; q < 8; ++q) v[q] = row < n && k0 + q < kMlpIn ? X[(size_t)row * kMlpIn + k0 + q] : 0.0f;
+        cv_u32x4 b;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            b[q] = pack_bf2(v[2 * q], v[2 * q + 1]);
+            S.hs[0][(k0 + 2 * q) * 64 + lane] = (uint16_t)b[q];
+            S.hs[0][(k0 + 2 * q + 1) * 64 + lane] = (uint16_t)(b[q] >> 16);
         }
+        *(cv_u32x4*)(S.xs + lane * kMlpInPad + k0) = b;
     }
     __syncthreads();
 
-    // ---- forward, saving Z_l and H_{l+1}
-    cv_u32x4 B[4][2];
-#pragma unroll
-    for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-        for (int s = 0; s < 2; ++s) B[s][nt] = x_operand(S.xs, 32 * nt + c, s, h);
-    cv_f32x16 acc[2][2];
+    // ---- forward, keeping Z_l and storing H_{l+1}
+    cv_f32x16 z[4];
 #pragma unroll
     for (int l = 0; l < 4; ++l) {
-        if (l == 0) mlp_layer64<2>(w, 0, B, acc, lane);
-        else mlp_layer64<4>(w, l, B, acc, lane);
+        const int KS = l == 0 ? 2 : 4;
+        cv_f32x16 a = bias_init(w.bias, mlp_bpad0(l) + 32 * mt, h);
 #pragma unroll
-        for (int mt = 0; mt < 2; ++mt)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt)
-#pragma unroll
-                for (int j = 0; j < 16; ++j) {
-                    float z = acc[mt][nt][j];
-                    S.zs[l][mt * 2 + nt][j][lane] = z;
-                    float a = gelu_f(z);
-                    acc[mt][nt][j] = a;
-                    S.hs[l + 1][(32 * mt + mlp_crow(h, j)) * 64 + 32 * nt + c] = (uint16_t)f2bf_bits(a);
-                }
-#pragma unroll
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int nt = 0; nt < 2; ++nt) B[s][nt] = chain_b(acc[s >> 1][nt], s & 1);
-    }
-    cv_f32x16 y[2];
-    {
-        cv_f32x16 y0 = bias_init(w.bias, mlp_bpad0(4), h);
-        cv_f32x16 y1 = y0;
-#pragma unroll
-        for (int s = 0; s < 4; ++s) {
-            cv_u32x4 a = load_blk(w.fwd, mlp_fblk0(4) + s, lane);
-            y0 = mfma_bf16(a, B[s][0], y0);
-            y1 = mfma_bf16(a, B[s][1], y1);
+        for (int s = 0; s < KS; ++s) {
+            const cv_u32x4 B = l == 0 ? x_operand(S.xs, 32 * nt + c, s, h) : S.xch[l & 1][nt][s][lane];
+            a = mfma_bf16(load_blk(w.fwd, mlp_fblk0(l) + mt * KS + s, lane), B, a);
         }
-        y[0] = y0;
-        y[1] = y1;
+        z[l] = a;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            a[j] = gelu_f(a[j]);
+            S.hs[l + 1][(32 * mt + mlp_crow(h, j)) * 64 + 32 * nt + c] = (uint16_t)f2bf_bits(a[j]);
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s) S.xch[(l + 1) & 1][nt][2 * mt + s][lane] = chain_b(a, s);
+        __syncthreads();
     }
 
-    // ---- loss gradient in accumulator layout: rows 0..3 in registers 0..3
-    // of half 0, row 4 in register 0 of half 1
-    cv_f32x16 g[2][2];
-    float lsum = 0.0f;
+    // ---- output layer and loss gradient (the waves of units 0..31), in
+    // accumulator layout: rows 0..3 in registers 0..3 of half 0, row 4 in
+    // register 0 of half 1
+    cv_f32x16 g;
 #pragma unroll
-    for (int nt = 0; nt < 2; ++nt) {
+    for (int j = 0; j < 16; ++j) g[j] = 0.0f;
+    float d4[4] = {0.0f, 0.0f, 0.0f, 0.0f}, w2 = 0.0f;  // loss terms w2 d4^2
+    if (mt == 0) {
+        cv_f32x16 y = bias_init(w.bias, mlp_bpad0(4), h);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) y = mfma_bf16(load_blk(w.fwd, mlp_fblk0(4) + s, lane), S.xch[0][nt][s][lane], y);
         const int row = row0 + 32 * nt + c;
         const bool valid = row < n;
-        float e = 0.0f, wt = 0.0f;
-        float d4[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+        float e = 0.0f;
         if (h == 0 && valid) {
             const float* t = T + (size_t)row * kMlpOut;
-            wt = t[4];
+            w2 = t[4] * t[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                d4[q] = y[nt][q] - t[q];
-                e = fmaxf(e, fabsf(fminf(fmaxf(y[nt][q], 0.0f), 1.0f) - t[q]));
+                d4[q] = y[q] - t[q];
+                e = fmaxf(e, fabsf(fminf(fmaxf(y[q], 0.0f), 1.0f) - t[q]));
             }
         }
-        float e_hi = __shfl(e, c, 64);
-#pragma unroll
-        for (int j = 0; j < 16; ++j) g[0][nt][j] = 0.0f;
+        const float e_hi = __shfl(e, c, 64);
         if (valid) {
             if (h == 0) {
-                const float w2 = wt * wt;
 #pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    g[0][nt][q] = 2.0f * w2 * d4[q] * inv_n;
-                    lsum = fmaf(w2 * d4[q], d4[q], lsum);
-                }
+                for (int q = 0; q < 4; ++q) g[q] = 2.0f * w2 * d4[q] * inv_n;
             } else {
-                const float de = y[nt][0] - e_hi;
-                g[0][nt][0] = 2.0f * de * inv_n;
-                lsum = fmaf(de, de, lsum);
+                const float de = y[0] - e_hi;
+                g[0] = 2.0f * de * inv_n;
+                d4[0] = de;
+                w2 = 1.0f;
             }
         }
+        if (nt == 0) {
+            float lsum = 0.0f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) lsum = fmaf(w2 * d4[q], d4[q], lsum);
+            S.loss[lane] = lsum;
+        }
     }
-    {
+
+    // ---- backward
+    store_grad(g, S, 1, mt, nt, lane);
+    __syncthreads();
+    if (wave == 1) {
+        // rows 32..63 go on from the sums of rows 0..31
+        float lsum = S.loss[lane];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) lsum = fmaf(w2 * d4[q], d4[q], lsum);
         float tot = lsum;
 #pragma unroll
         for (int off = 1; off < 64; off <<= 1) tot += __shfl_xor(tot, off, 64);
         if (lane == 0) loss_part[blockIdx.x] = tot * inv_n;
     }
-
-    // ---- backward
-    store_grad<1>(g, 4, S, part, lane);
-    __syncthreads();
-    weight_grad<1, 2>(4, S, part, lane);
-    back_layer<2>(w, 4, g, S, lane);
+    if (mt == 0) {
+        weight_grad(4, S, part, 0, nt, lane);
+        bias_grad(g, 4, S, part, mt, nt, lane);
+    }
+    back_layer<2>(w, 4, S, 1, z[3], g, mt, nt, lane);
     __syncthreads();
 #pragma unroll
     for (int l = 3; l >= 1; --l) {
-        store_grad<2>(g, l, S, part, lane);
+        store_grad(g, S, l & 1, mt, nt, lane);
         __syncthreads();
-        weight_grad<2, 2>(l, S, part, lane);
-        back_layer<4>(w, l, g, S, lane);
+        weight_grad(l, S, part, mt, nt, lane);
+        bias_grad(g, l, S, part, mt, nt, lane);
+        back_layer<4>(w, l, S, l & 1, z[l - 1], g, mt, nt, lane);
         __syncthreads();
     }
-    store_grad<2>(g, 0, S, part, lane);
+    store_grad(g, S, 0, mt, nt, lane);
     __syncthreads();
-    weight_grad<2, 1>(0, S, part, lane);
+    if (nt == 0) weight_grad(0, S, part, mt, 0, lane);
+    bias_grad(g, 0, S, part, mt, nt, lane);
+}
+
+// where parameter p's bf16 value goes in the packed blocks (k_mlp_pack's inverse)
+__device__ __forceinline__ void pack_param(int p, float v, uint16_t* __restrict__ fwd, uint16_t* __restrict__ bwd,
+                                           float* __restrict__ bias) {
+    int l = 0;
+    while (l < 4 && p >= mlp_woff(l + 1)) ++l;
+    if (p >= mlp_boff(l)) {
+        bias[mlp_bpad0(l) + p - mlp_boff(l)] = v;
+        return;
+    }
+    const int nin = mlp_in(l), m = (p - mlp_woff(l)) / nin, k = (p - mlp_woff(l)) % nin;
+    const uint16_t b = (uint16_t)f2bf_bits(v);
+    // slot q of lane half h holds offset 8 (q / 4) + 4 h + q % 4 of its 16-wide step
+    auto at = [](int blk, int row, int kk) {
+        const int q = ((kk >> 3) << 2) | (kk & 3), h = (kk >> 2) & 1;
+        return blk * 512 + (32 * h + (row & 31)) * 8 + q;
+    };
+    fwd[at(mlp_fblk0(l) + (m >> 5) * (mlp_kpad(l) / 16) + (k >> 4), m, k & 15)] = b;
+    if (l > 0) bwd[at(mlp_bblk0(l) + (k >> 5) * (mlp_mpad(l) / 16) + (m >> 4), k, m & 15)] = b;
 }
 
 // ---------------------------------------------------------------------------
-// gradient reduction (fixed order over workgroups) + Adam
+// gradient reduction (fixed order over workgroups), Adam and the packed weights
+// of the next step
+//
+// 14 MB of partials for 16384 rows: 64 parameters per workgroup spread them
+// over 219 CUs, 32 loads in flight per thread; the loss partials are a
+// workgroup's own (one thread walking them one by one was the kernel's 67 us).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ partial, int nwg,
-                                                  const float* __restrict__ loss_part, float* __restrict__ master,
-                                                  float* __restrict__ m1, float* __restrict__ m2,
-                                                  float* __restrict__ grad_out, float* __restrict__ loss_out,
-                                                  AdamStep st) {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p == 0 && loss_out) {
+__global__ void __launch_bounds__(64) k_mlp_adam(const float* __restrict__ partial, int nwg,
+                                                 const float* __restrict__ loss_part, float* __restrict__ master,
+                                                 float* __restrict__ m1, float* __restrict__ m2,
+                                                 float* __restrict__ grad_out, float* __restrict__ loss_out,
+                                                 AdamStep st, MlpPacked pk) {
+    if (blockIdx.x == gridDim.x - 1) {
         float s = 0.0f;
-        for (int i = 0; i < nwg; ++i) s += loss_part[i];
-        *loss_out = s;
+        for (int i0 = 0; i0 < nwg; i0 += 64) {
+            const int i = i0 + (int)threadIdx.x;
+            const float v = i < nwg ? loss_part[i] : 0.0f;
+            const int m = min(64, nwg - i0);
+            for (int q = 0; q < m; ++q) s += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), q));
+        }
+        if (threadIdx.x == 0 && loss_out) *loss_out = s;
+        return;
     }
+    const int p = blockIdx.x * 64 + threadIdx.x;
     if (p >= kMlpParams) return;
+    const float* src = partial + p;
     float gsum = 0.0f;
-    for (int i = 0; i < nwg; ++i) gsum += partial[(size_t)i * kMlpParamsPad + p];
+    int i = 0;
+    for (; i + 32 <= nwg; i += 32) {
+        float v[32];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) v[q] = src[(size_t)(i + q) * kMlpParamsPad];
+#pragma unroll
+        for (int q = 0; q < 32; ++q) gsum += v[q];
+    }
+    for (; i < nwg; ++i) gsum += src[(size_t)i * kMlpParamsPad];
     if (grad_out) grad_out[p] = gsum;
     if (st.apply) {
         float a = fmaf(st.beta1, m1[p], (1.0f - st.beta1) * gsum);
@@ -284,7 +344,9 @@ __global__ void __launch_bounds__(256) k_mlp_adam(const float* __restrict__ part
         m1[p] = a;
         m2[p] = b;
         float mh = a / st.bc1, vh = b / st.bc2;
-        master[p] = master[p] - st.lr * mh / (sqrtf(vh) + st.eps);
+        const float v = master[p] - st.lr * mh / (sqrtf(vh) + st.eps);
+        master[p] = v;
+        pack_param(p, v, pk.fwd, pk.bwd, pk.bias);
     }
 }
 
@@ -333,7 +395,8 @@ void launch_mlp_pack(const float* master, uint16_t* fwd, uint16_t* bwd, float* b
 
 void launch_mlp_forward(const MlpDev& w, const float* X, int n, float* Y, hipStream_t s) {
     if (n <= 0) return;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((n + 63) / 64), dim3(64), 0, s, w, X, n, Y);
+    const int per = 32 * kFwdWaves;
+    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((n + (long long)per - 1) / per)), dim3(64 * kFwdWaves), 0, s, w, X, n, Y);
 }
 
 int mlp_train_groups(int n) { return (n + 63) / 64; }
@@ -341,14 +404,14 @@ int mlp_train_groups(int n) { return (n + 63) / 64; }
 void launch_mlp_train(const MlpDev& w, const float* X, const float* T, int n, float* partial, float* loss_part,
                       hipStream_t s) {
     const int nwg = mlp_train_groups(n);
-    hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(64), 0, s, w, X, T, n, 1.0f / (float)n, partial,
+    hipLaunchKernelGGL(k_mlp_train, dim3(nwg), dim3(256), 0, s, w, X, T, n, 1.0f / (float)n, partial,
                        loss_part);
 }
 
 void launch_mlp_adam(const float* partial, int nwg, const float* loss_part, float* master, float* m1, float* m2,
-                     float* grad_out, float* loss_out, const AdamStep& st, hipStream_t s) {
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, s, partial, nwg, loss_part, master,
-                       m1, m2, grad_out, loss_out, st);
+                     float* grad_out, float* loss_out, const AdamStep& st, const MlpPacked& pk, hipStream_t s) {
+    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 63) / 64 + 1), dim3(64), 0, s, partial, nwg, loss_part, master,
+                       m1, m2, grad_out, loss_out, st, pk);
 }
 
 }  // namespace cv

@@ -8,6 +8,11 @@
 
 namespace cv {
 
+// the packed weights an Adam step renews (pads stay as launch_mlp_pack set them)
+struct MlpPacked {
+    uint16_t *fwd, *bwd;
+    float* bias;
+};
 struct AdamStep {
     float lr, beta1, beta2, eps;
     float bc1, bc2;  // bias corrections 1 - beta^t
@@ -20,6 +25,6 @@ int mlp_train_groups(int n);
 void launch_mlp_train(const MlpDev& w, const float* X, const float* T, int n, float* partial, float* loss_part,
                       hipStream_t s);
 void launch_mlp_adam(const float* partial, int nwg, const float* loss_part, float* master, float* m1, float* m2,
-                     float* grad_out, float* loss_out, const AdamStep& st, hipStream_t s);
+                     float* grad_out, float* loss_out, const AdamStep& st, const MlpPacked& pk, hipStream_t s);
 
 }  // namespace cv

@@ -1798,8 +1798,8 @@ static int mlp_launch_step(cr_mlp m, const float* d_x, const float* d_t, int n, 
     } else {
         st.bc1 = st.bc2 = 1.0f;
     }
-    launch_mlp_adam(partial, nwg, loss_part, m->d_master, m->d_m1, m->d_m2, m->d_grad, m->d_loss, st, s);
-    if (apply) launch_mlp_pack(m->d_master, m->d_fwd, m->d_bwd, m->d_bias, s);
+    launch_mlp_adam(partial, nwg, loss_part, m->d_master, m->d_m1, m->d_m2, m->d_grad, m->d_loss, st,
+                    MlpPacked{m->d_fwd, m->d_bwd, m->d_bias}, s);
     CR_HIP(ctx, hipGetLastError());
     return CR_OK;
 }

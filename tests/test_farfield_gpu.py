@@ -272,3 +272,56 @@ def test_learned_fp16_against_fp64(cv, gpu_ctx):
     log(f"[farfield] FP16 plain max-abs vs FP64 {err_plain:.2e}; learned + FP16 vs FP64 {p_learned:.2f} dB")
     assert err_plain <= 2e-3
     assert p_learned >= 40.0
+
+
+@pytest.mark.parametrize("n", [1, 31, 32, 33, 64, 127, 128, 129, 1000])
+def test_mlp_rows_do_not_depend_on_the_batch(cv, gpu_ctx, n):
+    """Row tiles of 32 and workgroups of 128: every row of a batch of n equals
+    the same row of a larger batch, and nothing is written past row n."""
+    import ctypes as C
+
+    import torch
+    log(f"[mlp] {n} rows")
+    mlp = cv.FarFieldMLP(gpu_ctx, cv.FarFieldMLP.init_params(3))
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n)
+    x = torch.randn((2048, 17), generator=g, device="cuda")
+    try:
+        full = mlp.forward(x)
+        out = torch.full((n + 64, 5), 7.0, device="cuda")
+        rc = cv.lib().cr_mlp_forward(mlp.handle, C.c_void_p(x.data_ptr()), n, C.c_void_p(out.data_ptr()),
+                                     C.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        assert torch.equal(out[:n], full[:n])
+        assert bool((out[n:] == 7.0).all())
+    finally:
+        mlp.close()
+
+
+@pytest.mark.parametrize("n", [1, 63, 64, 65, 2113])
+def test_mlp_step_sizes(cv, gpu_ctx, n):
+    """Training steps of part-filled workgroups and of workgroup counts off the
+    reduction's unrolling (33 + 1): the step moves the parameters by Adam's
+    first step of the gradient, and the packed weights follow."""
+    import torch
+    log(f"[mlp] step of {n} rows")
+    p0 = cv.FarFieldMLP.init_params(4)
+    mlp = cv.FarFieldMLP(gpu_ctx, p0)
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 17)).astype(np.float32)
+    T = rng.uniform(0.1, 0.9, size=(n, 5)).astype(np.float32)
+    xd, td = torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda()
+    try:
+        g, loss = mlp.gradient(xd, td)
+        go, lo = O.mlp_grad(p0, X, T)
+        assert abs(loss - lo) <= 1e-2 * lo
+        assert np.linalg.norm(g - go) <= 2e-2 * np.linalg.norm(go)
+        mlp.train_step(xd, td, 1e-3)
+        q = mlp.get_params()
+        gf = g.astype(np.float64)
+        assert np.allclose(q, p0 - 1e-3 * gf / (np.abs(gf) + 1e-8), rtol=1e-5, atol=1e-6)
+        fresh = cv.FarFieldMLP(gpu_ctx, q)
+        assert torch.equal(mlp.forward(xd), fresh.forward(xd))
+        fresh.close()
+    finally:
+        mlp.close()
