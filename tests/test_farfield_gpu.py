@@ -157,6 +157,31 @@ def test_segments_match_oracle(cv, gpu_ctx, fmt, k):
     assert np.array_equal(t.view(np.uint32), to.view(np.uint32))
 
 
+# one start (16 lanes); groups that end inside a wave, fill a workgroup, start
+# the next; plain and compensated sums
+@pytest.mark.parametrize("fmt,n", [(1, 1), (1, 15), (2, 16), (1, 17), (2, 4099)])
+def test_segments_group_sizes(cv, gpu_ctx, fmt, n):
+    import torch
+    sc = _seg_scene(cv, fmt)
+    log(f"[farfield] segments fmt={fmt} n={n}")
+    p0 = np.tile(farfield_starts.starts(cv, sc, min(n, 2000), 17), (9, 1))[:n].copy()
+    p0[:, 1] += np.linspace(0.0, 0.02, n, dtype=np.float32)
+    vol, sun, cam, vox, tr = cv.scene_objects(sc, 0, context=gpu_ctx)
+    try:
+        vox.voxelize(vol, sun)
+        f, t, v = tr.segments(vol, sun, torch.from_numpy(p0).cuda(), 21)
+        torch.cuda.synchronize()
+        f, t, v = f.cpu().numpy(), t.cpu().numpy(), v.cpu().numpy()
+    finally:
+        vol.close()
+    vr = O.voxelize(sc)
+    nat, _, _, _ = O.build_levels(sc, vr.shell, vr.fill, want_f64=False)
+    fo, to, vo = O.segments(O.volume_of(sc), nat, O.cone_of(sc.cone), O.light_of(sc), 21, p0)
+    assert np.array_equal(v, vo)
+    assert np.array_equal(f.view(np.uint32), fo.view(np.uint32))
+    assert np.array_equal(t.view(np.uint32), to.view(np.uint32))
+
+
 def _render(cv, ctx, scene, fn):
     import torch
     vol, sun, cam, vox, tr = cv.scene_objects(scene, 0, context=ctx)
