@@ -167,15 +167,21 @@ struct FillSeg {
 void launch_fill_multi(const FillSeg* segs, int nseg, hipStream_t s);  // up to 4 segments, one launch
 size_t light_items_bound(int S, float max_radius, const LightView& lv, const GridDesc& g, int chord);
 
+// How the raster kernel walks the chords (cv_kernels.hip: k_light_raster_body)
+constexpr int kRasterGeneral = 0, kRasterPow2 = 1, kRasterQueue = 2;
 // LDS bitmap words of the raster kernel for this grid (its WORDS)
 __host__ __device__ inline int raster_words(const GridDesc& g) {
-    const bool p2 = g.pow2_range && g.pow2_N && g.pow2_step;
-    return p2 && g.nb0 <= 64 ? 2048 : 4096;
+    return g.pow2_range && g.nb0 <= 64 ? 2048 : 4096;
 }
 // The chord walk of a pass-1 item runs from the queue (the flat walk) when the
-// grid has power-of-two extents and the chord fill is on.
-__host__ __device__ inline bool raster_flat(const GridDesc& g, int chord) {
-    return chord && g.pow2_range && g.pow2_N && g.pow2_step;
+// grid has power-of-two world extents and the chord fill is on.
+__host__ __device__ inline bool raster_flat(const GridDesc& g, int chord) { return chord && g.pow2_range; }
+// Raster kernel of a grid: 0, 1 kRasterPow2, 2, 3 kRasterQueue (each with 2048,
+// 4096 bitmap words), 4 kRasterGeneral with 4096
+inline int raster_variant(const GridDesc& g, int chord) {
+    const int big = raster_words(g) == 2048 ? 0 : 1;
+    if (g.pow2_range && g.pow2_N && g.pow2_step) return big;
+    return raster_flat(g, chord) ? 2 + big : 4;
 }
 // Depth slices of a billboard's flat-walk items: the smallest power of two
 // K <= 32 for which the brick box of a full tile's chord slab cut into K
@@ -330,8 +336,8 @@ void launch_batch_stage(int stage, int variant, const BatchVox* scenes, const Ba
 // scenes the batched stages handle: sides multiple of 16, fused build up to
 // level 4 and every further level in the tail, at most 16384 billboards
 bool batch_vox_eligible(const GridDesc& g, const VolumeDesc& vd, int S);
-// launch shape of a stage for one scene: workgroups, and the variant (raster
-// <P2, WORDS> and sort width) that groups scenes into one launch
+// launch shape of a stage for one scene: workgroups, and the variant (raster_variant
+// and sort width) that groups scenes into one launch
 void batch_stage_shape(int stage, const BatchVox& b, int* blocks, int* variant);
 // segmented fill: one launch over many (pointer, count, value) segments
 void launch_fill_segments(const FillSeg* d_segs, const int* d_first, int nseg, int total_blocks, hipStream_t s);

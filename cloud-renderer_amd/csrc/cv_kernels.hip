@@ -112,25 +112,12 @@ __device__ __forceinline__ bool voxel_word_bit(const GridDesc& g, float px, floa
 }
 
 // same map, returning the brick coordinates and the bit inside the fill word
-// P2: the grid's extents are powers of two, x / range == x * (1 / range) exactly
-template <bool P2>
-__device__ __forceinline__ float div_range_t(const GridDesc& g, float x, int a) {
-    return P2 ? x * g.inv_range[a] : x / g.range[a];
-}
-template <bool P2 = false>
 __device__ __forceinline__ bool voxel_brick_bit(const GridDesc& g, float px, float py, float pz, int* bx, int* by,
                                                 int* bz, uint32_t* bit) {
     float fN = (float)g.N;
-    float lx, ly, lz;
-    if (P2) {
-        lx = fN * div_range_t<true>(g, px - g.lo[0], 0);
-        ly = fN * div_range_t<true>(g, py - g.lo[1], 1);
-        lz = fN * div_range_t<true>(g, pz - g.lo[2], 2);
-    } else {
-        lx = fN * div_range(g, px - g.lo[0], 0);
-        ly = fN * div_range(g, py - g.lo[1], 1);
-        lz = fN * div_range(g, pz - g.lo[2], 2);
-    }
+    float lx = fN * div_range(g, px - g.lo[0], 0);
+    float ly = fN * div_range(g, py - g.lo[1], 1);
+    float lz = fN * div_range(g, pz - g.lo[2], 2);
     if (!(lx > -1.0f && lx < fN && ly > -1.0f && ly < fN && lz > -1.0f && lz < fN)) return false;
     uint32_t ix = (uint32_t)(int)lx, iy = (uint32_t)(int)ly, iz = (uint32_t)(int)lz;
     *bx = (int)(ix >> 2);
@@ -478,10 +465,27 @@ __global__ void __launch_bounds__(256) k_light_prep(GridDesc g, LightView lv, co
 constexpr int kTilePixels = kLightTile * kLightTile;
 constexpr int kRasterThreads = 256;  // workgroup size of the raster kernels
 
-// P2: power-of-two extents (multiplications instead of IEEE divisions in
-// the index map, and an exact k * stepSize chord counter); WORDS: size of the
-// LDS chord bitmap (bigger volumes have bigger slabs behind a tile)
-template <bool P2, int WORDS>
+// Samples of the chord loop for (float i = 0; i < lim; i += step).  The k-th
+// counter value is within k^2 / 2^24 steps of k * step and lim * inv_step
+// within x / 2^23 of lim / step, so an x clear of every integer by more than
+// both decides alone; otherwise the counter runs.
+__device__ __forceinline__ int chord_samples(float lim, float step, float inv_step) {
+    if (!(lim > 0.0f)) return 0;
+    const float x = lim * inv_step;
+    if (fabsf(x - rintf(x)) > (x + 4.0f) * x * 0x1p-22f) return (int)ceilf(x);
+    int n = 0;
+    for (float i = 0.0f; i < lim; i += step) ++n;
+    return n;
+}
+
+// MODE 1 (kRasterPow2): power-of-two extents (multiplications instead of IEEE
+// divisions in the index map, and an exact k * stepSize chord counter).
+// MODE 2 (kRasterQueue): power-of-two world extents with any voxel count: the
+// index map is one multiplication too, the chord counter is accumulated.
+// MODE 0 (kRasterGeneral): any extents, and volumes without a chord fill.
+// WORDS: size of the LDS chord bitmap (bigger volumes have bigger slabs
+// behind a tile)
+template <int MODE, int WORDS>
 __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, int chord,
                                                       const int* __restrict__ total_ptr,
                                                       const RasterItem* __restrict__ items, int cap,
@@ -493,12 +497,15 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
     // margin for rounding) and flush non-zero words with one global atomic
     // each.  Stores falling outside the box (none expected) go straight to HBM.
     //
-    // With a power-of-two stepSize the chord loop counter i += stepSize is
-    // exactly k * stepSize: covered fragments are queued in LDS with their
-    // sample counts and the chords are walked from the queue, so no lane
-    // idles on a pixel outside the disc.  The queue is ordered by sample
-    // count, longest first (a counting sort over 128 buckets), so the 64
-    // chords a wave walks together have nearly the same length.
+    // Where a chord's sample count is known ahead (MODE 1: the loop counter
+    // i += stepSize is exactly k * stepSize; MODE 2: chord_samples), covered
+    // fragments are queued in LDS with their counts and the chords are walked
+    // from the queue, so no lane idles on a pixel outside the disc.  The queue
+    // is ordered by sample count, longest first (a counting sort over 128
+    // buckets), so the 64 chords a wave walks together have nearly the same
+    // length.  MODE 2 against a walk per pixel (MODE 0, which the extents then
+    // took): 57 -> 32 us at N = 150, 1001 billboards; 839 -> 537 us for the
+    // 96^3 and 192^3 scenes of a batch of 64.
     static_assert(WORDS <= 4096, "the flush decodes word indices below 4096 with float products");
     static_assert(kTilePixels % kRasterThreads == 0, "whole pixel rounds");
     constexpr int kRounds = kTilePixels / kRasterThreads;
@@ -510,7 +517,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
     __shared__ int q_start[128];  // chord-length buckets: counts, then first queue slots
     const int tid = threadIdx.x;
     const int total = min(*total_ptr, cap);
-    const bool flat = P2 && chord;
+    const bool flat = MODE != kRasterGeneral && chord;
     unsigned long long nfrag = 0, nchord = 0;
     // The item's setup comes from the work list.  The next item is fetched
     // while this one is rasterized: lanes 0..23 of every wave load one word
@@ -593,7 +600,9 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
             float lim = 2.0f * dist;
             if (flat) {
                 // k * stepSize < lim  <=>  k < lim / stepSize (exact: power-of-two scaling)
-                const int n = lim > 0.0f ? (int)ceilf(lim * g.inv_step) : 0;
+                const int n = MODE == kRasterQueue ? chord_samples(lim, g.stepSize, g.inv_step)
+                              : lim > 0.0f         ? (int)ceilf(lim * g.inv_step)
+                                                   : 0;
                 // this slice's samples k in [k0, k1): the first sample index
                 // whose depth -dist + k * stepSize reaches the slice bound
                 int k0 = 0, k1 = n;
@@ -625,7 +634,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                     int gx, gy, gz;
                     uint32_t b;
                     ++nchord;
-                    if (!voxel_brick_bit<P2>(g, qx, qy, qz, &gx, &gy, &gz, &b)) continue;
+                    if (!voxel_brick_bit(g, qx, qy, qz, &gx, &gy, &gz, &b)) continue;
                     if (gx != cbx || gy != cby || gz != cbz) {
                         flush(cbx, cby, cbz, cur_b);
                         cbx = gx; cby = gy; cbz = gz;
@@ -680,19 +689,24 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
         const int nfr = nfr_s;
         const float fN = (float)g.N;
         const float Bx = lv.B[0], By = lv.B[1], Bz = lv.B[2];
-        // N * ((q - lo) * (1 / range)): both factors are powers of two, so
-        // scaling once by their product rounds identically
+        // N * ((q - lo) * (1 / range)): the product with 1 / range is exact, so
+        // scaling once by N / range rounds identically
         const float kx = fN * g.inv_range[0], ky = fN * g.inv_range[1], kz = fN * g.inv_range[2];
         const uint32_t uN = (uint32_t)g.N;
+        // N a power of two: the three bounds fold into one test of the OR
+        auto all_below = [&](uint32_t ix, uint32_t iy, uint32_t iz) {
+            return MODE == kRasterQueue ? (ix < uN) & (iy < uN) & (iz < uN) : (ix | iy | iz) < uN;
+        };
         const uint32_t ubx = (uint32_t)bx0, uby = (uint32_t)by0, ubz = (uint32_t)bz0;
         const uint32_t unx = (uint32_t)nbx, uny = (uint32_t)nby, unz = (uint32_t)nbz;
         // word of brick (X, Y, Z) in the box: Z * unxy + Y * unx + X - wbase
         // (mod 2^32; the true value is in [0, words) for a brick in the box)
         const uint32_t unxy = unx * uny, wbase = (ubz * uny + uby) * unx + ubx;
         const float step = g.stepSize;
-        // k is a power of two, so scaling the operands of each rounded step by
-        // k scales its result exactly: ((s + B i) - lo) k == (s k + (B k) i) - lo k
-        // bit for bit (a subnormal B i vanishes in the add in both forms)
+        // MODE 1: k is a power of two, so scaling the operands of each rounded
+        // step by k scales its result exactly: ((s + B i) - lo) k ==
+        // (s k + (B k) i) - lo k bit for bit (a subnormal B i vanishes in the
+        // add in both forms)
         const float Bkx = Bx * kx, Bky = By * ky, Bkz = Bz * kz;
         const float lkx = g.lo[0] * kx, lky = g.lo[1] * ky, lkz = g.lo[2] * kz;
         for (int f0 = tid & ~63; f0 < nfr; f0 += blockDim.x) {
@@ -704,7 +718,11 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
             const int fn_ = f_n[f];
             const int n = nsl > 1 ? (fn_ & 0xffff) : fn_;  // samples k0 .. k0 + n - 1 of the chord
             const int k0 = nsl > 1 ? (fn_ >> 16) : 0;
-            const float i0 = (float)k0 * step;  // exact: power-of-two step
+            float i0 = (float)k0 * step;  // exact with a power-of-two step
+            if constexpr (MODE == kRasterQueue) {
+                i0 = 0.0f;
+                for (int k = 0; k < k0; ++k) i0 += step;
+            }
             if (use_lds) {
                 // the LDS word of the current brick, its bits OR-ed in a
                 // register: a brick change costs one LDS atomic
@@ -716,7 +734,9 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                 // chords skip the per-sample bounds tests.
                 bool inner;
                 {
-                    const float ie = (float)(k0 + n - 1) * g.stepSize;
+                    // MODE 2: an upper bound of the last sample's counter (chord_samples' error)
+                    const float ie = MODE == kRasterQueue ? ((float)(k0 + n - 1) + 0.01f) * step
+                                                          : (float)(k0 + n - 1) * step;
                     const float ax = ((sx + Bx * i0) - g.lo[0]) * kx, ay = ((sy + By * i0) - g.lo[1]) * ky;
                     const float az = ((sz + Bz * i0) - g.lo[2]) * kz;
                     const float bx = ((sx + Bx * ie) - g.lo[0]) * kx, by = ((sy + By * ie) - g.lo[1]) * ky;
@@ -726,7 +746,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                         return ((uint32_t)(int)l >> 2) - b0 < nb;
                     };
                     inner = ok(ax, ubx, unx) && ok(bx, ubx, unx) && ok(ay, uby, uny) && ok(by, uby, uny) &&
-                            ok(az, ubz, unz) && ok(bz, ubz, unz);
+                            ok(az, ubz, unz) && ok(bz, ubz, unz) && (MODE != kRasterQueue || k0 + n <= 256);
                 }
                 // the longest inner chord of the wave (every lane is active here)
                 int nmax = inner ? n : 0;
@@ -734,14 +754,20 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                 nmax = __builtin_amdgcn_readfirstlane(nmax);
                 if (inner) {
                     const float skx = sx * kx, sky = sy * ky, skz = sz * kz;
-                    // step k at i = min(k, n - 1) * stepSize: a lane past its
-                    // last sample repeats it.  i is accumulated: with a
-                    // power-of-two step every partial sum is exact.
+                    // a lane past its last sample repeats it.  i is accumulated, as
+                    // in the loop (with a power-of-two step every partial sum is
+                    // exact: step k lies at i = min(k, n - 1) * stepSize).
                     const float ilast = (float)(k0 + n - 1) * step;
                     auto voxel = [&](float i, uint32_t& ix, uint32_t& iy, uint32_t& iz) {
-                        ix = (uint32_t)(int)((skx + Bkx * i) - lkx);
-                        iy = (uint32_t)(int)((sky + Bky * i) - lky);
-                        iz = (uint32_t)(int)((skz + Bkz * i) - lkz);
+                        if constexpr (MODE == kRasterQueue) {
+                            ix = (uint32_t)(int)(((sx + Bx * i) - g.lo[0]) * kx);
+                            iy = (uint32_t)(int)(((sy + By * i) - g.lo[1]) * ky);
+                            iz = (uint32_t)(int)(((sz + Bz * i) - g.lo[2]) * kz);
+                        } else {
+                            ix = (uint32_t)(int)((skx + Bkx * i) - lkx);
+                            iy = (uint32_t)(int)((sky + Bky * i) - lky);
+                            iz = (uint32_t)(int)((skz + Bkz * i) - lkz);
+                        }
                     };
                     // byte offset of the brick's word in the box,
                     // ((Z * unxy + Y * unx + X) - wbase) * 8 mod 2^32 (factors
@@ -757,8 +783,13 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                     cur_b = bit64_mod(rot_bit_index(ix, iy, iz));
                     float iacc = i0;
                     for (int k = 1; k < nmax; ++k) {
-                        iacc += step;
-                        voxel(min_no_nan(iacc, ilast), ix, iy, iz);
+                        if constexpr (MODE == kRasterQueue) {
+                            iacc = k < n ? iacc + step : iacc;
+                            voxel(iacc, ix, iy, iz);
+                        } else {
+                            iacc += step;
+                            voxel(min_no_nan(iacc, ilast), ix, iy, iz);
+                        }
                         const uint32_t a = waddr(ix, iy, iz);
                         const unsigned long long m = bit64_mod(rot_bit_index(ix, iy, iz));
                         if (a != cur_a) {
@@ -778,7 +809,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                     const float ly = __builtin_amdgcn_fmed3f((qy - g.lo[1]) * ky, -2.0f, fN);
                     const float lz = __builtin_amdgcn_fmed3f((qz - g.lo[2]) * kz, -2.0f, fN);
                     const uint32_t ix = (uint32_t)(int)lx, iy = (uint32_t)(int)ly, iz = (uint32_t)(int)lz;
-                    const bool in = (ix | iy | iz) < uN;
+                    const bool in = all_below(ix, iy, iz);
                     // brick offsets in the slab's box (unsigned: below the box wraps high)
                     const uint32_t ux = (ix >> 2) - ubx, uy = (iy >> 2) - uby, uz = (iz >> 2) - ubz;
                     const bool inbox = (ux < unx) & (uy < uny) & (uz < unz);
@@ -802,18 +833,16 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
             // bricks per axis), bits of the current word OR-ed in a register
             uint32_t cur_key = 0xffffffffu;
             unsigned long long cur_b = 0ull;
-            for (int k = k0; k < k0 + n; ++k) {
-                const float i = (float)k * g.stepSize;
+            float i = i0;
+            for (int k = 0; k < n; ++k, i += step) {
                 const float qx = sx + Bx * i, qy = sy + By * i, qz = sz + Bz * i;
-                // voxel_brick_bit with power-of-two extents, branch free
-                // clamped to [-2, N]: -1 < l < N  <=>  0 <= (int)l < N (truncation
-                // toward zero), and with N a power of two the three unsigned
-                // bounds fold into one test of the OR
+                // voxel_brick_bit, branch free: clamped to [-2, N],
+                // -1 < l < N  <=>  0 <= (int)l < N (truncation toward zero)
                 const float lx = __builtin_amdgcn_fmed3f((qx - g.lo[0]) * kx, -2.0f, fN);
                 const float ly = __builtin_amdgcn_fmed3f((qy - g.lo[1]) * ky, -2.0f, fN);
                 const float lz = __builtin_amdgcn_fmed3f((qz - g.lo[2]) * kz, -2.0f, fN);
                 const uint32_t ix = (uint32_t)(int)lx, iy = (uint32_t)(int)ly, iz = (uint32_t)(int)lz;
-                const bool in = (ix | iy | iz) < uN;
+                const bool in = all_below(ix, iy, iz);
                 // brick coordinates (< 512) in 9-bit fields
                 const uint32_t key = (ix >> 2) | ((iy << 7) & 0x3fe00u) | ((iz << 16) & 0x7fc0000u);
                 const unsigned long long m = 1ull << ((ix & 3u) | ((iy << 2) & 0xcu) | ((iz << 4) & 0x30u));
@@ -860,14 +889,14 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
         }
     }
 }
-template <bool P2, int WORDS>
+template <int MODE, int WORDS>
 __global__ void __launch_bounds__(256) k_light_raster(GridDesc g, LightView lv, int chord,
                                                       const int* __restrict__ total_ptr,
                                                       const RasterItem* __restrict__ items, int cap,
                                                       unsigned long long* __restrict__ keys,
                                                       unsigned long long* __restrict__ fillbits,
                                                       unsigned long long* __restrict__ counters) {
-    k_light_raster_body<P2, WORDS>(g, lv, chord, total_ptr, items, cap, keys, fillbits, counters, (int)blockIdx.x, (int)gridDim.x);
+    k_light_raster_body<MODE, WORDS>(g, lv, chord, total_ptr, items, cap, keys, fillbits, counters, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -3948,17 +3977,18 @@ void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const
     if (S <= 0) return;
     const int cap = (int)std::min<size_t>(ls.items_cap, 0x7fffffff);
     unsigned grid = (unsigned)std::min<size_t>(ls.items_cap, 4096);
-    const bool p2 = g.pow2_range && g.pow2_N && g.pow2_step;
     const int chord = mode == 1 ? 1 : 0;
-    if (p2 && raster_words(g) == 2048)
-        hipLaunchKernelGGL((k_light_raster<true, 2048>), dim3(grid), dim3(256), 0, s, g, lv, chord, ls.offsets + S,
-                           ls.items, cap, keys, fillbits, counters);
-    else if (p2)
-        hipLaunchKernelGGL((k_light_raster<true, 4096>), dim3(grid), dim3(256), 0, s, g, lv, chord, ls.offsets + S,
-                           ls.items, cap, keys, fillbits, counters);
-    else
-        hipLaunchKernelGGL((k_light_raster<false, 4096>), dim3(grid), dim3(256), 0, s, g, lv, chord, ls.offsets + S,
-                           ls.items, cap, keys, fillbits, counters);
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(grid), dim3(256), 0, s, g, lv, chord, ls.offsets + S, ls.items, cap, keys,
+                           fillbits, counters);
+    };
+    switch (raster_variant(g, chord)) {
+        case 0: go(k_light_raster<kRasterPow2, 2048>); break;
+        case 1: go(k_light_raster<kRasterPow2, 4096>); break;
+        case 2: go(k_light_raster<kRasterQueue, 2048>); break;
+        case 3: go(k_light_raster<kRasterQueue, 4096>); break;
+        default: go(k_light_raster<kRasterGeneral, 4096>);
+    }
 }
 
 size_t light_items_bound(int S, float max_radius, const LightView& lv, const GridDesc& g, int chord) {
@@ -4389,11 +4419,11 @@ __global__ void __launch_bounds__(256) kb_light_prep(const BatchVox* __restrict_
     k_light_prep_body(B.g, B.lv, B.boards, B.lbox, B.offsets + B.S, B.items, (int)min(B.items_cap, 0x7fffffff), B.chord,
                       B.words, q.bid, q.nblk);
 }
-template <bool P2, int WORDS>
+template <int MODE, int WORDS>
 __global__ void __launch_bounds__(256) kb_light_raster(const BatchVox* __restrict__ sc, BatchStage st) {
     const StageSlot q = stage_slot(st);
     const BatchVox& B = sc[q.sc];
-    k_light_raster_body<P2, WORDS>(B.g, B.lv, B.chord, B.offsets + B.S, B.items, (int)min(B.items_cap, 0x7fffffff),
+    k_light_raster_body<MODE, WORDS>(B.g, B.lv, B.chord, B.offsets + B.S, B.items, (int)min(B.items_cap, 0x7fffffff),
                                    B.keys, B.fill, nullptr, q.bid, q.nblk);
 }
 __global__ void __launch_bounds__(256) kb_light_splat(const BatchVox* __restrict__ sc, BatchStage st) {
@@ -4477,8 +4507,7 @@ void batch_stage_shape(int stage, const BatchVox& b, int* blocks, int* variant) 
             break;
         case kBsRaster: {
             *blocks = S > 0 ? (int)std::min<size_t>((size_t)b.items_cap, 4096) : 0;
-            const bool p2 = b.g.pow2_range && b.g.pow2_N && b.g.pow2_step;
-            *variant = p2 ? (raster_words(b.g) == 2048 ? 0 : 1) : 2;
+            *variant = raster_variant(b.g, b.chord);
             break;
         }
         case kBsSplat:
@@ -4523,9 +4552,11 @@ void launch_batch_stage(int stage, int variant, const BatchVox* scenes, const Ba
         case kBsExpand: hipLaunchKernelGGL(kb_light_expand, grid, dim3(256), 0, s, scenes, st); break;
         case kBsPrep: hipLaunchKernelGGL(kb_light_prep, grid, dim3(256), 0, s, scenes, st); break;
         case kBsRaster:
-            if (variant == 0) hipLaunchKernelGGL((kb_light_raster<true, 2048>), grid, dim3(256), 0, s, scenes, st);
-            else if (variant == 1) hipLaunchKernelGGL((kb_light_raster<true, 4096>), grid, dim3(256), 0, s, scenes, st);
-            else hipLaunchKernelGGL((kb_light_raster<false, 4096>), grid, dim3(256), 0, s, scenes, st);
+            if (variant == 0) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, 2048>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 1) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, 4096>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 2) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, 2048>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 3) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, 4096>), grid, dim3(256), 0, s, scenes, st);
+            else hipLaunchKernelGGL((kb_light_raster<kRasterGeneral, 4096>), grid, dim3(256), 0, s, scenes, st);
             break;
         case kBsSplat: hipLaunchKernelGGL(kb_light_splat, grid, dim3(256), 0, s, scenes, st); break;
         case kBsBuild:
