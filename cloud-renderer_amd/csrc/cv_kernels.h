@@ -282,7 +282,6 @@ struct BatchScene {
     const unsigned long long* masks;
     void* image;
     int words;
-    int tile0;  // first global tile of the scene
 };
 
 // One scene of a batch's voxelization and camera pass, as the batched stage
@@ -345,17 +344,26 @@ int fill_segment_blocks(uint64_t n);
 // fills the kernel-derived fields of b (raster bitmap words, fused build shape)
 void batch_vox_complete(BatchVox& b);
 
-// batched cone trace: work items are global tiles in `order` (heavy first);
+// batched cone trace: work items are the scenes' tiles in `order` (scene i's
+// from place tile0[i] on, heavy first, by their index in the scene);
 // waves_per_group waves per workgroup, `groups` workgroups striding over the
 // items (groups = 0: one workgroup per waves_per_group items)
 void launch_cone_batch(const BatchScene* scenes, const int* tile0, int nscenes, const int* order, int total_tiles,
                        int format, int cone_mode, int composite, int waves_per_group, int groups,
                        unsigned long long* counters, hipStream_t s);
-// binning into a caller-given tile_count array, and the heavy-first order of
-// an array of tile counts (scratch: 64 + ntiles ints)
+// binning into a caller-given tile_count array
 void launch_bin_counts(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int words,
                        unsigned long long* masks, int* tile_count, hipStream_t s);
-void launch_tile_order(const int* tile_count, int ntiles, int* scratch, int* tile_order, hipStream_t s);
+// up to kTileBlock tiles of one scene of a batch: tiles tile .. tile + n - 1 of
+// the scene, whose counts start at t0; order0: the scene's first place in the order
+constexpr int kTileBlock = 1024;
+struct TileBlock {
+    int scene, t0, n, tile, order0;
+};
+// heavy-first order of every scene's tiles (scratch: 64 nscenes + tiles ints,
+// the first 64 nscenes cleared)
+void launch_batch_order(const TileBlock* blocks, int nblocks, int nscenes, const int* tile_count, int* scratch,
+                        int* tile_order, hipStream_t s);
 
 // LDS tables of the table-addressed cone kernel: per level, word offsets of
 // three arrays indexed by floor(u) + 1 for the in-volume range

@@ -2520,7 +2520,7 @@ __global__ void __launch_bounds__(256) k_tile_scatter(const int* __restrict__ bu
             bfirst[threadIdx.x] = f;
             bshift[threadIdx.x] = sh;
         }
-        if (total && blockIdx.x == 0 && threadIdx.x == 0) *total = all;
+        if (blockIdx.x == 0 && threadIdx.x == 0) *total = all;
     }
     __syncthreads();
     if (threadIdx.x < 32 && lh[threadIdx.x] > 0) lbase[threadIdx.x] = atomicAdd(&cursor[threadIdx.x], lh[threadIdx.x]);
@@ -2528,9 +2528,62 @@ __global__ void __launch_bounds__(256) k_tile_scatter(const int* __restrict__ bu
     if (key < 0) return;
     const int sh = bshift[key];
     int* o = tile_order + bfirst[key] + ((lbase[key] + lrank) << sh);
-    if (!total) *o = t;  // whole tiles by their index
-    else
-        for (int p = 0; p < 1 << sh; ++p) o[p] = tile_item(t, p, sh);
+    for (int p = 0; p < 1 << sh; ++p) o[p] = tile_item(t, p, sh);
+}
+
+// The heavy-first order of the tiles of every scene of a batch, each scene's
+// tiles in their own range of the order: k_tile_bucket and k_tile_scatter with
+// a histogram per scene.  A workgroup takes up to kTileBlock tiles of one
+// scene.  With one order over all scenes every workgroup added to the same 32
+// counters: 58 us against 12 for 64 scenes.
+__global__ void __launch_bounds__(256) k_batch_bucket(const TileBlock* __restrict__ blocks,
+                                                      const int* __restrict__ tile_count, int* __restrict__ bucket_of,
+                                                      int* __restrict__ hist) {
+    __shared__ int lh[32];
+    const TileBlock b = blocks[blockIdx.x];
+    if (threadIdx.x < 32) lh[threadIdx.x] = 0;
+    __syncthreads();
+    for (int t = b.t0 + (int)threadIdx.x; t < b.t0 + b.n; t += 256) {
+        const int c = tile_count[t];
+        const int key = 31 - (c == 0 ? 0 : 32 - __clz(c));
+        bucket_of[t] = key;
+        atomicAdd(&lh[key], 1);
+    }
+    __syncthreads();
+    if (threadIdx.x < 32 && lh[threadIdx.x] > 0) atomicAdd(&hist[b.scene * 32 + threadIdx.x], lh[threadIdx.x]);
+}
+__global__ void __launch_bounds__(256) k_batch_scatter(const TileBlock* __restrict__ blocks,
+                                                       const int* __restrict__ bucket_of, const int* __restrict__ hist,
+                                                       int* __restrict__ cursor, int* __restrict__ tile_order) {
+    static_assert(kTileBlock % 256 == 0, "whole rounds of 256 threads");
+    __shared__ int lh[32], lbase[32];
+    const TileBlock b = blocks[blockIdx.x];
+    const int tid = threadIdx.x;
+    if (tid < 32) lh[tid] = 0;
+    __syncthreads();
+    int key[kTileBlock / 256], rank[kTileBlock / 256];
+#pragma unroll
+    for (int e = 0; e < kTileBlock / 256; ++e) {
+        const int t = tid + 256 * e;
+        key[e] = t < b.n ? bucket_of[b.t0 + t] : -1;
+        rank[e] = key[e] >= 0 ? atomicAdd(&lh[key[e]], 1) : 0;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        // first rank of each bucket in the scene, then this workgroup's part of it
+        const int h = tid < 32 ? hist[b.scene * 32 + tid] : 0;
+        int incl = h;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const int y = __shfl_up(incl, o, 64);
+            if (tid >= o) incl += y;
+        }
+        if (tid < 32 && lh[tid] > 0) lbase[tid] = incl - h + atomicAdd(&cursor[b.scene * 32 + tid], lh[tid]);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kTileBlock / 256; ++e)
+        if (key[e] >= 0) tile_order[b.order0 + lbase[key[e]] + rank[e]] = b.tile + tid + 256 * e;
 }
 
 // ---------------------------------------------------------------------------
@@ -3650,10 +3703,11 @@ __global__ void __launch_bounds__(512, 6) k_cone_tab(GridDesc g, VolumeDesc vd, 
     }
 }
 
-// Batched cone trace: global tiles of many scenes (heavy first), each wave
-// finds its scene by binary search over the scenes' first tiles.
+// Batched cone trace: the tiles of many scenes, scene after scene and heavy
+// first in each; a wave finds its item's scene by binary search over the
+// scenes' first items.
 template <int FMT, int CONE, int COMP>
-__global__ void __launch_bounds__(256) k_cone_batch(const BatchScene* __restrict__ scenes,
+__global__ void __launch_bounds__(256, 5) k_cone_batch(const BatchScene* __restrict__ scenes,
                                                     const int* __restrict__ tile0, int nscenes,
                                                     const int* __restrict__ gorder, int total,
                                                     unsigned long long* __restrict__ counters) {
@@ -3664,17 +3718,17 @@ __global__ void __launch_bounds__(256) k_cone_batch(const BatchScene* __restrict
     uint32_t nfrag = 0, nsamp = 0, ntwo = 0, nrows = 0, nfall = 0, nevals = 0;
     const MlpDev none{nullptr, nullptr, nullptr};
     for (int item = blockIdx.x * wpg + wave; item < total; item += gridDim.x * wpg) {
-        const int gt = __builtin_amdgcn_readfirstlane(gorder[item]);
+        const int tile = __builtin_amdgcn_readfirstlane(gorder[item]);
         int lo = 0, hi = nscenes - 1;
-        while (lo < hi) {  // last scene with tile0 <= gt
+        while (lo < hi) {  // last scene with tile0 <= item
             const int mid = (lo + hi + 1) >> 1;
-            if (tile0[mid] <= gt) lo = mid;
+            if (tile0[mid] <= item) lo = mid;
             else hi = mid - 1;
         }
         const int sidx = __builtin_amdgcn_readfirstlane(lo);
         const BatchScene& B = scenes[sidx];
         cone_tile<FMT, CONE, COMP, 0>(B.g, B.vd, B.cv, B.cd, B.levels, B.sph_world, B.sph_view, B.order, B.masks,
-                                      B.words, B.image, none, nullptr, L[wave], gt - B.tile0, 0, 0, lane,
+                                      B.words, B.image, none, nullptr, L[wave], tile, 0, 0, lane,
                                       counters != nullptr, nfrag, nsamp, ntwo, nrows, nfall, nevals);
     }
     if (counters) {
@@ -4181,16 +4235,14 @@ void launch_bin_counts(const int4* sph_tiles, const int32_t* order, int S, int t
                            tile_count);
 }
 
-// heavy-first order of ntiles tile counts; scratch: hist[32] | cursor[32] | bucket_of[ntiles]
-void launch_tile_order(const int* tile_count, int ntiles, int* scratch, int* tile_order, hipStream_t s) {
+// scratch: hist[32 nscenes] | cursor[32 nscenes] (cleared by the caller) | bucket_of[tiles]
+void launch_batch_order(const TileBlock* blocks, int nblocks, int nscenes, const int* tile_count, int* scratch,
+                        int* tile_order, hipStream_t s) {
     int* hist = scratch;
-    int* cursor = scratch + 32;
-    int* bucket_of = scratch + 64;
-    launch_fill_u64((uint64_t*)scratch, 32, 0, s);
-    hipLaunchKernelGGL(k_tile_bucket, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, tile_count, ntiles, bucket_of,
-                       hist);
-    hipLaunchKernelGGL(k_tile_scatter, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, bucket_of, ntiles, hist, cursor,
-                       tile_order, TileSplit{0.0f, 0, 0}, (int*)nullptr);
+    int* cursor = scratch + 32 * (size_t)nscenes;
+    int* bucket_of = scratch + 64 * (size_t)nscenes;
+    hipLaunchKernelGGL(k_batch_bucket, dim3(nblocks), dim3(256), 0, s, blocks, tile_count, bucket_of, hist);
+    hipLaunchKernelGGL(k_batch_scatter, dim3(nblocks), dim3(256), 0, s, blocks, bucket_of, hist, cursor, tile_order);
 }
 
 // Binning plus the heavy-first item order.  tile scratch (ints): hist[32] |
