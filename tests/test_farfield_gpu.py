@@ -350,3 +350,23 @@ def test_mlp_step_sizes(cv, gpu_ctx, n):
         fresh.close()
     finally:
         mlp.close()
+
+
+@pytest.mark.parametrize("n", [16384, 16385, 32769])
+def test_mlp_reduction_rounds(cv, gpu_ctx, n):
+    """256, 257 and 513 workgroups' partials (one, two and three rounds of the
+    reduction): gradient and loss of the oracle."""
+    import torch
+    log(f"[mlp] gradient of {n} rows")
+    p0 = cv.FarFieldMLP.init_params(4)
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 17)).astype(np.float32)
+    T = rng.uniform(0.1, 0.9, size=(n, 5)).astype(np.float32)
+    mlp = cv.FarFieldMLP(gpu_ctx, p0)
+    try:
+        g, loss = mlp.gradient(torch.from_numpy(X).cuda(), torch.from_numpy(T).cuda())
+    finally:
+        mlp.close()
+    go, lo = O.mlp_grad(p0, X, T)
+    assert abs(loss - lo) <= 1e-2 * lo
+    assert np.linalg.norm(g - go) <= 2e-2 * np.linalg.norm(go)
