@@ -211,9 +211,10 @@ __host__ __device__ inline int light_slices(const GridDesc& g, const LightView& 
     if (2.0f * s / g.stepSize >= 65535.0f) return 1;
     return light_slices_box(g, lv, s, words);  // non-decreasing in s: the work-list bound takes the largest s
 }
-// the pass-1 work list (boxes, scan, items); launch_light_raster reads it
+// the pass-1 work list (boxes, scan, items; launch_light_raster reads it) and
+// the fill of up to 4 segments, which its first launch takes along
 void launch_light_items(const GridDesc& g, const LightView& lv, int mode, const float4* boards, int S,
-                        const LightScratch& ls, hipStream_t s);
+                        const LightScratch& ls, const FillSeg* segs, int nseg, hipStream_t s);
 void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const float4* boards, int S,
                          const LightScratch& ls, unsigned long long* keys, unsigned long long* fillbits,
                          unsigned long long* counters, hipStream_t s);
@@ -237,7 +238,13 @@ size_t foot_slots(VolumeDesc& vd);
 void launch_foot_r8(const GridDesc& g, const VolumeDesc& vd, const unsigned long long* shellbits, const void* levels,
                     uint2* foot, uint8_t* zero, hipStream_t s);
 void launch_cam_setup(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
-                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, hipStream_t s);
+                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, const FillSeg* segs, int nseg,
+                      hipStream_t s);
+// camera setup, draw order (upload: the identity) and the fill in one launch;
+// false (nothing launched) beyond 1024 billboards
+bool launch_cam_front(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
+                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, int32_t* order, int* tie_flag,
+                      bool upload, const FillSeg* segs, int nseg, hipStream_t s);
 size_t sort_scratch_words(int S);
 // keys of a sort far to near from `point` alone (CloudVolume::sortBoards), and
 // the identity order (billboards drawn in upload order)
@@ -266,6 +273,8 @@ struct TileSplit {
     int fixed;
 };
 size_t tile_scratch_ints(int ntiles);
+// what launch_bin needs cleared
+void bin_clear_segs(unsigned long long* masks, int* scratch, int ntiles, int words, FillSeg out[2]);
 TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int tiles_y, int words,
                      unsigned long long* masks, int* scratch, bool every_fragment, hipStream_t s);
 // One scene of a batched cone-trace launch (device resident; the batched

@@ -219,9 +219,9 @@ struct FillArgs {
     uint64_t v[4];
     int nseg;
 };
-__global__ void k_fill_multi(FillArgs a) {
-    uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const uint64_t stride = (uint64_t)gridDim.x * blockDim.x;
+__device__ __forceinline__ void fill_multi_body(const FillArgs& a, uint32_t bid, uint32_t nblk) {
+    uint64_t i = (uint64_t)bid * blockDim.x + threadIdx.x;
+    const uint64_t stride = (uint64_t)nblk * blockDim.x;
     const uint64_t total = a.n[0] + a.n[1] + a.n[2] + a.n[3];
     for (; i < total; i += stride) {
         uint64_t r = i;
@@ -230,6 +230,7 @@ __global__ void k_fill_multi(FillArgs a) {
         a.p[k][r] = a.v[k];
     }
 }
+__global__ void k_fill_multi(FillArgs a) { fill_multi_body(a, blockIdx.x, gridDim.x); }
 
 // ---------------------------------------------------------------------------
 // pass 1: light-view raster (res/first_voxelize.glsl:39-64)
@@ -306,6 +307,7 @@ __device__ __forceinline__ int light_box(const GridDesc& g, const LightView& lv,
     return cnt;
 }
 
+constexpr int kListOne = 1024;  // k_light_front
 // The pass-1 work list: every billboard's pixel box (lbox) and tile count,
 // the exclusive scan of the counts (offsets[S] = the uncut item count) and
 // the (billboard, tile) items in billboard order, cut at cap.  Three small
@@ -320,10 +322,6 @@ __device__ __forceinline__ void k_light_boxes_body(GridDesc g, LightView lv, con
     int4 box;
     counts[j] = light_box(g, lv, boards[j], raster_flat(g, chord) ? 1 : 0, raster_words(g), &box);
     lbox[j] = box;
-}
-__global__ void __launch_bounds__(256) k_light_boxes(GridDesc g, LightView lv, const float4* __restrict__ boards,
-                                                     int S, int4* __restrict__ lbox, int* __restrict__ counts, int chord) {
-    k_light_boxes_body(g, lv, boards, S, lbox, counts, chord, (int)blockIdx.x, (int)gridDim.x);
 }
 
 // one workgroup: 4096 counts per round, 16 consecutive per thread
@@ -426,14 +424,60 @@ __global__ void __launch_bounds__(256) k_light_expand(const int* __restrict__ of
     k_light_expand_body(offsets, S, items, cap, (int)blockIdx.x, (int)gridDim.x);
 }
 
+// The first launch of a voxelization: `nfront` workgroups for the work list,
+// the others clear.  A small frame is its launches (16 of them for 82 us of
+// kernels, 150 us a frame), so up to kListOne billboards one workgroup takes
+// all boxes and scans them, and the items' setup finds its billboards in the
+// offsets; more take their boxes here, and the scan and the enumeration of the
+// items launches of their own.  With the camera passes in one launch and the
+// tile order in one (k_cam_front, k_tile_order), 10 launches: a 32^3, 256 x 256
+// frame 164 -> 129 us among others.  (Items enumerated in the one workgroup
+// took 20 us where 200 billboards have 900 tiles each.)
+__global__ void __launch_bounds__(256) k_light_front(GridDesc g, LightView lv, const float4* boards, int S,
+                                                     int4* lbox, int* counts, int* offsets, int chord, int nfront,
+                                                     FillArgs fill) {
+    if ((int)blockIdx.x >= nfront) {
+        fill_multi_body(fill, blockIdx.x - nfront, gridDim.x - nfront);
+        return;
+    }
+    if (S > kListOne) {
+        k_light_boxes_body(g, lv, boards, S, lbox, counts, chord, (int)blockIdx.x, nfront);
+        return;
+    }
+    for (int b = 0; b * 256 < S; ++b) k_light_boxes_body(g, lv, boards, S, lbox, counts, chord, b, 0);
+    __syncthreads();
+    k_light_scan_body(counts, S, offsets);
+}
+
 // one thread per item: the tile's rectangle, the billboard's light-view data
-// and the slab box
+// and the slab box.  SEARCH (at most kListOne billboards): the item's billboard
+// from the offsets, kept in LDS, instead of its first two words.
+template <bool SEARCH>
 __device__ __forceinline__ void k_light_prep_body(GridDesc g, LightView lv, const float4* __restrict__ boards,
-                                                    const int4* __restrict__ lbox, const int* __restrict__ total_ptr,
-                                                    RasterItem* __restrict__ items, int cap, int chord, int words, int bid, int nblk) {
-    const int n = min(*total_ptr, cap);
+                                                    const int4* __restrict__ lbox, const int* __restrict__ offsets,
+                                                    int S, RasterItem* __restrict__ items, int cap, int chord,
+                                                    int words, int bid, int nblk) {
+    __shared__ int first[SEARCH ? kListOne : 1];
+    const int n = min(offsets[S], cap);
+    if (bid * 256 >= n) return;
+    if constexpr (SEARCH) {
+        for (int j = threadIdx.x; j < S; j += 256) first[j] = offsets[j];
+        __syncthreads();
+    }
     for (int i = bid * 256 + threadIdx.x; i < n; i += nblk * 256) {
-    const int2 jt = *(const int2*)&items[i];
+    int2 jt;
+    if constexpr (SEARCH) {
+        // the last billboard whose first item is at most i (the ones without items share the next one's)
+        int lo = 0, hi = S - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi + 1) >> 1;
+            if (first[mid] <= i) lo = mid;
+            else hi = mid - 1;
+        }
+        jt = make_int2(lo, i - first[lo]);
+    } else {
+        jt = *(const int2*)&items[i];
+    }
     const int j = jt.x;
     const LightSphere o = light_sphere(g, lv, boards[j]);
     // item t of the billboard: tile t / K, depth slice t % K (light_box's K)
@@ -456,10 +500,12 @@ __device__ __forceinline__ void k_light_prep_body(GridDesc g, LightView lv, cons
     items[i] = it;
     }
 }
+template <bool SEARCH>
 __global__ void __launch_bounds__(256) k_light_prep(GridDesc g, LightView lv, const float4* __restrict__ boards,
-                                                    const int4* __restrict__ lbox, const int* __restrict__ total_ptr,
+                                                    const int4* __restrict__ lbox, const int* __restrict__ offsets, int S,
                                                     RasterItem* __restrict__ items, int cap, int chord, int words) {
-    k_light_prep_body(g, lv, boards, lbox, total_ptr, items, cap, chord, words, (int)blockIdx.x, (int)gridDim.x);
+    k_light_prep_body<SEARCH>(g, lv, boards, lbox, offsets, S, items, cap, chord, words, (int)blockIdx.x,
+                              (int)gridDim.x);
 }
 
 constexpr int kTilePixels = kLightTile * kLightTile;
@@ -1946,8 +1992,12 @@ __device__ __forceinline__ void k_cam_setup_body(GridDesc g, CameraView cv, cons
 __global__ void __launch_bounds__(256) k_cam_setup(GridDesc g, CameraView cv, const float4* __restrict__ boards, int S,
                                                    float4* __restrict__ sph_world, float4* __restrict__ sph_view,
                                                    int4* __restrict__ sph_tiles, unsigned long long* __restrict__ keys,
-                                                   int* __restrict__ ranks) {
-    k_cam_setup_body(g, cv, boards, S, sph_world, sph_view, sph_tiles, keys, ranks, (int)blockIdx.x, (int)gridDim.x);
+                                                   int* __restrict__ ranks, int nfront, FillArgs fill) {
+    if ((int)blockIdx.x >= nfront) {  // the other workgroups clear
+        fill_multi_body(fill, blockIdx.x - nfront, gridDim.x - nfront);
+        return;
+    }
+    k_cam_setup_body(g, cv, boards, S, sph_world, sph_view, sph_tiles, keys, ranks, (int)blockIdx.x, nfront);
 }
 
 // ---------------------------------------------------------------------------
@@ -2231,13 +2281,13 @@ __device__ __forceinline__ void wave_bitonic(unsigned long long (&v)[E], int lan
 // a binary search gives each thread its E outputs).  The keys are
 // (~distance bits << 32 | index), distinct for distinct billboards, so the
 // ascending order is the draw order up to runs of equal distances.
-template <int E>
+template <int E, int NT = 1024>
 __device__ __forceinline__ void k_sort_lds_body(const unsigned long long* __restrict__ keys_in, int S,
                                                    int32_t* __restrict__ order, int* __restrict__ tie_flag) {
     extern __shared__ unsigned long long sk[];
     __shared__ int tie;
-    constexpr int npad = 1024 * E;
-    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
+    constexpr int npad = NT * E, nt = NT;
+    const int tid = threadIdx.x, lane = tid & 63;
     if (tid == 0) tie = 0;
     {
         unsigned long long v[E];
@@ -2280,10 +2330,10 @@ __device__ __forceinline__ void k_sort_lds_body(const unsigned long long* __rest
         for (int e = 0; e < E; ++e) sk[pos + e] = out[e];
         __syncthreads();
     }
-    // Reuse the key storage for the steps' words.  Chunk c of 1024 keys is read
-    // before its words are written; those writes cover keys [512 c, 512 c +
-    // 512), all of which were read in chunks <= c, and the previous key of the
-    // next chunk (index 1024 (c+1) - 1) is not touched.
+    // Reuse the key storage for the steps' words.  Chunk c of NT keys is read
+    // before its words are written; those writes cover keys [NT / 2 c, NT / 2 c +
+    // NT / 2), all of which were read in chunks <= c, and the previous key of the
+    // next chunk (index NT (c+1) - 1) is not touched.
     uint32_t* w = (uint32_t*)sk;
     for (int c = 0; c < npad; c += nt) {
         const int i = c + tid;
@@ -2314,6 +2364,27 @@ __device__ __forceinline__ void k_sort_lds_body(const unsigned long long* __rest
 __global__ void __launch_bounds__(1024) k_sort_lds(const unsigned long long* __restrict__ keys_in, int S,
                                                    int32_t* __restrict__ order, int* __restrict__ tie_flag) {
     k_sort_lds_body<1>(keys_in, S, order, tie_flag);
+}
+
+// Camera setup and draw order of at most 1024 billboards in one workgroup, the
+// others clear: one launch instead of three.  256 threads a workgroup, which
+// find room on CUs that the previous frame's kernels keep busy.
+__global__ void __launch_bounds__(256) k_cam_front(GridDesc g, CameraView cv, const float4* boards, int S,
+                                                   float4* sph_world, float4* sph_view, int4* sph_tiles,
+                                                   unsigned long long* keys, int32_t* order, int* tie_flag, int upload,
+                                                   FillArgs fill) {
+    if (blockIdx.x > 0) {
+        fill_multi_body(fill, blockIdx.x - 1, gridDim.x - 1);
+        return;
+    }
+    for (int b = 0; b * 256 < S; ++b)
+        k_cam_setup_body(g, cv, boards, S, sph_world, sph_view, sph_tiles, keys, nullptr, b, 0);
+    __syncthreads();
+    if (upload) {
+        for (int j = threadIdx.x; j < S; j += 256) order[j] = j;
+    } else {
+        k_sort_lds_body<4, 256>(keys, S, order, tie_flag);
+    }
 }
 
 // Draw order of 1025 .. 16384 billboards by counting: a key's rank is the
@@ -2529,6 +2600,43 @@ __global__ void __launch_bounds__(256) k_tile_scatter(const int* __restrict__ bu
     const int sh = bshift[key];
     int* o = tile_order + bfirst[key] + ((lbase[key] + lrank) << sh);
     for (int p = 0; p < 1 << sh; ++p) o[p] = tile_item(t, p, sh);
+}
+
+// k_tile_bucket and k_tile_scatter of at most kTileOne tiles in one workgroup
+constexpr int kTileOne = 4096;
+__global__ void __launch_bounds__(1024) k_tile_order(const int* __restrict__ tile_count, int ntiles,
+                                                     int* __restrict__ tile_order, TileSplit sp,
+                                                     int* __restrict__ total) {
+    __shared__ int lh[32], bfirst[32], bshift[32];
+    const int tid = threadIdx.x;
+    if (tid < 32) lh[tid] = 0;
+    __syncthreads();
+    int key[kTileOne / 1024], rank[kTileOne / 1024];
+#pragma unroll
+    for (int e = 0; e < kTileOne / 1024; ++e) {
+        const int t = tid + 1024 * e;
+        const int c = t < ntiles ? tile_count[t] : 0;
+        key[e] = t < ntiles ? 31 - (c == 0 ? 0 : 32 - __clz(c)) : -1;
+        rank[e] = key[e] >= 0 ? atomicAdd(&lh[key[e]], 1) : 0;
+    }
+    __syncthreads();
+    if (tid < 64) {
+        int sh, all;
+        const int f = tile_split(lh, tid, sp, &sh, &all);
+        if (tid < 32) {
+            bfirst[tid] = f;
+            bshift[tid] = sh;
+        }
+        if (tid == 0) *total = all;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < kTileOne / 1024; ++e) {
+        if (key[e] < 0) continue;
+        const int sh = bshift[key[e]];
+        int* o = tile_order + bfirst[key[e]] + (rank[e] << sh);
+        for (int p = 0; p < 1 << sh; ++p) o[p] = tile_item(tid + 1024 * e, p, sh);
+    }
 }
 
 // The heavy-first order of the tiles of every scene of a batch, each scene's
@@ -3984,8 +4092,8 @@ static inline unsigned blocks_for(uint64_t n, unsigned bs) { return (unsigned)((
 
 size_t texel_bytes(int format) { return format == 0 ? 1 : (format == 1 ? 16 : 8); }
 
-void launch_fill_multi(const FillSeg* segs, int nseg, hipStream_t s) {
-    FillArgs a{};
+static uint64_t fill_args(const FillSeg* segs, int nseg, FillArgs& a) {
+    a = FillArgs{};
     uint64_t total = 0;
     int k = 0;
     for (int i = 0; i < nseg && k < 4; ++i) {
@@ -3997,11 +4105,16 @@ void launch_fill_multi(const FillSeg* segs, int nseg, hipStream_t s) {
         ++k;
     }
     a.nseg = k;
-    if (total == 0) return;
     for (int i = k; i < 4; ++i) a.p[i] = a.p[0];  // empty segments (n = 0)
-    unsigned nb = blocks_for(total, 256);
-    if (nb > 65536) nb = 65536;
-    hipLaunchKernelGGL(k_fill_multi, dim3(nb), dim3(256), 0, s, a);
+    return total;
+}
+static unsigned fill_blocks(uint64_t total, unsigned threads) { return std::min(blocks_for(total, threads), 65536u); }
+
+void launch_fill_multi(const FillSeg* segs, int nseg, hipStream_t s) {
+    FillArgs a;
+    const uint64_t total = fill_args(segs, nseg, a);
+    if (total == 0) return;
+    hipLaunchKernelGGL(k_fill_multi, dim3(fill_blocks(total, 256)), dim3(256), 0, s, a);
 }
 
 void launch_fill_u64(uint64_t* p, uint64_t n, uint64_t value, hipStream_t s) {
@@ -4013,16 +4126,29 @@ void launch_fill_u64(uint64_t* p, uint64_t n, uint64_t value, hipStream_t s) {
 
 
 void launch_light_items(const GridDesc& g, const LightView& lv, int mode, const float4* boards, int S,
-                        const LightScratch& ls, hipStream_t s) {
-    if (S <= 0) return;
+                        const LightScratch& ls, const FillSeg* segs, int nseg, hipStream_t s) {
+    if (S <= 0) {
+        launch_fill_multi(segs, nseg, s);
+        return;
+    }
     const int cap = (int)std::min<size_t>(ls.items_cap, 0x7fffffff);
-    const dim3 bgrid((unsigned)((S + 255) / 256));
-    hipLaunchKernelGGL(k_light_boxes, bgrid, dim3(256), 0, s, g, lv, boards, S, ls.lbox, ls.counts, mode == 1 ? 1 : 0);
-    hipLaunchKernelGGL(k_light_scan, dim3(1), dim3(256), 0, s, ls.counts, S, ls.offsets);
-    hipLaunchKernelGGL(k_light_expand, bgrid, dim3(256), 0, s, ls.offsets, S, ls.items, cap);
+    FillArgs fill;
+    const uint64_t total = fill_args(segs, nseg, fill);
+    const unsigned boards_grid = (unsigned)((S + 255) / 256), front = S <= kListOne ? 1 : boards_grid;
+    hipLaunchKernelGGL(k_light_front, dim3(front + fill_blocks(total, 256)), dim3(256), 0, s, g, lv, boards, S, ls.lbox,
+                       ls.counts, ls.offsets, mode == 1 ? 1 : 0, (int)front, fill);
+    if (S > kListOne) {
+        hipLaunchKernelGGL(k_light_scan, dim3(1), dim3(256), 0, s, ls.counts, S, ls.offsets);
+        hipLaunchKernelGGL(k_light_expand, dim3(boards_grid), dim3(256), 0, s, ls.offsets, S, ls.items, cap);
+    }
     const dim3 igrid((unsigned)std::min<size_t>((ls.items_cap + 255) / 256, 2048));
-    hipLaunchKernelGGL(k_light_prep, igrid, dim3(256), 0, s, g, lv, boards, ls.lbox, ls.offsets + S, ls.items, cap,
-                       mode == 1 ? 1 : 0, raster_words(g));
+    const int chord = mode == 1 ? 1 : 0, words = raster_words(g);
+    if (S <= kListOne)
+        hipLaunchKernelGGL(k_light_prep<true>, igrid, dim3(256), 0, s, g, lv, boards, ls.lbox, ls.offsets, S, ls.items,
+                           cap, chord, words);
+    else
+        hipLaunchKernelGGL(k_light_prep<false>, igrid, dim3(256), 0, s, g, lv, boards, ls.lbox, ls.offsets, S, ls.items,
+                           cap, chord, words);
 }
 
 void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const float4* boards, int S,
@@ -4138,10 +4264,28 @@ static int* sort_ranks(unsigned long long* keys, int S) {
 }
 
 void launch_cam_setup(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
-                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, hipStream_t s) {
-    if (S <= 0) return;
-    hipLaunchKernelGGL(k_cam_setup, dim3(blocks_for(S, 256)), dim3(256), 0, s, g, cv, boards, S, sph_world, sph_view,
-                       sph_tiles, keys, sort_ranks(keys, S));
+                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, const FillSeg* segs, int nseg,
+                      hipStream_t s) {
+    if (S <= 0) {
+        launch_fill_multi(segs, nseg, s);
+        return;
+    }
+    FillArgs fill;
+    const uint64_t total = fill_args(segs, nseg, fill);
+    const unsigned front = blocks_for(S, 256);
+    hipLaunchKernelGGL(k_cam_setup, dim3(front + fill_blocks(total, 256)), dim3(256), 0, s, g, cv, boards, S, sph_world,
+                       sph_view, sph_tiles, keys, sort_ranks(keys, S), (int)front, fill);
+}
+
+bool launch_cam_front(const GridDesc& g, const CameraView& cv, const float4* boards, int S, float4* sph_world,
+                      float4* sph_view, int4* sph_tiles, unsigned long long* keys, int32_t* order, int* tie_flag,
+                      bool upload, const FillSeg* segs, int nseg, hipStream_t s) {
+    if (S <= 0 || S > 1024) return false;
+    FillArgs fill;
+    const uint64_t total = fill_args(segs, nseg, fill);
+    hipLaunchKernelGGL(k_cam_front, dim3(1 + fill_blocks(total, 256)), dim3(256), 1024 * sizeof(unsigned long long), s, g,
+                       cv, boards, S, sph_world, sph_view, sph_tiles, keys, order, tie_flag, upload ? 1 : 0, fill);
+    return true;
 }
 
 // Scratch `keys` (sort_scratch_words(S) u64 words): [0, npad) the keys written
@@ -4245,9 +4389,15 @@ void launch_batch_order(const TileBlock* blocks, int nblocks, int nscenes, const
     hipLaunchKernelGGL(k_batch_scatter, dim3(nblocks), dim3(256), 0, s, blocks, bucket_of, hist, cursor, tile_order);
 }
 
+void bin_clear_segs(unsigned long long* masks, int* scratch, int ntiles, int words, FillSeg out[2]) {
+    out[0] = {(uint64_t*)masks, (uint64_t)ntiles * (uint64_t)words, 0};
+    out[1] = {(uint64_t*)scratch, (uint64_t)(66 + ntiles + 1) / 2, 0};
+}
+
 // Binning plus the heavy-first item order.  tile scratch (ints): hist[32] |
 // cursor[32] | item total, 1 unused | tile_count[ntiles] | bucket_of | items.
-// The masks and the scratch up to tile_count are cleared by one fill launch.
+// The caller has cleared bin_clear_segs' ranges: the masks and the scratch up
+// to bucket_of.
 // every_fragment: the composite blends all of a pixel's fragments (a
 // front-to-back one stops after a few, whatever is binned behind them).
 TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int tiles_x, int tiles_y, int words,
@@ -4257,17 +4407,18 @@ TileQueue launch_bin(const int4* sph_tiles, const int32_t* order, int S, int til
     const TileSplit sp = tile_split_rule(ntiles, every_fragment);
     int* tile_count = scratch + 66;
     int* tile_order = tile_count + 2 * (size_t)ntiles;
-    const FillSeg segs[2] = {{(uint64_t*)masks, (uint64_t)ntiles * (uint64_t)words, 0},
-                             {(uint64_t*)scratch, (uint64_t)(66 + ntiles + 1) / 2, 0}};
-    launch_fill_multi(segs, 2, s);
     launch_bin_counts(sph_tiles, order, S, tiles_x, words, masks, tile_count, s);
     int* hist = scratch;
     int* cursor = scratch + 32;
     int* bucket_of = tile_count + ntiles;
-    hipLaunchKernelGGL(k_tile_bucket, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, tile_count, ntiles, bucket_of,
-                       hist);
-    hipLaunchKernelGGL(k_tile_scatter, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, bucket_of, ntiles, hist, cursor,
-                       tile_order, sp, total);
+    if (ntiles <= kTileOne) {
+        hipLaunchKernelGGL(k_tile_order, dim3(1), dim3(1024), 0, s, tile_count, ntiles, tile_order, sp, total);
+    } else {
+        hipLaunchKernelGGL(k_tile_bucket, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, tile_count, ntiles, bucket_of,
+                           hist);
+        hipLaunchKernelGGL(k_tile_scatter, dim3(blocks_for(ntiles, 256)), dim3(256), 0, s, bucket_of, ntiles, hist,
+                           cursor, tile_order, sp, total);
+    }
     return TileQueue{total, tile_order, (unsigned)(ntiles + sp.budget)};
 }
 
@@ -4468,8 +4619,8 @@ __global__ void __launch_bounds__(256) kb_light_expand(const BatchVox* __restric
 __global__ void __launch_bounds__(256) kb_light_prep(const BatchVox* __restrict__ sc, BatchStage st) {
     const StageSlot q = stage_slot(st);
     const BatchVox& B = sc[q.sc];
-    k_light_prep_body(B.g, B.lv, B.boards, B.lbox, B.offsets + B.S, B.items, (int)min(B.items_cap, 0x7fffffff), B.chord,
-                      B.words, q.bid, q.nblk);
+    k_light_prep_body<false>(B.g, B.lv, B.boards, B.lbox, B.offsets, B.S, B.items, (int)min(B.items_cap, 0x7fffffff),
+                             B.chord, B.words, q.bid, q.nblk);
 }
 template <int MODE, int WORDS>
 __global__ void __launch_bounds__(256) kb_light_raster(const BatchVox* __restrict__ sc, BatchStage st) {

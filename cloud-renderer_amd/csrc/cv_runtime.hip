@@ -966,8 +966,7 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
                              {(uint64_t*)shell, (uint64_t)v->nbricks0, 0},
                              {(uint64_t*)fill, (uint64_t)v->nbricks0, 0},
                              {(uint64_t*)counters, counters ? 9u : 0u, 0}};
-    launch_fill_multi(segs, 4, ls);
-    launch_light_items(v->g, plan.lv, v->mode, v->d_boards, v->S, plan.ls, ls);
+    launch_light_items(v->g, plan.lv, v->mode, v->d_boards, v->S, plan.ls, segs, 4, ls);
     if (ls != vs) {
         (void)hipEventRecord(v->ev_items, ls);
         (void)hipStreamWaitEvent(vs, v->ev_items, 0);
@@ -1330,12 +1329,20 @@ static int cone_prepare(cr_volume v, const cr_light* light, const cr_camera* cam
     return CR_OK;
 }
 
-// camera setup + draw order (kernels only)
+// camera setup + draw order, and the fill of nseg segments (kernels only)
 // (CR_ORDER_UPLOAD: the billboards are drawn in upload order, nothing sorted)
-static void cone_enqueue_sort(cr_volume v, const ConePlan& plan, StageEvents* ev, hipStream_t s) {
-    launch_cam_setup(v->g, plan.cv, v->d_boards, plan.S, v->d_sph_world, v->d_sph_view, v->d_sph_tiles, v->d_sort, s);
+static void cone_enqueue_sort(cr_volume v, const ConePlan& plan, StageEvents* ev, const FillSeg* segs, int nseg,
+                              hipStream_t s) {
+    const bool upload = v->order_mode == CR_ORDER_UPLOAD;
+    // one launch for all of it, unless its stages are timed apart
+    if (!v->ctx->profiling &&
+        launch_cam_front(v->g, plan.cv, v->d_boards, plan.S, v->d_sph_world, v->d_sph_view, v->d_sph_tiles, v->d_sort,
+                         v->d_order, v->d_tie, upload, segs, nseg, s))
+        return;
+    launch_cam_setup(v->g, plan.cv, v->d_boards, plan.S, v->d_sph_world, v->d_sph_view, v->d_sph_tiles, v->d_sort, segs,
+                     nseg, s);
     if (ev) ev->mark(1);
-    if (v->order_mode == CR_ORDER_UPLOAD) launch_iota(v->d_order, plan.S, s);
+    if (upload) launch_iota(v->d_order, plan.S, s);
     else launch_sort(v->d_sort, plan.S, v->d_order, v->d_tie, s);
     if (ev) ev->mark(2);
 }
@@ -1408,7 +1415,9 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     if ((rc = ev.begin(ctx, cs, 1))) return rc;
     ev.mark(0);
     if (counters) launch_fill_u64((uint64_t*)counters, 9, 0, s);
-    cone_enqueue_sort(v, plan, &ev, cs);
+    FillSeg clear[2];
+    bin_clear_segs(v->d_masks, v->d_tiles, (int)plan.ntiles, plan.words, clear);
+    cone_enqueue_sort(v, plan, &ev, clear, 2, cs);
     TileQueue tq = launch_bin(v->d_sph_tiles, v->d_order, plan.S, plan.cv.tiles_x, plan.cv.tiles_y, plan.words,
                               v->d_masks, v->d_tiles, plan.cd.composite == CR_COMPOSITE_GL_BLEND, cs);
     ev.mark(3);
@@ -2122,8 +2131,8 @@ void batch_enqueue(cr_batch b, const std::vector<VoxPlan>& vp, const std::vector
     for (size_t i = 0; i < n; ++i) {
         cr_volume v = b->items[i].volume;
         if (!b->batched[i]) {
-            cone_enqueue_sort(v, cp[i], nullptr, cs);
-            launch_fill_u64((uint64_t*)v->d_masks, cp[i].nmask, 0, cs);
+            const FillSeg clear{(uint64_t*)v->d_masks, (uint64_t)cp[i].nmask, 0};
+            cone_enqueue_sort(v, cp[i], nullptr, &clear, 1, cs);
             launch_bin_counts(v->d_sph_tiles, v->d_order, cp[i].S, cp[i].cv.tiles_x, cp[i].words, v->d_masks,
                               b->d_counts + t0, cs);
         }
