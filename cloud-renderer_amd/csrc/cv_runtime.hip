@@ -120,6 +120,7 @@ struct cr_volume_s {
     float max_radius = 0.0f;
     float4* d_boards = nullptr;
     int boards_cap = 0;
+    bool boards_on_caller = false;  // passes that read the boards were enqueued on a caller's stream
     // pass 1
     int lw = 0, lh = 0;
     unsigned long long* d_keys = nullptr;
@@ -859,16 +860,26 @@ int cr_volume_set_billboards(cr_volume v, const float* xyz, const float* scales,
         h[j] = make_float4(xyz[3 * j], xyz[3 * j + 1], xyz[3 * j + 2], r);
         maxr = std::max(maxr, r);
     }
-    // pending camera or voxelization passes read the boards
-    if (v->side) CR_HIP(ctx, hipStreamSynchronize(v->side));
-    if (v->vside) CR_HIP(ctx, hipStreamSynchronize(v->vside));
-    if (v->bside) CR_HIP(ctx, hipStreamSynchronize(v->bside));
-    if (v->lside) CR_HIP(ctx, hipStreamSynchronize(v->lside));
+    // pending camera passes, work lists and splats read the boards; the level
+    // build and the cone trace do not
+    CR_HIP(ctx, hipStreamSynchronize(ctx->lside));
+    CR_HIP(ctx, hipStreamSynchronize(ctx->vside));
     size_t cap = (size_t)v->boards_cap;
     rc = ensure(ctx, &v->d_boards, (size_t)std::max(count, 1), &cap);
     if (rc) return rc;
     v->boards_cap = (int)cap;
-    if (count > 0) CR_HIP(ctx, hipMemcpy(v->d_boards, h.data(), (size_t)count * sizeof(float4), hipMemcpyHostToDevice));
+    // A copy on the null stream waits for the cone trace a caller enqueued there,
+    // so a frame with new billboards had nothing of the next one beside it (the
+    // application frame 570 us, now 488); it is needed only after passes
+    // on a caller's stream (one occupancy set, batches).
+    const size_t bytes = (size_t)count * sizeof(float4);
+    if (count > 0 && v->boards_on_caller) {
+        CR_HIP(ctx, hipMemcpy(v->d_boards, h.data(), bytes, hipMemcpyHostToDevice));
+    } else if (count > 0) {
+        CR_HIP(ctx, hipMemcpyAsync(v->d_boards, h.data(), bytes, hipMemcpyHostToDevice, ctx->lside));
+        CR_HIP(ctx, hipStreamSynchronize(ctx->lside));
+    }
+    v->boards_on_caller = false;
     v->S = count;
     v->max_radius = maxr;
     v->sorted_count = -1;
@@ -1081,6 +1092,7 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
         v->d_fill = v->d_fill_s[nxt];
     } else {
         v->s_sync_needed = true;
+        v->boards_on_caller = true;
     }
     CR_HIP(ctx, hipGetLastError());
     if (ctx->profiling == 1) {
@@ -2340,6 +2352,7 @@ int cr_batch_run(cr_batch b, void* stream) {
         cr_volume v = it.volume;
         v->cam_sync_needed = true;  // its next camera pass follows this run
         v->s_sync_needed = true;  // its next voxelization follows this run
+        v->boards_on_caller = true;
         if (v->cur != 0) {  // the batch's sets (0) become current
             CR_HIP(ctx, hipEventRecord(v->ev_release[v->cur], s));
             v->release_valid[v->cur] = true;

@@ -29,3 +29,36 @@ def test_frame(cv, gpu_ctx, S, W, H, light, fmt):
     g = run_gpu(cv, sc, ctx=gpu_ctx, read_levels=False)
     assert np.array_equal(g.state, o.vox.state())
     assert_bit_equal("image", g.image, o.img32)
+
+
+@pytest.mark.parametrize("own_stream", [False, True])
+def test_uploads_between_frames(cv, gpu_ctx, own_stream):
+    """New billboards for every frame, nothing waited for in between: each
+    image is the one of its own billboards."""
+    import torch
+
+    log(f"[launches] uploads between frames, own stream {own_stream}")
+    base = cv.scenes.small32(3)
+    sets = []
+    for q in range(5):
+        rng = np.random.default_rng(q)
+        S = (300, 7, 1500, 300, 64)[q]
+        sets.append((rng.uniform(-0.7, 0.7, size=(S, 3)).astype(np.float32),
+                     rng.uniform(0.02, 0.2, size=S).astype(np.float32)))
+    want = [run_oracle(replace(base, xyz=x, scales=r), want_f64=False).img32 for x, r in sets]
+    vol, sun, cam, vox, tr = cv.scene_objects(base, 0, context=gpu_ctx)
+    try:
+        for _ in range(2):
+            imgs = [torch.zeros((base.H, base.W, 4), dtype=torch.float32, device="cuda") for _ in sets]
+            stream = torch.cuda.Stream() if own_stream else torch.cuda.current_stream()
+            stream.wait_stream(torch.cuda.current_stream())
+            for (x, r), img in zip(sets, imgs):
+                vol.billboards.positions, vol.billboards.scales = x, r
+                vol.update()
+                vox.voxelize(vol, sun, stream=stream)
+                tr.coneTrace(vol, sun, cam, img, base.W, base.H, stream=stream)
+            torch.cuda.synchronize()
+            for q, img in enumerate(imgs):
+                assert_bit_equal(f"image {q}", img.cpu().numpy(), want[q])
+    finally:
+        vol.close()
