@@ -169,17 +169,26 @@ size_t light_items_bound(int S, float max_radius, const LightView& lv, const Gri
 
 // How the raster kernel walks the chords (cv_kernels.hip: k_light_raster_body)
 constexpr int kRasterGeneral = 0, kRasterPow2 = 1, kRasterQueue = 2;
-// LDS bitmap words of the raster kernel for this grid (its WORDS)
+// LDS bitmap words of the raster kernel for this grid (its WORDS).  The kernel
+// waits on its barriers and LDS as much as it issues, so what counts is how
+// many workgroups fit a CU beside the 17 KB of their queues: 5 with 1792 words,
+// 4 with 2816.  us alone, words 4096 / 2816 / 2304 / 1792 / 1216: 512^3 with
+// 16384 billboards 1100 / 970 / 1005 / 931 / 1046, 256^3 with 4096 billboards
+// (2048 words: 187) - / - / - / 175 / 164, a batch's 96^3 and 192^3 scenes
+// (2048: 537) - / - / - / 462 / 460.  Below 1792 the depth slices that small
+// bitmaps need eat the gain on most sizes; above 256^3 four large workgroups
+// leave more to the cone trace beside them (frame 1800 / 1600 / - / 1634 / 1699).
+constexpr int kRasterWords = 1792, kRasterWordsBig = 2816, kRasterWordsGeneral = 4096;
 __host__ __device__ inline int raster_words(const GridDesc& g) {
-    return g.pow2_range && g.nb0 <= 64 ? 2048 : 4096;
+    return !g.pow2_range ? kRasterWordsGeneral : g.nb0 <= 64 ? kRasterWords : kRasterWordsBig;
 }
 // The chord walk of a pass-1 item runs from the queue (the flat walk) when the
 // grid has power-of-two world extents and the chord fill is on.
 __host__ __device__ inline bool raster_flat(const GridDesc& g, int chord) { return chord && g.pow2_range; }
-// Raster kernel of a grid: 0, 1 kRasterPow2, 2, 3 kRasterQueue (each with 2048,
-// 4096 bitmap words), 4 kRasterGeneral with 4096
+// Raster kernel of a grid: 0, 1 kRasterPow2, 2, 3 kRasterQueue (each with
+// kRasterWords, kRasterWordsBig), 4 kRasterGeneral
 inline int raster_variant(const GridDesc& g, int chord) {
-    const int big = raster_words(g) == 2048 ? 0 : 1;
+    const int big = raster_words(g) == kRasterWords ? 0 : 1;
     if (g.pow2_range && g.pow2_N && g.pow2_step) return big;
     return raster_flat(g, chord) ? 2 + big : 4;
 }

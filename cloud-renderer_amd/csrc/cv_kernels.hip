@@ -4163,11 +4163,11 @@ void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const
                            fillbits, counters);
     };
     switch (raster_variant(g, chord)) {
-        case 0: go(k_light_raster<kRasterPow2, 2048>); break;
-        case 1: go(k_light_raster<kRasterPow2, 4096>); break;
-        case 2: go(k_light_raster<kRasterQueue, 2048>); break;
-        case 3: go(k_light_raster<kRasterQueue, 4096>); break;
-        default: go(k_light_raster<kRasterGeneral, 4096>);
+        case 0: go(k_light_raster<kRasterPow2, kRasterWords>); break;
+        case 1: go(k_light_raster<kRasterPow2, kRasterWordsBig>); break;
+        case 2: go(k_light_raster<kRasterQueue, kRasterWords>); break;
+        case 3: go(k_light_raster<kRasterQueue, kRasterWordsBig>); break;
+        default: go(k_light_raster<kRasterGeneral, kRasterWordsGeneral>);
     }
 }
 
@@ -4755,11 +4755,11 @@ void launch_batch_stage(int stage, int variant, const BatchVox* scenes, const Ba
         case kBsExpand: hipLaunchKernelGGL(kb_light_expand, grid, dim3(256), 0, s, scenes, st); break;
         case kBsPrep: hipLaunchKernelGGL(kb_light_prep, grid, dim3(256), 0, s, scenes, st); break;
         case kBsRaster:
-            if (variant == 0) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, 2048>), grid, dim3(256), 0, s, scenes, st);
-            else if (variant == 1) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, 4096>), grid, dim3(256), 0, s, scenes, st);
-            else if (variant == 2) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, 2048>), grid, dim3(256), 0, s, scenes, st);
-            else if (variant == 3) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, 4096>), grid, dim3(256), 0, s, scenes, st);
-            else hipLaunchKernelGGL((kb_light_raster<kRasterGeneral, 4096>), grid, dim3(256), 0, s, scenes, st);
+            if (variant == 0) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, kRasterWords>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 1) hipLaunchKernelGGL((kb_light_raster<kRasterPow2, kRasterWordsBig>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 2) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, kRasterWords>), grid, dim3(256), 0, s, scenes, st);
+            else if (variant == 3) hipLaunchKernelGGL((kb_light_raster<kRasterQueue, kRasterWordsBig>), grid, dim3(256), 0, s, scenes, st);
+            else hipLaunchKernelGGL((kb_light_raster<kRasterGeneral, kRasterWordsGeneral>), grid, dim3(256), 0, s, scenes, st);
             break;
         case kBsSplat: hipLaunchKernelGGL(kb_light_splat, grid, dim3(256), 0, s, scenes, st); break;
         case kBsBuild:
