@@ -3774,9 +3774,10 @@ __device__ void build_cone_tabs(const VolumeDesc& vd, const ConeTab& t, uint32_t
 // workgroup share the LDS tables of every level (built once per
 // workgroup); wave w of workgroup b shades item b * wpg + w.
 // Dynamic LDS: the tables (t.words words), then per wave the gather lists
-// (kConeChunk coverage masks and ids).
-template <int FMT, int COMP>
-__global__ void __launch_bounds__(512, 6) k_cone_tab(GridDesc g, VolumeDesc vd, CameraView cv, ConeDesc cd, ConeTab t,
+// (kConeChunk coverage masks and ids).  WAVES: waves per SIMD to make room for;
+// RGBA32F spills 7 registers at 6.
+template <int FMT, int COMP, int WAVES>
+__global__ void __launch_bounds__(512, WAVES) k_cone_tab(GridDesc g, VolumeDesc vd, CameraView cv, ConeDesc cd, ConeTab t,
                                                      const void* __restrict__ vol,
                                                      const float4* __restrict__ sph_world,
                                                      const float4* __restrict__ sph_view,
@@ -4360,10 +4361,11 @@ int launch_sort(unsigned long long* keys, int S, int32_t* order, int* tie_flag, 
 //     alone; the frame among others 379 us whole, 387 in halves);
 //   * GL blending marches every fragment, so a tile costs what is binned into
 //     it, and the heaviest (a clump's centre) were the tail: cut by weight.
+constexpr int kFewTiles = 8192;
 static TileSplit tile_split_rule(int ntiles, bool every_fragment) {
     TileSplit sp;
     sp.inv_slots = 1.0f / 12288.0f;  // two rounds of the 6144 waves that fit the device
-    sp.fixed = every_fragment ? -1 : ntiles <= 8192 ? 2 : ntiles <= 16384 ? 1 : 0;
+    sp.fixed = every_fragment ? -1 : ntiles <= kFewTiles ? 2 : ntiles <= 16384 ? 1 : 0;
     sp.budget = every_fragment ? std::max(ntiles, 16384) : ntiles * ((1 << sp.fixed) - 1);
     return sp;
 }
@@ -4489,9 +4491,16 @@ static void launch_cone_t(const ConeLaunch& a, hipStream_t s) {
         ConeTab t;
         if (!a.nmap && a.table_addressing && cone_tab_plan(a.vd, t)) {
             const unsigned grid = (nitems + (unsigned)t.wpg - 1u) / (unsigned)t.wpg;
-            hipLaunchKernelGGL((k_cone_tab<FMT, COMP>), dim3(grid), dim3(64 * t.wpg), cone_tab_lds_bytes(t), s, a.g,
-                               a.vd, a.cv, a.cd, t, a.levels, a.sph_world, a.sph_view, a.order, a.masks, a.words,
-                               a.image, a.counters, a.items);
+            auto go = [&](auto kernel) {
+                hipLaunchKernelGGL(kernel, dim3(grid), dim3(64 * t.wpg), cone_tab_lds_bytes(t), s, a.g, a.vd, a.cv,
+                                   a.cd, t, a.levels, a.sph_world, a.sph_view, a.order, a.masks, a.words, a.image,
+                                   a.counters, a.items);
+            };
+            // small images do not fill the device for long: the shorter steps of
+            // the unspilled kernel count for more than a sixth wave (four 640 x
+            // 360 views 488 -> 473 us, a 1920 x 1080 frame 335 -> 340)
+            if (FMT == 1 && a.cv.tiles_x * a.cv.tiles_y <= kFewTiles) go(k_cone_tab<FMT, COMP, FMT == 1 ? 5 : 6>);
+            else go(k_cone_tab<FMT, COMP, 6>);
             return;
         }
     }
