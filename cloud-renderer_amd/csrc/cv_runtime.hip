@@ -140,6 +140,7 @@ struct cr_volume_s {
     hipStream_t lside = nullptr;  // the context's, once used
     hipEvent_t ev_items = nullptr;
     hipEvent_t ev_lfree[2] = {nullptr, nullptr};
+    bool chained = false;  // the last overlapped voxelization ran on lside alone (small_frame)
     bool lfree_valid[2] = {false, false};
     // camera pass
     float4* d_sph_world = nullptr;
@@ -190,11 +191,11 @@ struct cr_volume_s {
     // overlapping the cone trace that reads the current set; the level build
     // follows on the context's bside after the splat (ev_splat), into the
     // level set that is not current, and the caller's stream waits for it
-    // (ev_built).  ev_bfree[i]: the end of the last build that read occupancy
+    // (ev_bfree).  ev_bfree[i]: the end of the last build that read occupancy
     // set i.  ev_sync orders the side streams after the caller's stream when
     // s_sync_needed (first call, after a serial call or a batch).
     hipStream_t vside = nullptr, bside = nullptr;
-    hipEvent_t ev_splat = nullptr, ev_built = nullptr, ev_sync = nullptr;
+    hipEvent_t ev_splat = nullptr, ev_sync = nullptr;
     hipEvent_t ev_bfree[2] = {nullptr, nullptr};
     bool bfree_valid[2] = {false, false};
     bool s_sync_needed = true;
@@ -663,7 +664,7 @@ int cr_volume_destroy(cr_volume v) {
     if (v->ctx) (void)hipSetDevice(v->ctx->device);
     for (hipStream_t st : {v->side, v->vside, v->bside, v->lside})  // the context's streams: drain, keep
         if (st) (void)hipStreamSynchronize(st);
-    for (hipEvent_t e : {v->ev_cam, v->ev_csync, v->ev_cfree[0], v->ev_cfree[1], v->ev_splat, v->ev_built, v->ev_sync, v->ev_release[0],
+    for (hipEvent_t e : {v->ev_cam, v->ev_csync, v->ev_cfree[0], v->ev_cfree[1], v->ev_splat, v->ev_sync, v->ev_release[0],
                          v->ev_release[1], v->ev_bfree[0], v->ev_bfree[1], v->ev_items, v->ev_lfree[0],
                          v->ev_lfree[1]})
         if (e) (void)hipEventDestroy(e);
@@ -1002,6 +1003,16 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
     if (ev) ev->mark_on(4, bs);
 }
 
+// A frame whose kernels take a few us each is bound by the host, and most of
+// the host's time is events (3 us to record one, 4 to wait for one) that order
+// the three side streams: its passes follow one another on one of them
+// (a 32^3, 256 x 256 frame of 64 billboards 111 -> 84 us, 40^3 137 -> 94).
+// Larger frames run theirs beside the next frame's: 96^3 with 818 billboards
+// and 1426 x 542 pixels took 192 us as a chain, 140 on three streams.
+static bool small_frame(cr_volume v, const VoxPlan& plan) {
+    return v->S <= 1024 && v->N <= 96 && plan.npx <= (size_t)1 << 18 && plan.nitems <= 4096;
+}
+
 int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, void* stream) {
     VoxPlan plan;
     int rc = voxelize_prepare(v, light, light_w, light_h, plan);
@@ -1024,7 +1035,7 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
             v->vside = ctx->vside;
             v->bside = ctx->bside;
             v->lside = ctx->lside;
-            for (hipEvent_t* e : {&v->ev_splat, &v->ev_built, &v->ev_sync, &v->ev_release[0], &v->ev_release[1],
+            for (hipEvent_t* e : {&v->ev_splat, &v->ev_sync, &v->ev_release[0], &v->ev_release[1],
                                   &v->ev_bfree[0], &v->ev_bfree[1], &v->ev_items, &v->ev_lfree[0], &v->ev_lfree[1]})
                 CR_HIP(ctx, hipEventCreateWithFlags(e, hipEventDisableTiming));
         }
@@ -1054,7 +1065,8 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
     }
     const bool two = overlap && v->d_lset[1] != nullptr;
     const int nxt = two ? v->cur ^ 1 : v->cur;
-    hipStream_t vs = two ? v->vside : s, bs = two ? v->bside : s, ls = two ? v->lside : s;
+    const bool chain = two && small_frame(v, plan);
+    hipStream_t ls = two ? v->lside : s, vs = two && !chain ? v->vside : ls, bs = two && !chain ? v->bside : ls;
     // the work list goes into the pair the previous voxelization did not use
     if (two) swap_light(v);
     if ((rc = light_scratch(v, plan))) {
@@ -1069,23 +1081,30 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
         }
     }
     // the clear waits for the passes that last read its key pair and the
-    // build that last read its occupancy set
-    const hipEvent_t lwaits[2] = {two && v->lfree_valid[v->lset_i] ? v->ev_lfree[v->lset_i] : nullptr,
-                                  two && v->bfree_valid[nxt] ? v->ev_bfree[nxt] : nullptr};
+    // build that last read its occupancy set (a chain follows them on its
+    // stream, and the last passes of another kind of frame here; those of a
+    // chain precede whatever waits for this frame's work list)
+    if (chain && !v->chained)
+        for (hipStream_t st : {v->vside, v->bside}) {
+            CR_HIP(ctx, hipEventRecord(v->ev_sync, st));
+            CR_HIP(ctx, hipStreamWaitEvent(ls, v->ev_sync, 0));
+        }
+    v->chained = chain;
+    const hipEvent_t lwaits[2] = {two && !chain && v->lfree_valid[v->lset_i] ? v->ev_lfree[v->lset_i] : nullptr,
+                                  two && !chain && v->bfree_valid[nxt] ? v->ev_bfree[nxt] : nullptr};
     StageEvents ev;
     if ((rc = ev.begin(ctx, vs, 0))) return rc;
     voxelize_enqueue(v, plan, counters, &ev, ls, lwaits, vs, bs, nxt,
                      two && v->release_valid[nxt] ? v->ev_release[nxt] : nullptr);
     ev.end();
-    if (two) v->lfree_valid[v->lset_i] = true;
+    if (two && !chain) v->lfree_valid[v->lset_i] = true;
     if (two) {
         CR_HIP(ctx, hipEventRecord(v->ev_bfree[nxt], bs));
         v->bfree_valid[nxt] = true;
         // what was enqueued on s so far may read the current level set
         CR_HIP(ctx, hipEventRecord(v->ev_release[v->cur], s));
         v->release_valid[v->cur] = true;
-        CR_HIP(ctx, hipEventRecord(v->ev_built, bs));
-        CR_HIP(ctx, hipStreamWaitEvent(s, v->ev_built, 0));
+        CR_HIP(ctx, hipStreamWaitEvent(s, v->ev_bfree[nxt], 0));
         v->cur = nxt;
         v->d_levels = v->d_lset[nxt];
         v->d_shell = v->d_shell_s[nxt];

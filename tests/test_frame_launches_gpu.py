@@ -62,3 +62,32 @@ def test_uploads_between_frames(cv, gpu_ctx, own_stream):
                 assert_bit_equal(f"image {q}", img.cpu().numpy(), want[q])
     finally:
         vol.close()
+
+
+def test_alternating_light_sizes(cv, gpu_ctx):
+    """Frames of one volume that change between one side stream and three (the
+    light image's size decides): each image is the one of its own light image."""
+    import torch
+
+    log("[launches] one and three side streams in turn")
+    base = cv.scenes.small32(9)
+    sizes = [256, 1024, 256, 256, 1024, 1024, 256, 1024]
+    want = {n: run_oracle(replace(base, light_w=n, light_h=n), want_f64=False).img32 for n in set(sizes)}
+    vol, _, cam, vox, tr = cv.scene_objects(base, 0, context=gpu_ctx)
+    try:
+        suns, imgs = [], []
+        for n in sizes:
+            _, sun, _, vox_n, _ = cv.scene_objects(replace(base, light_w=n, light_h=n), 0, context=gpu_ctx)
+            img = torch.zeros((base.H, base.W, 4), dtype=torch.float32, device="cuda")
+            suns.append((sun, vox_n))
+            imgs.append(img)
+        torch.cuda.synchronize()
+        for _ in range(2):
+            for (sun, vox_n), img in zip(suns, imgs):
+                vox_n.voxelize(vol, sun, stream=torch.cuda.current_stream())
+                tr.coneTrace(vol, sun, cam, img, base.W, base.H)
+            torch.cuda.synchronize()
+            for n, img in zip(sizes, imgs):
+                assert_bit_equal(f"light {n}", img.cpu().numpy(), want[n])
+    finally:
+        vol.close()
