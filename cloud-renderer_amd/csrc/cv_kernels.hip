@@ -3709,10 +3709,17 @@ __device__ __forceinline__ void cone_tile(const GridDesc& g, const VolumeDesc& v
     }
 }
 
-// The learned variant asks for 3 waves per SIMD: the inline MLP needs ~100
-// registers beside the march state, and without the bound the kernel gets 2.
+// Waves per SIMD to make room for.  The learned variant asks for 3: the inline
+// MLP needs ~100 registers beside the march state, and without the bound the
+// kernel gets 2 (frame of plain256 689 us; 2: 785, 4: 767).  The footprint
+// slots of R8 volumes are one dependent load a sample, which more waves hide:
+// weighted plain256 1163 / 1123 / 1055 us a frame at 6 / 7 / 8, the application's
+// noise march 479 / 445 / 465 at 4 / 5 / 6.
+constexpr int cone_waves(int fmt, int learned, int nm) {
+    return learned ? 3 : fmt == 3 ? (nm ? 5 : 8) : nm ? 4 : 6;
+}
 template <int FMT, int CONE, int COMP, int LEARNED, int NM>
-__global__ void __launch_bounds__(64, LEARNED ? 3 : (NM ? 4 : 6)) k_cone(GridDesc g, VolumeDesc vd, CameraView cv, ConeDesc cd,
+__global__ void __launch_bounds__(64, cone_waves(FMT, LEARNED, NM)) k_cone(GridDesc g, VolumeDesc vd, CameraView cv, ConeDesc cd,
                                              const void* __restrict__ vol, const float4* __restrict__ sph_world,
                                              const float4* __restrict__ sph_view, const int32_t* __restrict__ order,
                                              const unsigned long long* __restrict__ masks, int words,
