@@ -310,10 +310,9 @@ __device__ __forceinline__ int light_box(const GridDesc& g, const LightView& lv,
 constexpr int kListOne = 1024;  // k_light_front
 // The pass-1 work list: every billboard's pixel box (lbox) and tile count,
 // the exclusive scan of the counts (offsets[S] = the uncut item count) and
-// the (billboard, tile) items in billboard order, cut at cap.  Three small
-// kernels (256-thread workgroups): they find room on CUs that the cone trace
-// of the previous frame keeps busy, where one 1024-thread workgroup waited
-// for a whole CU to drain.
+// the (billboard, tile) items in billboard order, cut at cap.  Workgroups of
+// 256 threads: they find room on CUs that the cone trace of the previous frame
+// keeps busy, where one 1024-thread workgroup waited for a whole CU to drain.
 __device__ __forceinline__ void k_light_boxes_body(GridDesc g, LightView lv, const float4* __restrict__ boards,
                                                      int S, int4* __restrict__ lbox, int* __restrict__ counts, int chord,
                                                      int bid, int nblk) {
