@@ -196,8 +196,8 @@ inline int raster_variant(const GridDesc& g, int chord) {
 // K <= 32 for which the brick box of a full tile's chord slab cut into K
 // equal depth ranges fits the raster's LDS bitmap (a bound of the box
 // slab_box computes: extent + 2 voxels of margin, +2 bricks of alignment);
-// 1 when the chords are long enough that a slice's first sample index
-// would not fit 16 bits.  Slices of one tile are separate work items.
+// 1 for chords of kSliceSamples steps or more (kSliceSamplesSum where the
+// counter accumulates).  Slices of one tile are separate work items.
 __host__ __device__ inline int light_slices_box(const GridDesc& g, const LightView& lv, float s, int words) {
     if (!(s > 0.0f)) return 1;
     const float wu = fminf((float)kLightTile * (2.0f * lv.lsx / (float)lv.W), 2.0f * s);
@@ -216,8 +216,15 @@ __host__ __device__ inline int light_slices_box(const GridDesc& g, const LightVi
     }
     return 32;
 }
+// A slice's first sample index and its count share a word, 16 bits each.  An
+// accumulated counter (steps that are no power of two) drifts from k * stepSize
+// by up to k^2 / 2^25 steps, more than a slice's margins from some thousand
+// steps on, and every slice counts up to its first sample: such chords, which
+// leave any volume but the most elongated, are walked whole.
+constexpr float kSliceSamples = 65535.0f, kSliceSamplesSum = 4096.0f;
 __host__ __device__ inline int light_slices(const GridDesc& g, const LightView& lv, float s, int words) {
-    if (2.0f * s / g.stepSize >= 65535.0f) return 1;
+    const bool exact = g.pow2_N && g.pow2_step;
+    if (2.0f * s / g.stepSize >= (exact ? kSliceSamples : kSliceSamplesSum)) return 1;
     return light_slices_box(g, lv, s, words);  // non-decreasing in s: the work-list bound takes the largest s
 }
 // the pass-1 work list (boxes, scan, items; launch_light_raster reads it) and

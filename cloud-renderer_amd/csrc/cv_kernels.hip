@@ -556,7 +556,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
     constexpr int kRounds = kTilePixels / kRasterThreads;
     __shared__ unsigned long long lbits[WORDS];
     __shared__ float f_sx[kTilePixels], f_sy[kTilePixels], f_sz[kTilePixels];
-    __shared__ int f_n[kTilePixels];
+    __shared__ uint32_t f_n[kTilePixels];
     __shared__ float h_x[kLightTile], h_y[kLightTile];  // the tile's pixel centres on the view plane
     __shared__ int nfr_s;
     __shared__ int q_start[128];  // chord-length buckets: counts, then first queue slots
@@ -724,7 +724,7 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
                 const int slot = q_start[min(q_n[r], 127)] + q_rank[r];
                 f_sx[slot] = q_sx[r]; f_sy[slot] = q_sy[r]; f_sz[slot] = q_sz[r];
                 // sliced items: first sample index above the count (both < 2^16, light_slices)
-                f_n[slot] = nsl > 1 ? (q_k0[r] << 16) | q_n[r] : q_n[r];
+                f_n[slot] = nsl > 1 ? (uint32_t)q_k0[r] << 16 | (uint32_t)q_n[r] : (uint32_t)q_n[r];
             }
         }
         __syncthreads();
@@ -760,9 +760,9 @@ __device__ __forceinline__ void k_light_raster_body(GridDesc g, LightView lv, in
             // is active, and the inner walk's trip count is wave-uniform
             const int f = min(f0 + (tid & 63), nfr - 1);
             const float sx = f_sx[f], sy = f_sy[f], sz = f_sz[f];
-            const int fn_ = f_n[f];
-            const int n = nsl > 1 ? (fn_ & 0xffff) : fn_;  // samples k0 .. k0 + n - 1 of the chord
-            const int k0 = nsl > 1 ? (fn_ >> 16) : 0;
+            const uint32_t fn_ = f_n[f];
+            const int n = (int)(nsl > 1 ? fn_ & 0xffffu : fn_);  // samples k0 .. k0 + n - 1 of the chord
+            const int k0 = nsl > 1 ? (int)(fn_ >> 16) : 0;
             float i0 = (float)k0 * step;  // exact with a power-of-two step
             if constexpr (MODE == kRasterQueue) {
                 i0 = 0.0f;
