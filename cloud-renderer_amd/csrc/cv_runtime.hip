@@ -15,6 +15,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
 #include <new>
 #include <string>
@@ -49,6 +50,24 @@ struct cr_context_s {
     struct Pending { int kind; size_t base; };  // kind 0 voxelize, 1 cone trace
     std::vector<Pending> pending;
 };
+
+// Marks the end of passes on a caller's stream that read billboards; a batch and
+// the volumes that wait for it share one, in whatever order they are destroyed.
+struct CallerMark {
+    hipEvent_t e = nullptr;
+    ~CallerMark() {
+        if (e) (void)hipEventDestroy(e);
+    }
+};
+static std::shared_ptr<CallerMark> caller_mark() {  // null: no memory or no event
+    try {
+        auto m = std::make_shared<CallerMark>();
+        if (hipEventCreateWithFlags(&m->e, hipEventDisableTiming) == hipSuccess) return m;
+        m->e = nullptr;
+    } catch (const std::bad_alloc&) {
+    }
+    return nullptr;
+}
 
 // pass-1 work-list buffers of one voxelization
 struct LightBufs {
@@ -120,7 +139,10 @@ struct cr_volume_s {
     float max_radius = 0.0f;
     float4* d_boards = nullptr;
     int boards_cap = 0;
-    bool boards_on_caller = false;  // passes that read the boards were enqueued on a caller's stream
+    // the last passes on a caller's stream that read the boards (one occupancy
+    // set, batches), until an upload has waited for them; own_mark: the
+    // volume's own, for its one-set voxelizations
+    std::shared_ptr<CallerMark> boards_mark, own_mark;
     // pass 1
     int lw = 0, lh = 0;
     unsigned long long* d_keys = nullptr;
@@ -871,16 +893,16 @@ int cr_volume_set_billboards(cr_volume v, const float* xyz, const float* scales,
     v->boards_cap = (int)cap;
     // A copy on the null stream waits for the cone trace a caller enqueued there,
     // so a frame with new billboards had nothing of the next one beside it (the
-    // application frame 570 us, now 488); it is needed only after passes
-    // on a caller's stream (one occupancy set, batches).
-    const size_t bytes = (size_t)count * sizeof(float4);
-    if (count > 0 && v->boards_on_caller) {
-        CR_HIP(ctx, hipMemcpy(v->d_boards, h.data(), bytes, hipMemcpyHostToDevice));
-    } else if (count > 0) {
-        CR_HIP(ctx, hipMemcpyAsync(v->d_boards, h.data(), bytes, hipMemcpyHostToDevice, ctx->lside));
+    // application frame 570 us, now 488).  On lside it follows the passes of the
+    // volume's own streams, and by their mark those of a caller's stream, of
+    // whatever kind that is.  Without billboards nothing is written.
+    if (count > 0) {
+        if (v->boards_mark) CR_HIP(ctx, hipStreamWaitEvent(ctx->lside, v->boards_mark->e, 0));
+        CR_HIP(ctx, hipMemcpyAsync(v->d_boards, h.data(), (size_t)count * sizeof(float4), hipMemcpyHostToDevice,
+                                   ctx->lside));
         CR_HIP(ctx, hipStreamSynchronize(ctx->lside));
+        v->boards_mark.reset();
     }
-    v->boards_on_caller = false;
     v->S = count;
     v->max_radius = maxr;
     v->sorted_count = -1;
@@ -1064,6 +1086,8 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
         }
     }
     const bool two = overlap && v->d_lset[1] != nullptr;
+    if (!two && !v->own_mark && !(v->own_mark = caller_mark()))
+        return fail(ctx, CR_ENOMEM, "cr_voxelize: no event");
     const int nxt = two ? v->cur ^ 1 : v->cur;
     const bool chain = two && small_frame(v, plan);
     hipStream_t ls = two ? v->lside : s, vs = two && !chain ? v->vside : ls, bs = two && !chain ? v->bside : ls;
@@ -1111,7 +1135,8 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
         v->d_fill = v->d_fill_s[nxt];
     } else {
         v->s_sync_needed = true;
-        v->boards_on_caller = true;
+        CR_HIP(ctx, hipEventRecord(v->own_mark->e, s));
+        v->boards_mark = v->own_mark;
     }
     CR_HIP(ctx, hipGetLastError());
     if (ctx->profiling == 1) {
@@ -1936,6 +1961,7 @@ struct cr_batch_s {
     unsigned long long* d_counters = nullptr;
     hipStream_t cap_stream = nullptr, cap_side = nullptr;  // capture: voxelization, camera passes
     hipEvent_t ev_fork = nullptr, ev_join = nullptr;
+    std::shared_ptr<CallerMark> mark;  // the end of the last run
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
     bool have_graph = false;
@@ -2271,6 +2297,10 @@ int cr_batch_create(cr_context ctx, const cr_batch_item* items, int count, cr_ba
         cr_batch_destroy(b);
         return fail(ctx, CR_EDEVICE, "hipStreamCreate: %s", hipGetErrorString(e));
     }
+    if (!(b->mark = caller_mark())) {
+        cr_batch_destroy(b);
+        return fail(ctx, CR_ENOMEM, "cr_batch_create: no event");
+    }
     // validate every scene once (and allocate its buffers)
     std::vector<VoxPlan> vp;
     std::vector<ConePlan> cp;
@@ -2366,12 +2396,13 @@ int cr_batch_run(cr_batch b, void* stream) {
         if (!graph_current(b) && (rc = batch_capture(b))) return rc;
         CR_HIP(ctx, hipGraphLaunch(b->exec, s));
     }
-    // and the next camera pass and voxelization of a volume wait for this run
+    // and the next camera pass, voxelization and upload of a volume wait for this run
+    CR_HIP(ctx, hipEventRecord(b->mark->e, s));
     for (const auto& it : b->items) {
         cr_volume v = it.volume;
         v->cam_sync_needed = true;  // its next camera pass follows this run
         v->s_sync_needed = true;  // its next voxelization follows this run
-        v->boards_on_caller = true;
+        v->boards_mark = b->mark;
         if (v->cur != 0) {  // the batch's sets (0) become current
             CR_HIP(ctx, hipEventRecord(v->ev_release[v->cur], s));
             v->release_valid[v->cur] = true;
