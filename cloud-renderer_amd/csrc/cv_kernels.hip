@@ -4550,9 +4550,14 @@ void launch_cone(const ConeLaunch& a, hipStream_t s) {
 void launch_segments(const GridDesc& g, const VolumeDesc& vd, const ConeDesc& cd, const void* levels,
                      const float* p0, int n, float* feat, float* tgt, int* valid, hipStream_t s) {
     if (n <= 0) return;
+    // a launch takes fewer than 2^32 threads, kSegLanes of them per start
+    constexpr int kMaxStarts = 1 << 27;
     auto go = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(blocks_for((uint64_t)n * kSegLanes, kSegThreads)), dim3(kSegThreads), 0, s, g,
-                           vd, cd, levels, p0, n, feat, tgt, valid);
+        for (int64_t i = 0; i < n; i += kMaxStarts) {
+            const int m = (int)std::min<int64_t>(kMaxStarts, n - i);
+            hipLaunchKernelGGL(kernel, dim3(blocks_for((uint64_t)m * kSegLanes, kSegThreads)), dim3(kSegThreads), 0, s,
+                               g, vd, cd, levels, p0 + 3 * i, m, feat + i * kMlpIn, tgt + i * kMlpOut, valid + i);
+        }
     };
     if (vd.format == 1)
         cd.compensated ? go(k_segments<1, true>) : go(k_segments<1, false>);
