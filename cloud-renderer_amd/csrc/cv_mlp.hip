@@ -415,8 +415,13 @@ void launch_mlp_pack(const float* master, uint16_t* fwd, uint16_t* bwd, float* b
 
 void launch_mlp_forward(const MlpDev& w, const float* X, int n, float* Y, hipStream_t s) {
     if (n <= 0) return;
-    const int per = 32 * kFwdWaves;
-    hipLaunchKernelGGL(k_mlp_forward, dim3((unsigned)((n + (long long)per - 1) / per)), dim3(64 * kFwdWaves), 0, s, w, X, n, Y);
+    // a launch takes fewer than 2^32 threads, two of them per row
+    constexpr int per = 32 * kFwdWaves, kMaxRows = 1 << 30;
+    for (int64_t i = 0; i < n; i += kMaxRows) {
+        const int m = n - i < kMaxRows ? (int)(n - i) : kMaxRows;
+        hipLaunchKernelGGL(k_mlp_forward, dim3((m + per - 1) / per), dim3(64 * kFwdWaves), 0, s, w, X + i * kMlpIn, m,
+                           Y + i * kMlpOut);
+    }
 }
 
 int mlp_train_groups(int n) { return (n + 63) / 64; }

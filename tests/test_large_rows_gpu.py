@@ -41,3 +41,29 @@ def test_segments(cv, gpu_ctx):
     finally:
         vol.close()
         torch.cuda.empty_cache()
+
+
+def test_forward(cv, gpu_ctx):
+    import torch
+
+    n, edge = (1 << 31) - 100, 3000
+    log(f"[large rows] forward of {n} rows")
+    _need(n * (17 + 5) * 4)
+    g = torch.Generator(device="cuda")
+    g.manual_seed(2)
+    mlp = cv.FarFieldMLP(context=gpu_ctx, params=cv.FarFieldMLP.init_params(3))
+    x = torch.zeros((n, 17), device="cuda")
+    # random rows at both ends and around the middle, zeros between
+    at = [0, (n >> 1) - edge, (1 << 30) - edge // 2, n - edge]
+    for a in at:
+        x[a:a + edge] = torch.rand((edge, 17), generator=g, device="cuda")
+    y = mlp.forward(x)
+    try:
+        for a in at:
+            want = mlp.forward(x[a:a + edge].clone())
+            assert torch.equal(y[a:a + edge].view(torch.int32), want.view(torch.int32)), f"rows from {a}"
+        zero = mlp.forward(torch.zeros((1, 17), device="cuda"))
+        assert torch.equal(y[n // 3:n // 3 + 5], zero.expand(5, -1))
+    finally:
+        del x, y
+        torch.cuda.empty_cache()
