@@ -42,6 +42,7 @@ struct GridDesc {
     int pow2_N;      // N is a power of two: x / N == x * invN exactly
     int pow2_step;   // stepSize is a power of two: the chord counter i += stepSize equals k * stepSize
     float inv_step;  // 1 / stepSize
+    int whole_chords;  // pass-1 chords are not cut into depth slices (no room for the longer work list)
 };
 
 // Light view of pass 1 (Sun::update output + derived billboard basis)
@@ -165,7 +166,17 @@ struct FillSeg {
     uint64_t value;
 };
 void launch_fill_multi(const FillSeg* segs, int nseg, hipStream_t s);  // up to 4 segments, one launch
-size_t light_items_bound(int S, float max_radius, const LightView& lv, const GridDesc& g, int chord);
+// Radii of the billboards: what the length of the pass-1 work list depends on
+struct BoardRadii {
+    float max = 0.0f;
+    double sum = 0.0, sum2 = 0.0;  // over the positive radii
+};
+// At most this many work items: of S billboards with these radii, and (uniform)
+// of S billboards that all have the largest
+struct ItemsBound {
+    size_t items, uniform;
+};
+ItemsBound light_items_bound(int S, const BoardRadii& r, const LightView& lv, const GridDesc& g, int chord);
 
 // How the raster kernel walks the chords (cv_kernels.hip: k_light_raster_body)
 constexpr int kRasterGeneral = 0, kRasterPow2 = 1, kRasterQueue = 2;
@@ -223,6 +234,7 @@ __host__ __device__ inline int light_slices_box(const GridDesc& g, const LightVi
 // leave any volume but the most elongated, are walked whole.
 constexpr float kSliceSamples = 65535.0f, kSliceSamplesSum = 4096.0f;
 __host__ __device__ inline int light_slices(const GridDesc& g, const LightView& lv, float s, int words) {
+    if (g.whole_chords) return 1;
     const bool exact = g.pow2_N && g.pow2_step;
     if (2.0f * s / g.stepSize >= (exact ? kSliceSamples : kSliceSamplesSum)) return 1;
     return light_slices_box(g, lv, s, words);  // non-decreasing in s: the work-list bound takes the largest s

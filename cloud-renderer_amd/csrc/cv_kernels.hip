@@ -4178,16 +4178,22 @@ void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const
     }
 }
 
-size_t light_items_bound(int S, float max_radius, const LightView& lv, const GridDesc& g, int chord) {
+ItemsBound light_items_bound(int S, const BoardRadii& r, const LightView& lv, const GridDesc& g, int chord) {
     // depth slices multiply the items; a billboard's slice count grows with its radius
-    const size_t kmax = raster_flat(g, chord) ? (size_t)light_slices_box(g, lv, max_radius, raster_words(g)) : 1;
-    // widest pixel box of a billboard of radius max_radius: the box spans
-    // s * W / lsx pixels plus at most 5 from floor/ceil and the 1-pixel margins
-    double wx = 2.0 * max_radius * lv.W / (2.0 * lv.lsx) + 6.0;
-    double wy = 2.0 * max_radius * lv.H / (2.0 * lv.lsy) + 6.0;
-    size_t tx = std::min<size_t>((size_t)(wx / kLightTile) + 2, (size_t)(lv.W / kLightTile) + 1);
-    size_t ty = std::min<size_t>((size_t)(wy / kLightTile) + 2, (size_t)(lv.H / kLightTile) + 1);
-    return std::max<size_t>((size_t)S * tx * ty * kmax, 1);
+    const size_t kmax = raster_flat(g, chord) && !g.whole_chords
+                            ? (size_t)light_slices_box(g, lv, r.max, raster_words(g)) : 1;
+    // pixel box of a billboard of radius s: it spans s * W / lsx pixels plus at
+    // most 5 from floor/ceil and the 1-pixel margins, ax s + b tiles across
+    const double ax = lv.W / (lv.lsx * kLightTile), ay = lv.H / (lv.lsy * kLightTile), b = 6.0 / kLightTile + 2.0;
+    size_t tx = std::min<size_t>((size_t)(ax * r.max + b), (size_t)(lv.W / kLightTile) + 1);
+    size_t ty = std::min<size_t>((size_t)(ay * r.max + b), (size_t)(lv.H / kLightTile) + 1);
+    ItemsBound n;
+    n.uniform = std::max<size_t>((size_t)S * tx * ty * kmax, 1);
+    // sum of (ax s + b) (ay s + b): one large billboard among many small ones
+    // counts once, not for all of them
+    const double sum = (ax * ay * r.sum2 + (ax + ay) * b * r.sum + b * b * S) * (double)kmax + 1.0;
+    n.items = sum < (double)n.uniform ? (size_t)sum : n.uniform;
+    return n;
 }
 
 void launch_light_splat(const GridDesc& g, const LightView& lv, const float4* boards, const unsigned long long* keys,

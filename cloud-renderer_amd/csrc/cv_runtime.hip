@@ -136,7 +136,7 @@ struct cr_volume_s {
     unsigned long long* d_fill_s[2] = {nullptr, nullptr};
     uint32_t nbricks0 = 0;
     int S = 0;
-    float max_radius = 0.0f;
+    BoardRadii radii;
     float4* d_boards = nullptr;
     int boards_cap = 0;
     // the last passes on a caller's stream that read the boards (one occupancy
@@ -874,14 +874,16 @@ int cr_volume_set_billboards(cr_volume v, const float* xyz, const float* scales,
     int rc = set_device(ctx);
     if (rc) return rc;
     std::vector<float4> h((size_t)std::max(count, 1));
-    float maxr = 0.0f;
+    BoardRadii radii;
     for (int j = 0; j < count; ++j) {
         // uploadBillboards (src/CloudVolume.cpp:153-160): scale * fluffiness
         float r = fluffiness != 1.0f ? scales[j] * fluffiness : scales[j];
         if (!finite3(xyz + 3 * j) || !std::isfinite(r))
             return fail(ctx, CR_EINVAL, "cr_volume_set_billboards: non-finite position or scale");
         h[j] = make_float4(xyz[3 * j], xyz[3 * j + 1], xyz[3 * j + 2], r);
-        maxr = std::max(maxr, r);
+        radii.max = std::max(radii.max, r);
+        radii.sum += std::max(r, 0.0f);
+        radii.sum2 += (double)std::max(r, 0.0f) * std::max(r, 0.0f);
     }
     // pending camera passes, work lists and splats read the boards; the level
     // build and the cone trace do not
@@ -904,7 +906,7 @@ int cr_volume_set_billboards(cr_volume v, const float* xyz, const float* scales,
         v->boards_mark.reset();
     }
     v->S = count;
-    v->max_radius = maxr;
+    v->radii = radii;
     v->sorted_count = -1;
     v->gen += 1;
     return CR_OK;
@@ -916,7 +918,16 @@ struct VoxPlan {
     LightScratch ls;
     size_t npx;
     size_t nitems;  // work-list capacity
+    size_t uniform;  // ItemsBound::uniform
 };
+
+static void plan_items(cr_volume v, VoxPlan& plan) {
+    plan.nitems = plan.uniform = 0;
+    if (v->S <= 0) return;
+    const ItemsBound n = light_items_bound(v->S, v->radii, plan.lv, v->g, v->mode == CR_MODE_RGBA ? 1 : 0);
+    plan.nitems = n.items;
+    plan.uniform = n.uniform;
+}
 
 static int voxelize_prepare(cr_volume v, const cr_light* light, int light_w, int light_h, VoxPlan& plan) {
     if (!v) return fail(nullptr, CR_EINVAL, "cr_voxelize: vol is NULL");
@@ -933,7 +944,7 @@ static int voxelize_prepare(cr_volume v, const cr_light* light, int light_w, int
     }
     // the chord fill walks 2 * radius in stepSize increments with a float
     // counter; bound it so the walk always advances and terminates
-    if (v->mode == CR_MODE_RGBA && (2.0f * v->max_radius) / v->g.stepSize > 1048576.0f)
+    if (v->mode == CR_MODE_RGBA && (2.0f * v->radii.max) / v->g.stepSize > 1048576.0f)
         return fail(ctx, CR_EUNSUPPORTED, "cr_voxelize: billboard radius exceeds 2^19 voxels (chord fill)");
     int rc = set_device(ctx);
     if (rc) return rc;
@@ -945,7 +956,7 @@ static int voxelize_prepare(cr_volume v, const cr_light* light, int light_w, int
     v->last_lv = plan.lv;  // the position map is rebuilt from the keys on request
     v->vox_gen = v->gen;
     plan.ls = LightScratch{};
-    plan.nitems = v->S > 0 ? light_items_bound(v->S, v->max_radius, plan.lv, v->g, v->mode == CR_MODE_RGBA ? 1 : 0) : 0;
+    plan_items(v, plan);
     return CR_OK;
 }
 
@@ -958,7 +969,20 @@ static int light_scratch(cr_volume v, VoxPlan& plan) {
     if (v->S <= 0) return CR_OK;
     if ((rc = ensure(ctx, &v->d_lbox, (size_t)v->S, &v->lbox_cap))) return rc;
     if ((rc = ensure(ctx, &v->d_lcounts, 2 * (size_t)v->S + 1, &v->lcounts_cap))) return rc;
-    if ((rc = ensure(ctx, &v->d_litems, plan.nitems, &v->litems_cap))) return rc;
+    // Depth slices make the work list up to 32 times as long.  Where it has no
+    // room so (or its indices none in 31 bits), the volume's chords stay whole
+    // from now on; captured batches hold the list's old shape.
+    const bool cut = v->mode == CR_MODE_RGBA && v->g.pow2_range && !v->g.whole_chords;
+    rc = cut && plan.nitems > 0x7fffffff ? CR_ENOMEM : ensure(ctx, &v->d_litems, plan.nitems, &v->litems_cap);
+    if (rc == CR_ENOMEM && cut) {
+        (void)hipGetLastError();
+        v->g.whole_chords = 1;
+        v->gen += 1;
+        v->vox_gen = v->gen;
+        plan_items(v, plan);
+        rc = ensure(ctx, &v->d_litems, plan.nitems, &v->litems_cap);
+    }
+    if (rc) return rc;
     plan.ls.lbox = v->d_lbox;
     plan.ls.counts = v->d_lcounts;
     plan.ls.offsets = v->d_lcounts + v->S;
@@ -1032,7 +1056,7 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
 // Larger frames run theirs beside the next frame's: 96^3 with 818 billboards
 // and 1426 x 542 pixels took 192 us as a chain, 140 on three streams.
 static bool small_frame(cr_volume v, const VoxPlan& plan) {
-    return v->S <= 1024 && v->N <= 96 && plan.npx <= (size_t)1 << 18 && plan.nitems <= 4096;
+    return v->S <= 1024 && v->N <= 96 && plan.npx <= (size_t)1 << 18 && plan.uniform <= 4096;
 }
 
 int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, void* stream) {
