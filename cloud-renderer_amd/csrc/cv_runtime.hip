@@ -121,9 +121,11 @@ struct cr_volume_s {
     size_t ntex_cap = 0;
     size_t zflags_bytes = 0;
     // R8 volumes: per set the cone's footprint slots and the level-0 bricks'
-    // zero flags (null without room for them: the cone samples the texels)
+    // zero flags, from the first cone trace on (foot_prepare; null without room
+    // for them: the cone samples the texels)
     uint2* d_foot[2] = {nullptr, nullptr};
     uint8_t* d_fzero[2] = {nullptr, nullptr};
+    bool foot_tried = false;
     int cur = 0;
     bool lset_failed = false;
     hipEvent_t ev_release[2] = {nullptr, nullptr};
@@ -584,6 +586,25 @@ static void foot_alloc(cr_volume v, int set, hipStream_t s) {
     launch_fill_u64((uint64_t*)v->d_fzero[set], zb / 8, 0x0101010101010101ull, s);
 }
 
+// The first cone trace of an R8 volume makes the footprint slots of its level
+// sets (8 bytes a texel, where the texels themselves take 1), so that volumes
+// which are only voxelized and read back pay nothing for them; later builds
+// renew them.  Only while they leave seven eighths of the free memory: what the
+// slots save is time, and whoever allocates next must not fail for them.
+static void foot_prepare(cr_volume v, hipStream_t s) {
+    if (v->format != CR_FORMAT_R8 || v->foot_tried || (v->ctx->flags & CR_CONTEXT_DIRECT_ADDRESSING)) return;
+    v->foot_tried = true;
+    const size_t bytes = 2 * foot_slots(v->vd) * sizeof(uint2);
+    size_t free_bytes = 0, total = 0;
+    if (hipMemGetInfo(&free_bytes, &total) != hipSuccess) (void)hipGetLastError();
+    if (bytes == 0 || bytes > free_bytes / 8) return;
+    for (int k = 0; k < 2; ++k)
+        if (v->d_lset[k]) foot_alloc(v, k, s);
+    if (v->d_foot[v->cur])
+        launch_foot_r8(v->g, v->vd, v->d_shell, v->d_levels, v->d_foot[v->cur], v->d_fzero[v->cur], s);
+    v->s_sync_needed = true;  // the next build, into the other set, follows the clear of its slots
+}
+
 int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const float bounds_hi[3],
                      const float position[3], int levels, int format, int mode, cr_volume* out) {
     if (!ctx || !out || !bounds_lo || !bounds_hi || !position)
@@ -666,7 +687,6 @@ int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const fl
         return fail(ctx, e == hipErrorOutOfMemory ? CR_ENOMEM : CR_EDEVICE, "cr_volume_create: hipMalloc: %s",
                     hipGetErrorString(e));
     }
-    foot_alloc(v, 0, nullptr);
     // zero the volume so reads before the first voxelize are defined
     launch_fill_u64((uint64_t*)v->d_levels, v->levels_bytes / 8, 0, nullptr);
     if (v->d_zflags[0]) launch_fill_u64((uint64_t*)v->d_zflags[0], v->zflags_bytes / 8, 0x0101010101010101ull, nullptr);
@@ -1104,7 +1124,7 @@ int cr_voxelize(cr_volume v, const cr_light* light, int light_w, int light_h, vo
                 v->d_fill_s[1] = fl;
                 launch_fill_u64((uint64_t*)p, v->levels_bytes / 8, 0, s);
                 if (z) launch_fill_u64((uint64_t*)z, v->zflags_bytes / 8, 0x0101010101010101ull, s);
-                foot_alloc(v, 1, s);
+                if (v->d_foot[0]) foot_alloc(v, 1, s);
                 v->s_sync_needed = true;  // the streams wait for these fills
             }
         }
@@ -1475,6 +1495,7 @@ static int cone_trace_impl(cr_volume v, const cr_light* light, const cr_camera* 
     }
     if (!v->voxelized) return fail(ctx, CR_ESTATE, "cr_cone_trace: volume not voxelized");
     hipStream_t s = (hipStream_t)stream;
+    foot_prepare(v, s);
     unsigned long long* counters = ctx->profiling == 1 ? v->d_counters : nullptr;
     hipStream_t cs = s;
     if (overlap) {

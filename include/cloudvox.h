@@ -156,7 +156,8 @@ typedef struct {
 /* ---- context ---------------------------------------------------------- */
 /* context flags */
 #define CR_CONTEXT_DIRECT_ADDRESSING 1u /* front-to-back cone traces compute every sample's texel addresses
-                                           instead of reading per-level offset tables from LDS (same images) */
+                                           instead of reading per-level offset tables from LDS, and those of
+                                           R8 volumes read the texels instead of footprint slots (same images) */
 int cr_context_create(int device, unsigned flags, cr_context *out);
 int cr_context_destroy(cr_context ctx);
 const char *cr_last_error(cr_context ctx);
