@@ -42,7 +42,7 @@ struct GridDesc {
     int pow2_N;      // N is a power of two: x / N == x * invN exactly
     int pow2_step;   // stepSize is a power of two: the chord counter i += stepSize equals k * stepSize
     float inv_step;  // 1 / stepSize
-    int whole_chords;  // pass-1 chords are not cut into depth slices (no room for the longer work list)
+    float slice_radius;  // billboards from this radius on have their chords walked whole (0: all, no room for more work items)
 };
 
 // Light view of pass 1 (Sun::update output + derived billboard basis)
@@ -231,12 +231,17 @@ __host__ __device__ inline int light_slices_box(const GridDesc& g, const LightVi
 // accumulated counter (steps that are no power of two) drifts from k * stepSize
 // by up to k^2 / 2^25 steps, more than a slice's margins from some thousand
 // steps on, and every slice counts up to its first sample: such chords, which
-// leave any volume but the most elongated, are walked whole.
-constexpr float kSliceSamples = 65535.0f, kSliceSamplesSum = 4096.0f;
+// leave any volume but the most elongated, are walked whole.  The rule is a
+// radius the host computes: with the division and the grid's flags in it,
+// k_light_front took 33 registers, and the 40 that are allotted for them have
+// no room beside the application frame's cone trace (17 -> 300 us, the frame
+// 452 -> 458).
+constexpr float kSliceSamples = 65534.0f, kSliceSamplesSum = 4096.0f;
+inline float slice_radius(const GridDesc& g) {
+    return 0.5f * (g.pow2_N && g.pow2_step ? kSliceSamples : kSliceSamplesSum) * g.stepSize;
+}
 __host__ __device__ inline int light_slices(const GridDesc& g, const LightView& lv, float s, int words) {
-    if (g.whole_chords) return 1;
-    const bool exact = g.pow2_N && g.pow2_step;
-    if (2.0f * s / g.stepSize >= (exact ? kSliceSamples : kSliceSamplesSum)) return 1;
+    if (s >= g.slice_radius) return 1;
     return light_slices_box(g, lv, s, words);  // non-decreasing in s: the work-list bound takes the largest s
 }
 // the pass-1 work list (boxes, scan, items; launch_light_raster reads it) and

@@ -4180,8 +4180,8 @@ void launch_light_raster(const GridDesc& g, const LightView& lv, int mode, const
 
 ItemsBound light_items_bound(int S, const BoardRadii& r, const LightView& lv, const GridDesc& g, int chord) {
     // depth slices multiply the items; a billboard's slice count grows with its radius
-    const size_t kmax = raster_flat(g, chord) && !g.whole_chords
-                            ? (size_t)light_slices_box(g, lv, r.max, raster_words(g)) : 1;
+    const size_t kmax = raster_flat(g, chord)
+                            ? (size_t)light_slices_box(g, lv, std::min(r.max, g.slice_radius), raster_words(g)) : 1;
     // pixel box of a billboard of radius s: it spans s * W / lsx pixels plus at
     // most 5 from floor/ceil and the 1-pixel margins, ax s + b tiles across
     const double ax = lv.W / (lv.lsx * kLightTile), ay = lv.H / (lv.lsy * kLightTile), b = 6.0 / kLightTile + 2.0;

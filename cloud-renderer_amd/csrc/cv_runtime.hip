@@ -668,6 +668,7 @@ int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const fl
     v->g.pow2_N = is_pow2((float)dim) ? 1 : 0;
     v->g.pow2_step = is_pow2(v->g.stepSize) ? 1 : 0;
     v->g.inv_step = 1.0f / v->g.stepSize;
+    v->g.slice_radius = slice_radius(v->g);
     v->g.invN = 1.0f / (float)dim;
     v->g.N = dim;
     v->g.nb0 = v->vd.lv[0].nb;
@@ -992,11 +993,11 @@ static int light_scratch(cr_volume v, VoxPlan& plan) {
     // Depth slices make the work list up to 32 times as long.  Where it has no
     // room so (or its indices none in 31 bits), the volume's chords stay whole
     // from now on; captured batches hold the list's old shape.
-    const bool cut = v->mode == CR_MODE_RGBA && v->g.pow2_range && !v->g.whole_chords;
+    const bool cut = v->mode == CR_MODE_RGBA && v->g.pow2_range && v->g.slice_radius > 0.0f;
     rc = cut && plan.nitems > 0x7fffffff ? CR_ENOMEM : ensure(ctx, &v->d_litems, plan.nitems, &v->litems_cap);
     if (rc == CR_ENOMEM && cut) {
         (void)hipGetLastError();
-        v->g.whole_chords = 1;
+        v->g.slice_radius = 0.0f;
         v->gen += 1;
         v->vox_gen = v->gen;
         plan_items(v, plan);
