@@ -2060,7 +2060,11 @@ __device__ void replay_ties(int S, const I* s_idx, const uint32_t* s_tie, P* pos
 // 0xFFFF = not yet known.  placed: one bit per element.
 constexpr uint32_t kStepElem = 0x3fffu, kStepTie = 0x4000u, kStepRun = 0x8000u, kStepOpen = 0xffff0000u;
 __device__ __forceinline__ int step_D(uint32_t w) { return (int)(w >> 16); }
-__device__ __forceinline__ void step_set_D(uint32_t* w, int t, int d) { ((uint16_t*)(w + t))[1] = (uint16_t)d; }
+// The half word alone is written: other threads read the word's element and
+// flags meanwhile.  A read of D beside the write gives 0xFFFF or the value (any
+// thread that evaluates a step finds the same one).
+typedef uint16_t __attribute__((may_alias)) step_half;
+__device__ __forceinline__ void step_set_D(uint32_t* w, int t, int d) { ((step_half*)(w + t))[1] = (uint16_t)d; }
 __device__ void replay_ties_block(int S, uint32_t* w, uint32_t* placed, int32_t* __restrict__ order) {
     __shared__ int seg_end;
     __shared__ int red_p[16], red_e[16];
