@@ -16,7 +16,6 @@ constexpr int kTile = 8;           // default camera tile: 8x8 pixels = one wave
 constexpr int kLdsSortMax = 16384; // billboards sorted in one workgroup's LDS
 constexpr int kBatchSortMax = 8192; // billboards a batched LDS sort takes (64 KiB of keys)
 constexpr int kFillChunk = 4096;    // elements per workgroup of the segmented fill
-constexpr int kChordLdsWords = 4096; // largest LDS bitmap (bricks) per pass-1 tile for chord-fill aggregation
 constexpr int kLightTile = 32;       // pass-1 work item: 32 x 32 light pixels of one billboard
 
 // One mip level in the bricked layout: 4x4x4 bricks, texels Morton-ordered
@@ -298,8 +297,8 @@ struct TileQueue {
     const int* order;
     unsigned bound;    // the total is at most this (launch size)
 };
-// rule of the cut: 1 / wave slots, extra items allowed, parts of every tile as
-// a shift (or -1: by weight)
+// rule of the cut: 1 / items that share the device (tile_split_rule), extra
+// items allowed, parts of every tile as a shift (or -1: by weight)
 struct TileSplit {
     float inv_slots;
     int budget;

@@ -3783,8 +3783,8 @@ __device__ void build_cone_tabs(const VolumeDesc& vd, const ConeTab& t, uint32_t
 // The front-to-back cone trace with table addressing: t.wpg waves per
 // workgroup share the LDS tables of every level (built once per
 // workgroup); wave w of workgroup b shades item b * wpg + w.
-// Dynamic LDS: the tables (t.words words), then per wave the gather lists
-// (kConeChunk coverage masks and ids).  WAVES: waves per SIMD to make room for;
+// Dynamic LDS: the tables (t.words words), then the waves' candidate lists
+// (ConeLds).  WAVES: waves per SIMD to make room for;
 // RGBA32F spills 7 registers at 6.
 template <int FMT, int COMP, int WAVES>
 __global__ void __launch_bounds__(512, WAVES) k_cone_tab(GridDesc g, VolumeDesc vd, CameraView cv, ConeDesc cd, ConeTab t,
@@ -3824,7 +3824,8 @@ __global__ void __launch_bounds__(512, WAVES) k_cone_tab(GridDesc g, VolumeDesc 
 
 // Batched cone trace: the tiles of many scenes, scene after scene and heavy
 // first in each; a wave finds its item's scene by binary search over the
-// scenes' first items.
+// scenes' first items.  Five waves per SIMD: what the kernel's 91 registers
+// give it anyway (batch of 64 scenes 6404 us, 6411 without a bound).
 template <int FMT, int CONE, int COMP>
 __global__ void __launch_bounds__(256, 5) k_cone_batch(const BatchScene* __restrict__ scenes,
                                                     const int* __restrict__ tile0, int nscenes,
@@ -4370,17 +4371,31 @@ int launch_sort(unsigned long long* keys, int S, int32_t* order, int* tie_flag, 
 //   * front-to-back composites: a pixel stops after a few fragments whatever
 //     is binned behind them, so every tile is cut alike, and only where the
 //     whole tiles leave the device idle: a wave of a 64-pixel tile takes
-//     200 us of dependent steps, which 3600 tiles (640 x 360) do not hide
-//     (plain256's cone: 225 us whole, 142 in halves, 104 in quarters, 115 in
-//     eighths), while at 32 400 tiles the device is full and parts only march
-//     more beyond the pixels' ends (234 whole, 232 in halves, 342 in quarters
-//     alone; the frame among others 379 us whole, 387 in halves);
+//     200 us of dependent steps, which few tiles do not hide, while on a full
+//     device parts only march more beyond the pixels' ends.  us of the cone
+//     trace among others, whole / halves / quarters, by tiles: 256^3 RGBA32F,
+//     4096 billboards: 3600 274 / 181 / 132, 8160 274 / 188 / 163, 9216 286 /
+//     192 / 176, 14 400 287 / 212 / 229, 16 928 306 / 219 / 233, 32 400 340 /
+//     318 / 404; 96^3 RGBA16F, 900 billboards: 3600 90 / 70 / 58, 8160 91 /
+//     73 / 88, 9216 90 / 74 / 92, 14 400 93 / 88 / 120, 16 928 95 / 87 / 124,
+//     32 400 110 / 122 / 214.  The lines lie where the two scenes part.
+//     Weighted cones under this composite follow the same rule.  They march
+//     every step of what is taken in vain, so where nearly every pixel ends at
+//     its first fragment whole tiles with one fragment at a time would be
+//     better (128^3, 100 steps, 1280 x 720: 149 us, 110 before tiles were cut
+//     and lanes shared), elsewhere the cut is (256^3 there 752, 1065 before; 16
+//     steps 152, 267 before): the content decides, which no size tells.
 //   * GL blending marches every fragment, so a tile costs what is binned into
-//     it, and the heaviest (a clump's centre) were the tail: cut by weight.
+//     it, and the heaviest (a clump's centre) were the tail: cut by weight,
+//     against a share of the device that is a tuned number of items, one for
+//     all kernels whatever their waves per SIMD.  us a frame at 3072 / 6144 /
+//     12 288 / 24 576: noise march of the application 451 / 435 / 451 / 529,
+//     blended RGBA16F at 150^3 170 / 176 / 195 / 195, weighted R8 at 256^3 1878 /
+//     1273 / 1144 / 1121.
 constexpr int kFewTiles = 8192;
 static TileSplit tile_split_rule(int ntiles, bool every_fragment) {
     TileSplit sp;
-    sp.inv_slots = 1.0f / 12288.0f;  // two rounds of the 6144 waves that fit the device
+    sp.inv_slots = 1.0f / 12288.0f;
     sp.fixed = every_fragment ? -1 : ntiles <= kFewTiles ? 2 : ntiles <= 16384 ? 1 : 0;
     sp.budget = every_fragment ? std::max(ntiles, 16384) : ntiles * ((1 << sp.fixed) - 1);
     return sp;

@@ -44,7 +44,7 @@ struct cr_context_s {
     std::string err;
     int profiling = 0;
     cr_stats stats{};  // level 1: last call; level 2: sums since the last cr_get_stats
-    // event pool: level 1 reuses the first 10 events, level 2 takes 5 per call
+    // event pool: level 1 reuses the first 12 events, level 2 takes 6 per call
     std::vector<hipEvent_t> pool;
     size_t pool_used = 0;
     struct Pending { int kind; size_t base; };  // kind 0 voxelize, 1 cone trace
@@ -2199,9 +2199,10 @@ int batch_prepare(cr_batch b, std::vector<VoxPlan>& vp, std::vector<ConePlan>& c
 }
 
 // kernels only: voxelize every scene, camera setup / sort / bin every scene,
-// a heavy-first order of every scene's tiles, one batched cone trace.  Scenes the batched stages take: one segmented fill, then
-// one launch per voxelization stage and per camera-pass stage over all of
-// them; the others: their own per-scene launches.  The camera passes (sorts of
+// a heavy-first order of every scene's tiles, one batched cone trace.  Scenes
+// the batched stages take: one segmented fill, then one launch per voxelization
+// stage and per camera-pass stage over all of them; the others: their own
+// per-scene launches.  The camera passes (sorts of
 // one workgroup per scene, binning) need only the billboards and the fill:
 // when cs is another stream than s they run beside the voxelization, from
 // ev_fork to ev_join (300 of the batch's 6900 us for 64 scenes).

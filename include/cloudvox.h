@@ -141,8 +141,9 @@ typedef struct {
 typedef struct {
     int64_t light_fragments; /* covered pass-1 fragments */
     int64_t shell_texels;    /* position-map texels with a > 0 */
-    int64_t fragments;       /* shaded camera fragments */
-    int64_t samples;         /* cone samples taken */
+    int64_t fragments;       /* composited camera fragments */
+    int64_t samples;         /* cone samples of those fragments (a front-to-back pixel's fragments are marched
+                                a few at a time: what is marched beyond its end is in no counter) */
     int64_t two_level;       /* samples that blended two mip levels */
     float ms_clear, ms_light_raster, ms_splat, ms_mip;  /* voxelize stages */
     float ms_setup, ms_sort, ms_bin, ms_cone;           /* cone-trace stages */
@@ -150,7 +151,7 @@ typedef struct {
     int64_t chord_stores;    /* chord-fill voxel stores of pass 1 (rgba mode) */
     int64_t mlp_rows;        /* cones whose far field the MLP predicted (learned trace) */
     int64_t mlp_fallbacks;   /* of those, cones that fell back to the plain march */
-    int64_t mlp_evals;       /* batched MLP evaluations (one per wave and billboard) */
+    int64_t mlp_evals;       /* batched MLP evaluations (one per wave and round of fragments) */
 } cr_stats;
 
 /* ---- context ---------------------------------------------------------- */
