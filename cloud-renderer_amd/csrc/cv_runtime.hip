@@ -602,7 +602,12 @@ static void foot_prepare(cr_volume v, hipStream_t s) {
         if (v->d_lset[k]) foot_alloc(v, k, s);
     if (v->d_foot[v->cur])
         launch_foot_r8(v->g, v->vd, v->d_shell, v->d_levels, v->d_foot[v->cur], v->d_fzero[v->cur], s);
-    v->s_sync_needed = true;  // the next build, into the other set, follows the clear of its slots
+    // the next build, into the other set, follows the clear of its slots, also
+    // where its voxelization is called on another stream than this trace
+    if (v->vside) {
+        (void)hipEventRecord(v->ev_sync, s);
+        for (hipStream_t st : {v->lside, v->bside}) (void)hipStreamWaitEvent(st, v->ev_sync, 0);
+    }
 }
 
 int cr_volume_create(cr_context ctx, int dim, const float bounds_lo[3], const float bounds_hi[3],

@@ -99,3 +99,35 @@ def test_first_trace_between_frames(cv, gpu_ctx, before):
             assert_bit_equal(f"frame {f}", img.cpu().numpy(), want[f])
     finally:
         vol.close()
+
+
+@pytest.mark.parametrize("light", [128, 1024])
+def test_first_trace_on_another_stream(cv, gpu_ctx, light):
+    """The next frame's voxelization on its own stream, beside a first trace that
+    is still queued on another (side streams in a chain and apart)."""
+    import torch
+
+    log(f"[slots] first trace on another stream, light {light}")
+    scene = replace(_scene(cv, 48, 6, 64, 16.0), light_w=light, light_h=light)
+    moved = [scene.xyz, (scene.xyz + np.float32(0.4)).astype(np.float32)]
+    want = [run_oracle(replace(scene, xyz=m), want_f64=False).img32 for m in moved]
+    for _ in range(2):
+        vol, sun, cam, vox, tr = cv.scene_objects(scene, context=gpu_ctx)
+        try:
+            a, b = torch.cuda.Stream(), torch.cuda.Stream()
+            imgs = [torch.zeros((scene.H, scene.W, 4), dtype=torch.float32, device="cuda") for _ in moved]
+            torch.cuda.synchronize()
+            for q in range(2):  # both level sets exist
+                vox.voxelize(vol, sun, stream=a)
+            b.wait_stream(a)
+            with torch.cuda.stream(b):
+                torch.cuda._sleep(20_000_000)
+            tr.coneTrace(vol, sun, cam, imgs[0], scene.W, scene.H, stream=b)
+            vol.set_billboards(moved[1], scene.scales)
+            vox.voxelize(vol, sun, stream=a)
+            tr.coneTrace(vol, sun, cam, imgs[1], scene.W, scene.H, stream=a)
+            torch.cuda.synchronize()
+            for f, img in enumerate(imgs):
+                assert_bit_equal(f"frame {f}", img.cpu().numpy(), want[f])
+        finally:
+            vol.close()
