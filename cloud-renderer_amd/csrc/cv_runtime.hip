@@ -1079,8 +1079,13 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
 // the host's time is events (3 us to record one, 4 to wait for one) that order
 // the three side streams: its passes follow one another on one of them
 // (a 32^3, 256 x 256 frame of 64 billboards 111 -> 84 us, 40^3 137 -> 94).
-// Larger frames run theirs beside the next frame's: 96^3 with 818 billboards
-// and 1426 x 542 pixels took 192 us as a chain, 140 on three streams.
+// Larger frames run theirs beside the next frame's.  us on three streams / as a
+// chain (64, 300, 1000 billboards; square light images), inside the lines: 96^3
+// 256^2 131 / 98, 128 / 95, 130 / 97; 96^3 512^2 130 / 98, 131 / 98, 131 / 129;
+// 64^3 512^2 131 / 98, 128 / 98, 132 / 118; 16^3 and 32^3 1.3 to 1.4 times at all of
+// them.  Outside: 1000 billboards and 800^2 at 64^3 135 / 146, 96^3 133 / 159,
+// 128^3 134 / 169; 128^3 512^2 134 / 140 (with 64 billboards 129 / 98: the lines
+// leave some of the gain).
 static bool small_frame(cr_volume v, const VoxPlan& plan) {
     return v->S <= 1024 && v->N <= 96 && plan.npx <= (size_t)1 << 18 && plan.uniform <= 4096;
 }
