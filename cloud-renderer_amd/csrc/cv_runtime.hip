@@ -1085,7 +1085,9 @@ static void voxelize_enqueue(cr_volume v, const VoxPlan& plan, unsigned long lon
 // 64^3 512^2 131 / 98, 128 / 98, 132 / 118; 16^3 and 32^3 1.3 to 1.4 times at all of
 // them.  Outside: 1000 billboards and 800^2 at 64^3 135 / 146, 96^3 133 / 159,
 // 128^3 134 / 169; 128^3 512^2 134 / 140 (with 64 billboards 129 / 98: the lines
-// leave some of the gain).
+// leave some of the gain).  Volumes of a context share the streams, so a chain's
+// wait for its level set stands before the work list of a larger volume too:
+// a 32^3 and a 256^3 frame in turn take 453 us, 470 before there were chains.
 static bool small_frame(cr_volume v, const VoxPlan& plan) {
     return v->S <= 1024 && v->N <= 96 && plan.npx <= (size_t)1 << 18 && plan.uniform <= 4096;
 }
