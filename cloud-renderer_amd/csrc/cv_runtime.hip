@@ -120,8 +120,8 @@ struct cr_volume_s {
     void* d_ntex = nullptr;  // density noise texture (vd.ntex), rebuilt by cr_volume_set_noise
     size_t ntex_cap = 0;
     size_t zflags_bytes = 0;
-    // R8 volumes: per set the cone's footprint slots and the level-0 bricks'
-    // zero flags, from the first cone trace on (foot_prepare; null without room
+    // R8 volumes: per set the cone's footprint slots and behind them the level-0
+    // bricks' zero flags, from the first cone trace on (foot_prepare; null without room
     // for them: the cone samples the texels)
     uint2* d_foot[2] = {nullptr, nullptr};
     uint8_t* d_fzero[2] = {nullptr, nullptr};
@@ -574,14 +574,12 @@ static void foot_alloc(cr_volume v, int set, hipStream_t s) {
     const size_t n = foot_slots(v->vd);
     if (n == 0) return;
     const size_t zb = ((size_t)v->nbricks0 + 7) & ~(size_t)7;
-    if (hipMalloc((void**)&v->d_foot[set], n * sizeof(uint2)) != hipSuccess ||
-        hipMalloc((void**)&v->d_fzero[set], zb) != hipSuccess) {
+    if (hipMalloc((void**)&v->d_foot[set], n * sizeof(uint2) + zb) != hipSuccess) {
         (void)hipGetLastError();
-        if (v->d_foot[set]) (void)hipFree(v->d_foot[set]);
         v->d_foot[set] = nullptr;
-        v->d_fzero[set] = nullptr;
         return;
     }
+    v->d_fzero[set] = (uint8_t*)(v->d_foot[set] + n);
     launch_fill_u64((uint64_t*)v->d_foot[set], n, 0, s);
     launch_fill_u64((uint64_t*)v->d_fzero[set], zb / 8, 0x0101010101010101ull, s);
 }
@@ -716,7 +714,7 @@ int cr_volume_destroy(cr_volume v) {
                          v->ev_release[1], v->ev_bfree[0], v->ev_bfree[1], v->ev_items, v->ev_lfree[0],
                          v->ev_lfree[1]})
         if (e) (void)hipEventDestroy(e);
-    void* ptrs[] = {v->d_lset[0], v->d_lset[1], v->d_zflags[0], v->d_zflags[1], v->d_foot[0], v->d_foot[1], v->d_fzero[0], v->d_fzero[1], v->d_shell_s[0], v->d_shell_s[1], v->d_fill_s[0], v->d_fill_s[1],    v->d_boards,    v->d_keys,      v->d_posmap,
+    void* ptrs[] = {v->d_lset[0], v->d_lset[1], v->d_zflags[0], v->d_zflags[1], v->d_foot[0], v->d_foot[1], v->d_shell_s[0], v->d_shell_s[1], v->d_fill_s[0], v->d_fill_s[1],    v->d_boards,    v->d_keys,      v->d_posmap,
                     v->d_lbox,   v->d_lcounts, v->d_litems,  v->d_sph_world, v->d_sph_view,  v->d_sph_tiles,
                     v->d_sort,   v->d_order,   v->d_tie,     v->d_masks,     v->d_counters,  v->d_scratch, v->d_tiles,
                     v->cam_spare.sph_world, v->cam_spare.sph_view, v->cam_spare.sph_tiles, v->cam_spare.sort,
